@@ -13,7 +13,7 @@ from pathlib import Path
 import torch  # noqa: F401  (load torch's HIP runtime first)
 
 LIB_PATH = Path(__file__).resolve().parent / "libcvfes_mi355x.so"
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 METHOD_STORED = 0
 METHOD_MATFREE = 1
@@ -55,7 +55,8 @@ class CvfesSystem(ctypes.Structure):
         ("uvalues", _vp), ("vblk", _vp), ("nnzu", _i64), ("row_order", _vp),
         ("color_ptr", _vp), ("color_elems", _vp), ("elems", _vp), ("cpos", _vp), ("n_colors", _i64),
         ("max_color_elems", _i64), ("waves_per_simd", _i64), ("row_records", _vp),
-        ("record_width", _i64), ("minv", _vp),
+        ("record_width", _i64), ("minv", _vp), ("fan", _vp),
+        ("tile_head", _vp), ("tile_cols", _vp), ("tile_ents", _vp), ("n_tiles", _i64),
     ]
 
 
@@ -82,7 +83,8 @@ class CvfesBatchMesh(ctypes.Structure):
 
     _fields_ = [("sys", CvfesSystem), ("method", _i64), ("state", _vp * 3), ("load", CvfesLoad),
                 ("dt", _f64), ("beta", _f64), ("damp", _f64), ("task0", _i64), ("lanes", _i64),
-                ("vw", _i64), ("packed", _i64), ("n_mtasks", _i64), ("slice", _i64), ("xtask0", _i64)]
+                ("vw", _i64), ("packed", _i64), ("n_mtasks", _i64), ("slice", _i64), ("xtask0", _i64),
+                ("tiled", _i64)]
 
 
 _SIGNATURES = {
@@ -93,6 +95,9 @@ _SIGNATURES = {
     "cvfes_stream_blocks": (_i64, [_i64]),
     "cvfes_stream_read": (_int, [_vp, _vp, _i64, _int, _vp]),
     "cvfes_stream_copy": (_int, [_vp, _vp, _i64, _int, _vp]),
+    "cvfes_node_fans": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp]),
+    "cvfes_tile_rows": (_i64, [_i64, _vp, _vp, _vp, _vp, _i64]),
+    "cvfes_tile_lists": (_int, [_vp, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _vp]),
     "cvfes_element_matrices": (_int, [_vp, _i64, _vp, _vp, _f64, _f64, _vp, _vp, _vp, _vp]),
     "cvfes_element_coef": (_int, [_vp, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _int, _vp]),
     "cvfes_lumped_mass_load": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64,
@@ -124,6 +129,13 @@ _SIGNATURES = {
     "cvfes_batch_plan": (_int, [_vp, ctypes.POINTER(CvfesBatchMesh), _int, _vp,
                                 ctypes.POINTER(_i64), ctypes.POINTER(_i64)]),
     "cvfes_batch_step": (_int, [_vp, _vp, _int, _i64, _int, _vp, _i64, _i64, _i64]),
+    "cvfes_batch_can_tile": (_int, [ctypes.POINTER(CvfesBatchMesh)]),
+    "cvfes_batch_tile_bytes": (_i64, [_int]),
+    "cvfes_batch_plan_tiles": (_int, [_vp, ctypes.POINTER(CvfesBatchMesh), _int, _vp,
+                                      ctypes.POINTER(_i64), ctypes.POINTER(_i64)]),
+    "cvfes_batch_step_tiles": (_int, [_vp, _vp, _vp, _int, _i64, _i64, _int, _vp, _i64]),
+    "cvfes_batch_graph_create_tiles": (_int, [_vp, _int, _i64, _vp, _i64, _int, _i64, _i64, _vp,
+                                              _i64, _i64, ctypes.POINTER(_vp)]),
     "cvfes_counter_add": (_int, [_vp, _vp, _i64]),
     "cvfes_batch_graph_create": (_int, [_vp, _int, _i64, _vp, _i64, _int, _i64, _i64,
                                         ctypes.POINTER(_vp)]),
@@ -132,6 +144,12 @@ _SIGNATURES = {
 }
 
 EXPORTED = tuple(_SIGNATURES)
+
+# Most elements around one node that cvfes_node_fans takes (CVFES_FAN_MAX_ELEMS).
+FAN_MAX_ELEMS = 341
+
+# Node tiles of the matrix-free kernels (CVFES_TILE_*).
+TILE_ROWS, TILE_COLS, TILE_ELEMS = 16, 39, 8
 
 # Doubles in the static device scratch of cvfes_initial_state_static (CVFES_STATIC_SCRATCH_DOUBLES).
 STATIC_SCRATCH_DOUBLES = 8 << 20

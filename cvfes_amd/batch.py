@@ -86,12 +86,21 @@ class BatchedEnsemble:
             m.load = self.loads[i].struct(0)
             m.dt, m.beta, m.damp = self.dts[i], self.betas[i], self.damps[i]
             m.vw = self.vw_hint
+            m.tiled = int(m.sys.n_tiles > 0 and self.lib.cvfes_batch_can_tile(ctypes.byref(m)) != 0)
         self._bufs = [(s.state[0], s.state[2], s.state[1]) for s in self.systems]   # state[0..2]
         nbytes = int(self.lib.cvfes_batch_plan_bytes(n))
         self.dev_meshes = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         n_tasks, kinds = ctypes.c_int64(0), ctypes.c_int64(0)
         check(self.lib.cvfes_batch_plan(self.stream, arr, n, self.dev_meshes.data_ptr(),
                                         ctypes.byref(n_tasks), ctypes.byref(kinds)))
+        self.n_blocks, self.tile_shape, self.dev_tiles = 0, 0, None
+        if any(int(m.tiled) for m in arr):
+            n_blocks, shape = ctypes.c_int64(0), ctypes.c_int64(0)
+            self.dev_tiles = torch.empty(int(self.lib.cvfes_batch_tile_bytes(n)), dtype=torch.uint8,
+                                         device=self.device)
+            check(self.lib.cvfes_batch_plan_tiles(self.stream, arr, n, self.dev_tiles.data_ptr(),
+                                                  ctypes.byref(n_blocks), ctypes.byref(shape)))
+            self.n_blocks, self.tile_shape = int(n_blocks.value), int(shape.value)
         self.host_meshes = arr
         # the kernels read load-table entry (absolute step) with no bound of their own
         self.max_steps = min(int(ld.n) for ld in self.loads)
@@ -127,6 +136,11 @@ class BatchedEnsemble:
             check(self.lib.cvfes_batch_step(self.stream, self.dev_meshes.data_ptr(),
                                             len(self.systems), self.n_tasks, self.phase, None,
                                             self.step_index, self.n_waves, self._kinds()))
+            if self.n_blocks:
+                check(self.lib.cvfes_batch_step_tiles(self.stream, self.dev_meshes.data_ptr(),
+                                                      self.dev_tiles.data_ptr(), len(self.systems),
+                                                      self.n_blocks, self.tile_shape, self.phase,
+                                                      None, self.step_index))
             self.phase = (self.phase + 1) % 3
             self.step_index += 1
 
@@ -134,10 +148,10 @@ class BatchedEnsemble:
         key = (block, self.phase, self.n_waves, self._kinds())
         if key not in self._graphs:
             g = ctypes.c_void_p()
-            check(self.lib.cvfes_batch_graph_create(self.dev_meshes.data_ptr(), len(self.systems),
-                                                    self.n_tasks, self.counter.data_ptr(), block,
-                                                    self.phase, self.n_waves, self._kinds(),
-                                                    ctypes.byref(g)))
+            check(self.lib.cvfes_batch_graph_create_tiles(
+                self.dev_meshes.data_ptr(), len(self.systems), self.n_tasks, self.counter.data_ptr(),
+                block, self.phase, self.n_waves, self._kinds(), ptr(self.dev_tiles), self.n_blocks,
+                self.tile_shape, ctypes.byref(g)))
             self._graphs[key] = g.value
         return self._graphs[key]
 

@@ -12,7 +12,7 @@
 // u_{-1} depends on K through the initial acceleration; its adjoint
 //   lambda_{-1} = -(1-gamma) mu_1 + b0 K A mu_1   (u_{-1} is not projected)
 // adds -coef_e (dt^2/2 M^-1 lambda_{-1})_e^T khat_e (u0 + beta du0)_e.
-#include "rowops.h"
+#include "tile.h"
 
 namespace cvfes {
 namespace {
@@ -86,38 +86,136 @@ __device__ __forceinline__ void adj_column(const AdjArgs &a, int64_t col, int64_
     }
 }
 
+// The same column for the fan product: the node's loads (load) and the column formed from them.
+template <bool UNI, bool BETA, int VW>
+struct AdjCol {
+    static constexpr int kCols = 1;
+    struct Raw {
+        Vec<VW> m1[3], m2[3], q;      // q: inverse mass (or mass) of the node
+    };
+    struct Own {
+        Vec<VW> m1[3], m2[3];
+    };
+    const AdjArgs &a;
+    uint32_t lane;
+
+    __device__ __forceinline__ Raw load(int32_t node) const {
+        Raw r;
+        const double *m = a.minv ? a.minv : a.lm;
+        if (a.lm_sstride) {
+            r.q = load_entry<UNI, VW>(m, node, a.k.n_smp, lane);
+        } else {
+            const double mv = m[node];
+#pragma unroll
+            for (int v = 0; v < VW; ++v) r.q.v[v] = mv;
+        }
+        load_node<UNI, VW>(a.mu1, node, a.k.n_smp, lane, r.m1);
+        if constexpr (BETA) load_node<UNI, VW>(a.mu2, node, a.k.n_smp, lane, r.m2);
+        return r;
+    }
+    __device__ __forceinline__ Own own(int32_t node) const {
+        Own o;
+        load_node<UNI, VW>(a.mu1, node, a.k.n_smp, lane, o.m1);
+        load_node<UNI, VW>(a.mu2, node, a.k.n_smp, lane, o.m2);
+        return o;
+    }
+    __device__ __forceinline__ void column(const Raw &r, double (&x)[3][VW]) const {
+#pragma unroll
+        for (int v = 0; v < VW; ++v) {
+            const double q = a.minv ? r.q.v[v] * a.dt2 : (r.q.v[v] != 0.0 ? a.dt2 / r.q.v[v] : 0.0);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                double comb = r.m1[j].v[v];
+                if constexpr (BETA) comb = fma(a.bdt, r.m1[j].v[v] - r.m2[j].v[v], r.m1[j].v[v]);
+                x[j][v] = comb * q;
+            }
+        }
+    }
+    __device__ __forceinline__ void value(const Raw &r, double (&x)[1][3][VW]) const { column(r, x[0]); }
+};
+
+// Forward and adjoint columns of the fused step, both applied with each operator load.
+template <bool UNI, bool BETA, int VW>
+struct FusedCol {
+    static constexpr int kCols = 2;
+    typedef StateCol<UNI, BETA, VW, const double *> F;
+    typedef AdjCol<UNI, BETA, VW> A;
+    struct Raw {
+        typename F::Raw f;
+        typename A::Raw a;
+    };
+    F f;
+    A a;
+    uint32_t lane;
+
+    __device__ __forceinline__ Raw load(int32_t node) const { return Raw{f.load(node), a.load(node)}; }
+    __device__ __forceinline__ void value(const Raw &r, double (&x)[2][3][VW]) const {
+        f.column(r.f, x[0]);
+        a.column(r.a, x[1]);
+    }
+};
+
 // lambda_n of one block row from acc = K A (b1 mu1 - b0 mu2) and the observation term; stores
 // mu_n = P lambda_n (or lambda when not projecting) when `active`.  Explicit fma throughout, so
 // the rounding is the same in the separate and the fused kernels.
 template <bool DAMP, int VW>
 __device__ __forceinline__ void adj_finish(const AdjArgs &a, int32_t row, int64_t s, bool active,
-                                           const double (&acc)[3][VW]) {
+                                           const double (&acc)[3][VW], const Vec<VW> (&m1)[3],
+                                           const Vec<VW> (&m2)[3]) {
     const int64_t S = a.k.n_smp;
     const bool fixed = a.project && a.fixed != nullptr && a.fixed[row] != 0;
-    const Vec<VW> m = mass_at<VW>(a, row, s);
+    const int64_t off = static_cast<int64_t>(row) * 3 * S + s;
+    Vec<VW> gam;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const int64_t off = (static_cast<int64_t>(row) * 3 + i) * S + s;
-        const Vec<VW> m1 = load_vec<VW>(a.mu1 + off);
-        const Vec<VW> m2 = load_vec<VW>(a.mu2 + off);
-        Vec<VW> o;
+    for (int v = 0; v < VW; ++v) gam.v[v] = 0.0;
+    if constexpr (DAMP) {
+        const Vec<VW> m = mass_at<VW>(a, row, s);
 #pragma unroll
-        for (int v = 0; v < VW; ++v) {
-            double gam = 0.0;
-            if constexpr (DAMP) gam = m.v[v] != 0.0 ? a.dtdamp / m.v[v] : 0.0;
-            double lam = fma(2.0 - gam, m1.v[v], -fma(1.0 - gam, m2.v[v], acc[i][v]));
-            if (a.obs_u) {
-                const double ref = a.obs_ref ? a.obs_ref[off + v] : 0.0;
-                const double w = a.obs_w ? a.obs_w[s + v] : 1.0;
-                lam = fma(w, a.obs_u[off + v] - ref, lam);
-            }
-            o.v[v] = fixed ? 0.0 : lam;
-        }
-        if (active) {   // not read again in this launch: large outputs are streamed (stream_out)
-            if (a.nt_out) store_vec_nt<VW>(a.out + off, o);
-            else store_vec<VW>(a.out + off, o);
+        for (int v = 0; v < VW; ++v) gam.v[v] = m.v[v] != 0.0 ? a.dtdamp / m.v[v] : 0.0;
+    }
+    Vec<VW> o[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int v = 0; v < VW; ++v)
+            o[i].v[v] = fma(2.0 - gam.v[v], m1[i].v[v], -fma(1.0 - gam.v[v], m2[i].v[v], acc[i][v]));
+    if (a.obs_u) {
+        Vec<VW> w;
+#pragma unroll
+        for (int v = 0; v < VW; ++v) w.v[v] = a.obs_w ? a.obs_w[s + v] : 1.0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const Vec<VW> u = load_vec<VW>(a.obs_u + off + i * S);
+            Vec<VW> ref;
+#pragma unroll
+            for (int v = 0; v < VW; ++v) ref.v[v] = a.obs_ref ? a.obs_ref[off + i * S + v] : 0.0;
+#pragma unroll
+            for (int v = 0; v < VW; ++v) o[i].v[v] = fma(w.v[v], u.v[v] - ref.v[v], o[i].v[v]);
         }
     }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+#pragma unroll
+        for (int v = 0; v < VW; ++v) o[i].v[v] = fixed ? 0.0 : o[i].v[v];
+        if (active) {   // not read again in this launch: large outputs are streamed (stream_out)
+            if (a.nt_out) store_vec_nt<VW>(a.out + off + i * S, o[i]);
+            else store_vec<VW>(a.out + off + i * S, o[i]);
+        }
+    }
+}
+
+// The same with the row's own adjoint states read here.
+template <bool DAMP, int VW>
+__device__ __forceinline__ void adj_finish(const AdjArgs &a, int32_t row, int64_t s, bool active,
+                                           const double (&acc)[3][VW]) {
+    Vec<VW> m1[3], m2[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int64_t off = (static_cast<int64_t>(row) * 3 + i) * a.k.n_smp + s;
+        m1[i] = load_vec<VW>(a.mu1 + off);
+        m2[i] = load_vec<VW>(a.mu2 + off);
+    }
+    adj_finish<DAMP, VW>(a, row, s, active, acc, m1, m2);
 }
 
 template <int OP, bool UNIFORM, bool BETA, bool DAMP, int VW>
@@ -126,6 +224,13 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_step(AdjArgs a) {
     int64_t s;
     bool active;
     if (!row_and_sample<UNIFORM, VW>(a.k.n_nodes, a.k.n_smp, row, s, active)) return;
+    if constexpr (OP == kOpFan) {
+        typedef AdjCol<UNIFORM, BETA, VW> Col;
+        double y[1][3][VW];
+        fan_product<UNIFORM, VW>(a.k, Col{a, static_cast<uint32_t>(s) * 8u}, row, y);
+        adj_finish<DAMP, VW>(a, row, s, active, y[0]);
+        return;
+    }
     double acc[3][VW];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -138,6 +243,21 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_step(AdjArgs a) {
         block_apply<OP, VW>(a.k, p, col < row, s, x, acc);
     }
     adj_finish<DAMP, VW>(a, row, s, active, acc);
+}
+
+// The matrix-free adjoint step by node tiles (tile.h); the bits are those of k_adjoint_step<kOpFan>.
+template <bool BETA, bool DAMP, int VW, int ELEMS, bool SMALL>
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void k_adjoint_tile(AdjArgs a, TileArgs t) {
+    TilePlace p;
+    if (!tile_place<VW>(t, a.k.n_smp, static_cast<uint32_t>(xcd_block()), p)) return;
+    typedef AdjCol<false, BETA, VW> Col;
+    const Col col{a, static_cast<uint32_t>(p.s) * 8u};
+    double acc[3][VW];
+    typename Col::Own own;
+    tile_product<ELEMS, VW, SMALL>(a.k, t, col, p.tile, p.i, p.l, p.in, p.rw, acc,
+                            [&](int32_t node) { own = col.own(node); });
+    if (p.active) adj_finish<DAMP, VW>(a, p.rw.x, p.s, true, acc, own.m1, own.m2);
 }
 
 // One forward step (the generic row kernel's operations) and one adjoint step in a single pass
@@ -155,6 +275,16 @@ __global__ __launch_bounds__(kBlock) void k_fused_step(StepArgs f, AdjArgs a, in
     int64_t s;
     bool active;
     if (!row_and_sample<UNIFORM, VW>(f.k.n_nodes, f.k.n_smp, row, s, active)) return;
+    if constexpr (OP == kOpFan) {
+        const uint32_t lane = static_cast<uint32_t>(s) * 8u;
+        typedef FusedCol<UNIFORM, BETA, VW> Col;
+        const Col col{{f.u, f.up, f.bdt, f.k.n_smp, lane}, {a, lane}, lane};
+        double y[2][3][VW];
+        fan_product<UNIFORM, VW>(f.k, col, row, y);
+        step_update<DAMP, VW>(f, row, s, active, step, y[0]);
+        adj_finish<DAMP, VW>(a, row, s, active, y[1]);
+        return;
+    }
     double accf[3][VW], acca[3][VW];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -353,6 +483,43 @@ void adj_launch(hipStream_t st, const AdjArgs &a, bool beta, bool damp) {
     }
 }
 
+template <int VW, int ELEMS, bool SMALL>
+void adj_tile_launch(hipStream_t st, const AdjArgs &a, const TileArgs &t, const TileShape &h, bool beta,
+                     bool damp) {
+    const dim3 g(tile_grid(t)), b(64 * h.waves);
+    const size_t lds = tile_lds(h.chunk, ELEMS);
+    if (beta) {
+        if (damp) hipLaunchKernelGGL((k_adjoint_tile<true, true, VW, ELEMS, SMALL>), g, b, lds, st, a, t);
+        else hipLaunchKernelGGL((k_adjoint_tile<true, false, VW, ELEMS, SMALL>), g, b, lds, st, a, t);
+    } else {
+        if (damp) hipLaunchKernelGGL((k_adjoint_tile<false, true, VW, ELEMS, SMALL>), g, b, lds, st, a, t);
+        else hipLaunchKernelGGL((k_adjoint_tile<false, false, VW, ELEMS, SMALL>), g, b, lds, st, a, t);
+    }
+}
+
+void adj_tile(hipStream_t st, const cvfes_system_t *sys, const AdjArgs &a, bool beta, bool damp) {
+    const TileShape h = tile_shape(sys->n_smp);
+    const TileArgs t = tile_args(sys, h);
+    const bool six = sys->max_node_elems <= 6, small = sys->n_smp <= kTileSmall;
+    if (h.vw == 2) {
+        if (small) {
+            if (six) adj_tile_launch<2, 6, true>(st, a, t, h, beta, damp);
+            else adj_tile_launch<2, 8, true>(st, a, t, h, beta, damp);
+        } else {
+            if (six) adj_tile_launch<2, 6, false>(st, a, t, h, beta, damp);
+            else adj_tile_launch<2, 8, false>(st, a, t, h, beta, damp);
+        }
+    } else {
+        if (small) {
+            if (six) adj_tile_launch<1, 6, true>(st, a, t, h, beta, damp);
+            else adj_tile_launch<1, 8, true>(st, a, t, h, beta, damp);
+        } else {
+            if (six) adj_tile_launch<1, 6, false>(st, a, t, h, beta, damp);
+            else adj_tile_launch<1, 8, false>(st, a, t, h, beta, damp);
+        }
+    }
+}
+
 // Lane width and row mapping as the generic forward kernel chooses them (generic_vw; wave-uniform
 // rows when they keep 3/4 of the lanes busy).
 template <int MF>
@@ -392,7 +559,8 @@ void fused_dispatch(hipStream_t st, const StepArgs &f, const AdjArgs &a, bool be
 // Operator form of the generic row kernels for this system and method (as the forward step's
 // generic kernel chooses it: full values when present, else the symmetric upper blocks).
 int operator_form(const cvfes_system_t *sys, int method) {
-    return method == CVFES_METHOD_MATFREE ? kOpMatfree : (sys->values ? kOpStored : kOpSym);
+    if (method == CVFES_METHOD_MATFREE) return fan_entries(sys) ? kOpFan : kOpMatfree;
+    return sys->values ? kOpStored : kOpSym;
 }
 
 int check_adjoint_args(const cvfes_system_t *sys, int method, const double *mu1, const double *mu2,
@@ -418,7 +586,8 @@ AdjArgs adjoint_args(const cvfes_system_t *sys, const double *mu1, const double 
                      double beta, double damp, int project) {
     AdjArgs a{};
     a.k = RowArgs{sys->n_nodes, sys->n_smp, sys->indptr, sys->indices, sys->values,
-                  sys->cptr, sys->celem, sys->khat, sys->coef, sys->uvalues, sys->vblk};
+                  sys->cptr, sys->celem, sys->khat, sys->coef, sys->uvalues, sys->vblk,
+                  sys->nptr, fan_entries(sys)};
     a.mu1 = mu1;
     a.mu2 = mu2;
     a.out = mu_out;
@@ -457,6 +626,10 @@ extern "C" int cvfes_adjoint_step(void *stream, const cvfes_system_t *sys, int m
     const AdjArgs a = adjoint_args(sys, mu1, mu2, mu_out, obs_u, obs_ref, obs_w, dt, beta, damp, project);
     hipStream_t st = static_cast<hipStream_t>(stream);
     switch (operator_form(sys, method)) {
+    case kOpFan:
+        if (tiles_apply(sys)) adj_tile(st, sys, a, beta != 0.0, damp != 0.0);
+        else adj_dispatch<kOpFan>(st, a, beta != 0.0, damp != 0.0);
+        break;
     case kOpMatfree: adj_dispatch<kOpMatfree>(st, a, beta != 0.0, damp != 0.0); break;
     case kOpStored: adj_dispatch<kOpStored>(st, a, beta != 0.0, damp != 0.0); break;
     default: adj_dispatch<kOpSym>(st, a, beta != 0.0, damp != 0.0); break;
@@ -487,7 +660,8 @@ extern "C" int cvfes_adjoint_fused_step(void *stream, const cvfes_system_t *sys,
                   static_cast<long long>(kern));
     StepArgs f{};
     f.k = RowArgs{sys->n_nodes, sys->n_smp, sys->indptr, sys->indices, sys->values,
-                  sys->cptr, sys->celem, sys->khat, sys->coef, sys->uvalues, sys->vblk};
+                  sys->cptr, sys->celem, sys->khat, sys->coef, sys->uvalues, sys->vblk,
+                  sys->nptr, fan_entries(sys)};
     f.u = state[0];
     f.up = state[1];
     f.out = state[2];
@@ -506,6 +680,7 @@ extern "C" int cvfes_adjoint_fused_step(void *stream, const cvfes_system_t *sys,
     const AdjArgs a = adjoint_args(sys, mu1, mu2, mu_out, obs_u, obs_ref, obs_w, dt, beta, damp, 1);
     hipStream_t st = static_cast<hipStream_t>(stream);
     switch (operator_form(sys, method)) {
+    case kOpFan: fused_dispatch<kOpFan>(st, f, a, beta != 0.0, damp != 0.0); break;
     case kOpMatfree: fused_dispatch<kOpMatfree>(st, f, a, beta != 0.0, damp != 0.0); break;
     case kOpStored: fused_dispatch<kOpStored>(st, f, a, beta != 0.0, damp != 0.0); break;
     default: fused_dispatch<kOpSym>(st, f, a, beta != 0.0, damp != 0.0); break;

@@ -16,7 +16,7 @@
 // out = state[(phase+1)%3].  The step index used for the load tables is *counter + k_local (or
 // k_local without a counter).  A captured graph holds a multiple of 3 steps plus one counter
 // increment, so a replay leaves the roles and the counter ready for the next replay.
-#include "rowops.h"
+#include "tile.h"
 
 #include <algorithm>
 #include <vector>
@@ -38,14 +38,13 @@ __device__ __forceinline__ const CVFES_K T *as_const(const T *p) {
     return (const CVFES_K T *)p;
 }
 
-template <int OP, bool BETA, bool DAMP, int VW>
-__device__ __forceinline__ void batch_task(const cvfes_batch_mesh_t &d, int phase, int64_t n,
-                                           int32_t row, int64_t s, bool active) {
+__device__ __forceinline__ GStepArgs batch_args(const cvfes_batch_mesh_t &d, int phase) {
     GStepArgs a;
     a.k = GRowArgs{d.sys.n_nodes, d.sys.n_smp, as_const(d.sys.indptr), as_const(d.sys.indices),
                    as_global(d.sys.values), as_const(d.sys.cptr), as_const(d.sys.celem),
                    as_const(d.sys.khat), as_global(d.sys.coef), as_global(d.sys.uvalues),
-                   as_const(d.sys.vblk)};
+                   as_const(d.sys.vblk), as_const(d.sys.nptr),
+                   as_const(reinterpret_cast<const fan_t *>(d.sys.fan))};
     a.u = as_global(d.state[phase]);
     a.up = as_global(d.state[(phase + 2) % 3]);
     a.out = (CVFES_G double *)d.state[(phase + 1) % 3];
@@ -60,47 +59,115 @@ __device__ __forceinline__ void batch_task(const cvfes_batch_mesh_t &d, int phas
     a.bdt = d.beta / d.dt;
     a.ddt = d.damp / d.dt;
     a.nt_out = false;   // ordinary stores: the ensemble measured faster without streaming them
-    step_row<OP, BETA, DAMP, VW>(a, row, s, active, n);
+    return a;
+}
+
+template <int OP, bool UNI, bool BETA, bool DAMP, int VW>
+__device__ __forceinline__ void batch_task(const cvfes_batch_mesh_t &d, int phase, int64_t n,
+                                           int32_t row, int64_t s, bool active) {
+    step_row<OP, UNI, BETA, DAMP, VW>(batch_args(d, phase), row, s, active, n);
+}
+
+// A tiled mesh's launch shape and its first workgroup in every XCD's list.
+struct BatchTiles {
+    TileArgs t;
+    int32_t vw, slice;
+    int64_t first;
+};
+
+// One step of the tiled meshes: workgroup b runs on XCD b mod 8 and takes item b / 8 of the XCD's
+// list (its slice of every tiled mesh, mesh after mesh).  The row kernels of the batch read a
+// row's columns from L1/L2 and its unit blocks through the scalar cache (or per lane); here both
+// come from LDS, as in the single-mesh tile step, whose bits these are.
+template <bool BD, int ELEMS>
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void k_batch_tile(const cvfes_batch_mesh_t *__restrict__ meshes, const BatchTiles *__restrict__ tiles,
+                  int n_mesh, int phase, const int64_t *__restrict__ counter, int64_t k_local) {
+    const int64_t *__restrict__ first = reinterpret_cast<const int64_t *>(tiles + n_mesh);
+    const int64_t item = blockIdx.x / kNumXcd;
+    const int lane = threadIdx.x & 63;
+    int mi = -1;                    // the last mesh whose first item is not behind this one
+    for (int base = 0; base < n_mesh; base += 64) {
+        const int m = base + lane;
+        mi += __popcll(__ballot(m < n_mesh && first[m] <= item));
+    }
+    const BatchTiles &bt = tiles[mi];
+    const int64_t local = item - bt.first;
+    if (local >= bt.slice) return;
+    const TileArgs t = bt.t;
+    if (static_cast<int>(threadIdx.x >> 6) * t.groups >= kTileRows) return;    // more waves than rows
+    const uint32_t b = static_cast<uint32_t>((blockIdx.x % kNumXcd) * bt.slice + local);
+    const cvfes_batch_mesh_t &d = meshes[mi];
+    const GStepArgs a = batch_args(d, phase);
+    const int64_t n = (counter ? counter[0] : 0) + k_local;
+    const bool beta = BD && d.beta != 0.0, damp = BD && d.damp != 0.0;
+    if (bt.vw == 2) {
+        if (beta) {
+            if (damp) tile_step<true, true, 2, ELEMS, false>(a, t, b, n);
+            else tile_step<true, false, 2, ELEMS, false>(a, t, b, n);
+        } else {
+            if (damp) tile_step<false, true, 2, ELEMS, false>(a, t, b, n);
+            else tile_step<false, false, 2, ELEMS, false>(a, t, b, n);
+        }
+    } else {
+        if (beta) {
+            if (damp) tile_step<true, true, 1, ELEMS, false>(a, t, b, n);
+            else tile_step<true, false, 1, ELEMS, false>(a, t, b, n);
+        } else {
+            if (damp) tile_step<false, true, 1, ELEMS, false>(a, t, b, n);
+            else tile_step<false, false, 1, ELEMS, false>(a, t, b, n);
+        }
+    }
 }
 
 // Path sets: a kernel instance only contains the operators and damping forms that occur in the
 // ensemble (cvfes_batch_plan reports them), so it needs no more registers than those paths do.
-template <int VW, bool STORED, bool BD>
+// FAN: every matrix-free mesh has fan entries; without it the matrix-free meshes that have none
+// walk block by block.
+template <int VW, bool UNI, bool STORED, bool BD, bool FAN>
 __device__ __forceinline__ void batch_dispatch(const cvfes_batch_mesh_t &d, int phase, int64_t n,
                                                int32_t row, int64_t s, bool active) {
     const bool mf = !STORED || d.method == CVFES_METHOD_MATFREE;
     const bool beta = BD && d.beta != 0.0, damp = BD && d.damp != 0.0;
-    if (mf) {
+    if (mf && (FAN || d.sys.fan)) {
         if (beta) {
-            if (damp) batch_task<kOpMatfree, true, true, VW>(d, phase, n, row, s, active);
-            else batch_task<kOpMatfree, true, false, VW>(d, phase, n, row, s, active);
+            if (damp) batch_task<kOpFan, UNI, true, true, VW>(d, phase, n, row, s, active);
+            else batch_task<kOpFan, UNI, true, false, VW>(d, phase, n, row, s, active);
         } else {
-            if (damp) batch_task<kOpMatfree, false, true, VW>(d, phase, n, row, s, active);
-            else batch_task<kOpMatfree, false, false, VW>(d, phase, n, row, s, active);
+            if (damp) batch_task<kOpFan, UNI, false, true, VW>(d, phase, n, row, s, active);
+            else batch_task<kOpFan, UNI, false, false, VW>(d, phase, n, row, s, active);
+        }
+    } else if (!FAN && mf) {
+        if (beta) {
+            if (damp) batch_task<kOpMatfree, UNI, true, true, VW>(d, phase, n, row, s, active);
+            else batch_task<kOpMatfree, UNI, true, false, VW>(d, phase, n, row, s, active);
+        } else {
+            if (damp) batch_task<kOpMatfree, UNI, false, true, VW>(d, phase, n, row, s, active);
+            else batch_task<kOpMatfree, UNI, false, false, VW>(d, phase, n, row, s, active);
         }
     } else if constexpr (STORED) {
         // stored values in full storage when the mesh holds them, else in symmetric storage
         if (d.sys.values) {
             if (beta) {
-                if (damp) batch_task<kOpStored, true, true, VW>(d, phase, n, row, s, active);
-                else batch_task<kOpStored, true, false, VW>(d, phase, n, row, s, active);
+                if (damp) batch_task<kOpStored, UNI, true, true, VW>(d, phase, n, row, s, active);
+                else batch_task<kOpStored, UNI, true, false, VW>(d, phase, n, row, s, active);
             } else {
-                if (damp) batch_task<kOpStored, false, true, VW>(d, phase, n, row, s, active);
-                else batch_task<kOpStored, false, false, VW>(d, phase, n, row, s, active);
+                if (damp) batch_task<kOpStored, UNI, false, true, VW>(d, phase, n, row, s, active);
+                else batch_task<kOpStored, UNI, false, false, VW>(d, phase, n, row, s, active);
             }
         } else {
             if (beta) {
-                if (damp) batch_task<kOpSym, true, true, VW>(d, phase, n, row, s, active);
-                else batch_task<kOpSym, true, false, VW>(d, phase, n, row, s, active);
+                if (damp) batch_task<kOpSym, UNI, true, true, VW>(d, phase, n, row, s, active);
+                else batch_task<kOpSym, UNI, true, false, VW>(d, phase, n, row, s, active);
             } else {
-                if (damp) batch_task<kOpSym, false, true, VW>(d, phase, n, row, s, active);
-                else batch_task<kOpSym, false, false, VW>(d, phase, n, row, s, active);
+                if (damp) batch_task<kOpSym, UNI, false, true, VW>(d, phase, n, row, s, active);
+                else batch_task<kOpSym, UNI, false, false, VW>(d, phase, n, row, s, active);
             }
         }
     }
 }
 
-template <bool ONE, bool U2, bool P2, bool V1, bool STORED, bool BD>
+template <bool ONE, bool U2, bool P2, bool V1, bool STORED, bool BD, bool FAN>
 __device__ __forceinline__ void batch_body(const cvfes_batch_mesh_t *__restrict__ meshes, int n_mesh,
                                            int64_t n_tasks, int phase,
                                            const int64_t *__restrict__ counter, int64_t k_local,
@@ -147,8 +214,8 @@ __device__ __forceinline__ void batch_body(const cvfes_batch_mesh_t *__restrict_
             const bool active = in && s < S;
             const int32_t row = in ? static_cast<int32_t>(r) : static_cast<int32_t>(d.sys.n_nodes - 1);
             if (!active) s = S - vw;
-            if (P2 && (!V1 || vw == 2)) batch_dispatch<2, STORED, BD>(d, phase, n, row, s, active);
-            else if (V1) batch_dispatch<1, STORED, BD>(d, phase, n, row, s, active);
+            if (P2 && (!V1 || vw == 2)) batch_dispatch<2, false, STORED, BD, FAN>(d, phase, n, row, s, active);
+            else if (V1) batch_dispatch<1, false, STORED, BD, FAN>(d, phase, n, row, s, active);
         } else {
             int32_t row;
             int64_t s;
@@ -166,58 +233,66 @@ __device__ __forceinline__ void batch_body(const cvfes_batch_mesh_t *__restrict_
             }
             const bool active = s < S;
             if (!active) s = S - vw;
-            if (U2 && (!V1 || vw == 2)) batch_dispatch<2, STORED, BD>(d, phase, n, row, s, active);
-            else if (V1) batch_dispatch<1, STORED, BD>(d, phase, n, row, s, active);
+            if (U2 && (!V1 || vw == 2)) batch_dispatch<2, true, STORED, BD, FAN>(d, phase, n, row, s, active);
+            else if (V1) batch_dispatch<1, true, STORED, BD, FAN>(d, phase, n, row, s, active);
         }
     }
 }
 
 // CAP: at most 64 registers (8 waves per SIMD), with spills where the paths need more; the
 // autotuner decides whether the extra waves pay for the spills.
-template <bool ONE, bool U2, bool P2, bool V1, bool STORED, bool BD, bool CAP>
+template <bool ONE, bool U2, bool P2, bool V1, bool STORED, bool BD, bool FAN, bool CAP>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CAP ? 8 : 1)))
 void k_batch_step(const cvfes_batch_mesh_t *__restrict__ meshes, int n_mesh, int64_t n_tasks,
                   int phase, const int64_t *__restrict__ counter, int64_t k_local, int groups_first) {
-    batch_body<ONE, U2, P2, V1, STORED, BD>(meshes, n_mesh, n_tasks, phase, counter, k_local,
+    batch_body<ONE, U2, P2, V1, STORED, BD, FAN>(meshes, n_mesh, n_tasks, phase, counter, k_local,
                                             groups_first);
 }
 
 using BatchKernel = void (*)(const cvfes_batch_mesh_t *, int, int64_t, int, const int64_t *, int64_t,
                              int);
 
+constexpr int64_t kKindNoFan = 1024;   // some matrix-free mesh has no fan entries
+
 // Smallest instance whose lane paths cover the plan's: (uniform two-sample, packed two-sample,
 // one-sample) in {(1,1,1), (1,1,0), (1,0,1), (1,0,0), (0,0,1)}.
-template <bool ONE, bool STORED, bool BD, bool CAP>
+template <bool ONE, bool STORED, bool BD, bool FAN, bool CAP>
 BatchKernel batch_kernel_lanes(int64_t kinds) {
     const bool u2 = kinds & 1, v1 = kinds & 2, p2 = kinds & 16;
-    if (p2) return v1 ? k_batch_step<ONE, true, true, true, STORED, BD, CAP>
-                      : k_batch_step<ONE, true, true, false, STORED, BD, CAP>;
-    if (u2) return v1 ? k_batch_step<ONE, true, false, true, STORED, BD, CAP>
-                      : k_batch_step<ONE, true, false, false, STORED, BD, CAP>;
-    return k_batch_step<ONE, false, false, true, STORED, BD, CAP>;
+    if (p2) return v1 ? k_batch_step<ONE, true, true, true, STORED, BD, FAN, CAP>
+                      : k_batch_step<ONE, true, true, false, STORED, BD, FAN, CAP>;
+    if (u2) return v1 ? k_batch_step<ONE, true, false, true, STORED, BD, FAN, CAP>
+                      : k_batch_step<ONE, true, false, false, STORED, BD, FAN, CAP>;
+    return k_batch_step<ONE, false, false, true, STORED, BD, FAN, CAP>;
+}
+
+template <bool ONE, bool FAN, bool CAP>
+BatchKernel batch_kernel_sb(int64_t kinds) {
+    const bool st = kinds & 4, bd = kinds & 8;
+    if (st) return bd ? batch_kernel_lanes<ONE, true, true, FAN, CAP>(kinds) : batch_kernel_lanes<ONE, true, false, FAN, CAP>(kinds);
+    return bd ? batch_kernel_lanes<ONE, false, true, FAN, CAP>(kinds) : batch_kernel_lanes<ONE, false, false, FAN, CAP>(kinds);
 }
 
 template <bool ONE, bool CAP>
-BatchKernel batch_kernel_sb(int64_t kinds) {
-    const bool st = kinds & 4, bd = kinds & 8;
-    if (st) return bd ? batch_kernel_lanes<ONE, true, true, CAP>(kinds) : batch_kernel_lanes<ONE, true, false, CAP>(kinds);
-    return bd ? batch_kernel_lanes<ONE, false, true, CAP>(kinds) : batch_kernel_lanes<ONE, false, false, CAP>(kinds);
+BatchKernel batch_kernel_fan(int64_t kinds) {
+    return kinds & kKindNoFan ? batch_kernel_sb<ONE, false, false>(kinds) : batch_kernel_sb<ONE, true, CAP>(kinds);
 }
 
 // kinds (from cvfes_batch_plan): bit 0 some wave-uniform mesh with two samples per lane, bit 1
 // some mesh with one sample per lane, bit 2 some stored mesh, bit 3 some mesh with beta or damp,
-// bit 4 some packed mesh with two samples per lane; bit 5 (set by the caller) caps the registers.
+// bit 4 some packed mesh with two samples per lane, bit 10 some matrix-free mesh without fan
+// entries; bit 5 (set by the caller) caps the registers.
 BatchKernel batch_kernel(int64_t kinds, bool one) {
     const bool cap = kinds & 32;
-    if (one) return cap ? batch_kernel_sb<true, true>(kinds) : batch_kernel_sb<true, false>(kinds);
-    return cap ? batch_kernel_sb<false, true>(kinds) : batch_kernel_sb<false, false>(kinds);
+    if (one) return cap ? batch_kernel_fan<true, true>(kinds) : batch_kernel_fan<true, false>(kinds);
+    return cap ? batch_kernel_fan<false, true>(kinds) : batch_kernel_fan<false, false>(kinds);
 }
 
-// kinds from cvfes_batch_plan (bits 0..4, at least one lane path), the caller's register cap (bit
-// 5), waves-per-SIMD cap (bits 6..8: 0 or 2..7) and sample-group-first wave order (bit 9).
+// kinds from cvfes_batch_plan (bits 0..4 and 10, at least one lane path), the caller's register cap
+// (bit 5), waves-per-SIMD cap (bits 6..8: 0 or 2..7) and sample-group-first wave order (bit 9).
 bool valid_kinds(int64_t kinds) {
     const int64_t w = (kinds >> 6) & 7;
-    return kinds >= 1 && kinds < 1024 && (kinds & 19) && (w == 0 || w >= 2);
+    return kinds >= 1 && kinds < 2 * kKindNoFan && (kinds & 19) && (w == 0 || w >= 2);
 }
 
 __global__ void k_counter_add(int64_t *counter, int64_t by) {
@@ -286,12 +361,15 @@ extern "C" int cvfes_batch_plan(void *stream, cvfes_batch_mesh_t *meshes, int n_
         }
         k |= m.vw == 1 ? 2 : (m.packed ? 16 : 1);
         if (m.method == CVFES_METHOD_STORED) k |= 4;
+        if (m.method == CVFES_METHOD_MATFREE && !fan_entries(&s)) k |= kKindNoFan;
         if (m.beta != 0.0 || m.damp != 0.0) k |= 8;
+        CVFES_REQUIRE(m.tiled == 0 || (m.tiled == 1 && cvfes_batch_can_tile(&m)),
+                      "cvfes_batch_plan: mesh %d cannot be tiled", i);
         m.lanes = m.packed ? l : padded;
         CVFES_REQUIRE(s.n_nodes * m.lanes < (int64_t(1) << 31) - 64,
                       "cvfes_batch_plan: mesh %d has too many row lanes", i);
         m.task0 = t;
-        m.n_mtasks = (s.n_nodes * m.lanes + 63) / 64;
+        m.n_mtasks = m.tiled ? 0 : (s.n_nodes * m.lanes + 63) / 64;
         m.slice = (m.n_mtasks + kNumXcd - 1) / kNumXcd;
         m.xtask0 = x;
         t += m.n_mtasks;
@@ -312,6 +390,86 @@ extern "C" int cvfes_batch_plan(void *stream, cvfes_batch_mesh_t *meshes, int n_
     return CVFES_OK;
 }
 
+extern "C" int cvfes_batch_can_tile(const cvfes_batch_mesh_t *mesh) {
+    return mesh && mesh->method == CVFES_METHOD_MATFREE && fan_entries(&mesh->sys) && mesh->sys.n_smp > kTileSmall &&
+           tiles_apply(&mesh->sys);
+}
+
+extern "C" int64_t cvfes_batch_tile_bytes(int n_mesh) {
+    return n_mesh < 1 ? -1 : static_cast<int64_t>(n_mesh) * (sizeof(BatchTiles) + sizeof(int64_t));
+}
+
+// shape: samples per chunk of the widest tiled mesh, bit 16 nodes with more than 6 elements, bit
+// 17 some mesh with beta or damp.
+extern "C" int cvfes_batch_plan_tiles(void *stream, const cvfes_batch_mesh_t *meshes, int n_mesh,
+                                      void *dev_tiles, int64_t *n_blocks, int64_t *shape) {
+    CVFES_REQUIRE(meshes && n_mesh >= 1 && dev_tiles && n_blocks && shape,
+                  "cvfes_batch_plan_tiles: bad arguments");
+    const size_t bytes = static_cast<size_t>(cvfes_batch_tile_bytes(n_mesh));
+    std::vector<char> host;
+    try {
+        host.assign(bytes, 0);
+    } catch (...) {
+        return fail(CVFES_ERR_ARG, "cvfes_batch_plan_tiles: out of host memory");
+    }
+    BatchTiles *tiles = reinterpret_cast<BatchTiles *>(host.data());
+    int64_t *first = reinterpret_cast<int64_t *>(tiles + n_mesh);
+    int64_t x = 0, chunk = 0, sh = 0;
+    for (int i = 0; i < n_mesh; ++i) {
+        const cvfes_batch_mesh_t &m = meshes[i];
+        tiles[i].first = first[i] = x;
+        if (m.tiled == 0) continue;
+        CVFES_REQUIRE(cvfes_batch_can_tile(&m), "cvfes_batch_plan_tiles: mesh %d cannot be tiled", i);
+        const TileShape h = tile_shape(m.sys.n_smp);
+        tiles[i].t = tile_args(&m.sys, h);
+        tiles[i].vw = h.vw;
+        tiles[i].slice = static_cast<int32_t>((m.sys.n_tiles * h.chunks + kNumXcd - 1) / kNumXcd);
+        x += tiles[i].slice;
+        if (h.chunk > chunk) chunk = h.chunk;
+        if (m.sys.max_node_elems > 6) sh |= 1 << 16;
+        if (m.beta != 0.0 || m.damp != 0.0) sh |= 1 << 17;
+    }
+    CVFES_REQUIRE(x * kNumXcd < (int64_t(1) << 31), "cvfes_batch_plan_tiles: too many tiles");
+    *n_blocks = x * kNumXcd;
+    *shape = sh | chunk;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    hipError_t err = hipMemcpyAsync(dev_tiles, host.data(), bytes, hipMemcpyHostToDevice, st);
+    if (err == hipSuccess) err = hipStreamSynchronize(st);
+    if (err != hipSuccess) return fail(CVFES_ERR_HIP, "cvfes_batch_plan_tiles: %s", hipGetErrorString(err));
+    return CVFES_OK;
+}
+
+namespace {
+
+bool valid_shape(int64_t shape) { return shape > 0 && shape < (1 << 18) && (shape & 0xffff) >= 1 && (shape & 0xffff) <= 64; }
+
+void launch_batch_tiles(hipStream_t st, const void *dev_meshes, const void *dev_tiles, int n_mesh,
+                        int64_t n_blocks, int64_t shape, int phase, const int64_t *counter, int64_t k_local) {
+    const bool eight = shape & (1 << 16), bd = shape & (1 << 17);
+    const auto kern = bd ? (eight ? k_batch_tile<true, 8> : k_batch_tile<true, 6>)
+                         : (eight ? k_batch_tile<false, 8> : k_batch_tile<false, 6>);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(n_blocks)), dim3(kTileThreads),
+                       tile_lds(static_cast<int>(shape & 0xffff), eight ? 8 : 6), st,
+                       static_cast<const cvfes_batch_mesh_t *>(dev_meshes),
+                       static_cast<const BatchTiles *>(dev_tiles), n_mesh, phase, counter, k_local);
+}
+
+}  // namespace
+
+extern "C" int cvfes_batch_step_tiles(void *stream, const void *dev_meshes, const void *dev_tiles, int n_mesh,
+                                      int64_t n_blocks, int64_t shape, int phase, const int64_t *counter,
+                                      int64_t k_local) {
+    CVFES_REQUIRE(dev_meshes && dev_tiles && n_mesh >= 1 && n_blocks >= 0 && n_blocks < (int64_t(1) << 31) &&
+                      n_blocks % kNumXcd == 0,
+                  "cvfes_batch_step_tiles: bad arguments");
+    CVFES_REQUIRE(phase >= 0 && phase < 3, "cvfes_batch_step_tiles: phase must be 0, 1 or 2");
+    if (n_blocks == 0) return CVFES_OK;
+    CVFES_REQUIRE(valid_shape(shape), "cvfes_batch_step_tiles: shape must come from cvfes_batch_plan_tiles");
+    launch_batch_tiles(static_cast<hipStream_t>(stream), dev_meshes, dev_tiles, n_mesh, n_blocks, shape, phase,
+                       counter, k_local);
+    return check_launch("k_batch_tile");
+}
+
 extern "C" int cvfes_batch_step(void *stream, const void *dev_meshes, int n_mesh, int64_t n_tasks,
                                 int phase, const int64_t *counter, int64_t k_local,
                                 int64_t n_waves, int64_t kinds) {
@@ -320,7 +478,7 @@ extern "C" int cvfes_batch_step(void *stream, const void *dev_meshes, int n_mesh
     CVFES_REQUIRE(valid_kinds(kinds), "cvfes_batch_step: kinds must come from cvfes_batch_plan");
     if (n_tasks == 0) return CVFES_OK;
     const int64_t w = n_waves > 0 ? n_waves : default_waves();
-    hipLaunchKernelGGL(batch_kernel(kinds & 63, w >= n_tasks), dim3(waves_to_blocks(w)), dim3(kBlock),
+    hipLaunchKernelGGL(batch_kernel(kinds, w >= n_tasks), dim3(waves_to_blocks(w)), dim3(kBlock),
                        occupancy_lds((kinds >> 6) & 7), static_cast<hipStream_t>(stream),
                        static_cast<const cvfes_batch_mesh_t *>(dev_meshes), n_mesh, n_tasks, phase,
                        counter, k_local, static_cast<int>((kinds >> 9) & 1));
@@ -334,9 +492,11 @@ extern "C" int cvfes_counter_add(void *stream, int64_t *counter, int64_t by) {
     return check_launch("k_counter_add");
 }
 
-extern "C" int cvfes_batch_graph_create(const void *dev_meshes, int n_mesh, int64_t n_tasks,
-                                        int64_t *counter, int64_t block_steps, int phase0,
-                                        int64_t n_waves, int64_t kinds, void **graph) {
+namespace {
+
+int graph_create(const void *dev_meshes, int n_mesh, int64_t n_tasks, int64_t *counter, int64_t block_steps,
+                 int phase0, int64_t n_waves, int64_t kinds, const void *dev_tiles, int64_t n_blocks,
+                 int64_t shape, bool rows, void **graph) {
     CVFES_REQUIRE(valid_kinds(kinds), "cvfes_batch_graph_create: kinds must come from cvfes_batch_plan");
     CVFES_REQUIRE(dev_meshes && n_mesh >= 1 && counter && graph, "cvfes_batch_graph_create: bad arguments");
     CVFES_REQUIRE(block_steps >= 3 && block_steps % 3 == 0,
@@ -351,12 +511,16 @@ extern "C" int cvfes_batch_graph_create(const void *dev_meshes, int n_mesh, int6
         (void)hipStreamDestroy(cs);
         return fail(CVFES_ERR_HIP, "hipStreamBeginCapture: %s", hipGetErrorString(err));
     }
-    for (int64_t k = 0; k < block_steps; ++k)
-        hipLaunchKernelGGL(batch_kernel(kinds & 63, w >= n_tasks), dim3(waves_to_blocks(w)), dim3(kBlock),
-                           occupancy_lds((kinds >> 6) & 7), cs,
-                           static_cast<const cvfes_batch_mesh_t *>(dev_meshes), n_mesh, n_tasks,
-                           static_cast<int>((phase0 + k) % 3), counter, k,
-                           static_cast<int>((kinds >> 9) & 1));
+    for (int64_t k = 0; k < block_steps; ++k) {
+        const int phase = static_cast<int>((phase0 + k) % 3);
+        if (rows)
+            hipLaunchKernelGGL(batch_kernel(kinds, w >= n_tasks), dim3(waves_to_blocks(w)), dim3(kBlock),
+                               occupancy_lds((kinds >> 6) & 7), cs,
+                               static_cast<const cvfes_batch_mesh_t *>(dev_meshes), n_mesh, n_tasks, phase,
+                               counter, k, static_cast<int>((kinds >> 9) & 1));
+        if (n_blocks > 0)
+            launch_batch_tiles(cs, dev_meshes, dev_tiles, n_mesh, n_blocks, shape, phase, counter, k);
+    }
     hipLaunchKernelGGL(k_counter_add, dim3(1), dim3(64), 0, cs, counter, block_steps);
     hipGraph_t g = nullptr;
     err = hipStreamEndCapture(cs, &g);
@@ -367,6 +531,26 @@ extern "C" int cvfes_batch_graph_create(const void *dev_meshes, int n_mesh, int6
     if (err != hipSuccess) return fail(CVFES_ERR_HIP, "graph capture: %s", hipGetErrorString(err));
     *graph = exec;
     return CVFES_OK;
+}
+
+}  // namespace
+
+extern "C" int cvfes_batch_graph_create(const void *dev_meshes, int n_mesh, int64_t n_tasks,
+                                        int64_t *counter, int64_t block_steps, int phase0,
+                                        int64_t n_waves, int64_t kinds, void **graph) {
+    return graph_create(dev_meshes, n_mesh, n_tasks, counter, block_steps, phase0, n_waves, kinds, nullptr, 0, 0,
+                        true, graph);
+}
+
+extern "C" int cvfes_batch_graph_create_tiles(const void *dev_meshes, int n_mesh, int64_t n_tasks,
+                                              int64_t *counter, int64_t block_steps, int phase0,
+                                              int64_t n_waves, int64_t kinds, const void *dev_tiles,
+                                              int64_t n_blocks, int64_t shape, void **graph) {
+    CVFES_REQUIRE(n_tasks >= 0 && n_blocks >= 0 && n_blocks < (int64_t(1) << 31) && n_blocks % kNumXcd == 0 &&
+                      (n_blocks == 0 || (dev_tiles && valid_shape(shape))),
+                  "cvfes_batch_graph_create_tiles: n_blocks and shape must come from cvfes_batch_plan_tiles");
+    return graph_create(dev_meshes, n_mesh, n_tasks, counter, block_steps, phase0, n_waves, kinds, dev_tiles,
+                        n_blocks, shape, n_tasks > 0, graph);
 }
 
 extern "C" int cvfes_graph_launch(void *graph, void *stream) {

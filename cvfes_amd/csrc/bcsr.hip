@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "rowops.h"
+#include "tile.h"
 
 namespace cvfes {
 namespace {
@@ -29,7 +30,18 @@ __global__ __launch_bounds__(kBlock) void k_spmv(StepArgs a) {
     bool active;
     if (!row_and_sample<UNIFORM, VW>(a.k.n_nodes, a.k.n_smp, row, s, active)) return;
     double acc[3][VW];
-    row_product<OP, false, VW>(a.k, a.u, static_cast<const double *>(nullptr), 0.0, row, s, acc);
+    if constexpr (OP == kOpFan) {
+        typedef StateCol<UNIFORM, false, VW, const double *> Col;
+        const Col col{a.u, nullptr, 0.0, a.k.n_smp, static_cast<uint32_t>(s) * 8u};
+        double y[1][3][VW];
+        fan_product<UNIFORM, VW>(a.k, col, row, y);
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int v = 0; v < VW; ++v) acc[i][v] = y[0][i][v];
+    } else {
+        row_product<OP, false, VW>(a.k, a.u, static_cast<const double *>(nullptr), 0.0, row, s, acc);
+    }
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         Vec<VW> o;
@@ -39,8 +51,11 @@ __global__ __launch_bounds__(kBlock) void k_spmv(StepArgs a) {
     }
 }
 
+#ifndef X_W
+#define X_W 1
+#endif
 template <int OP, bool UNIFORM, bool BETA, bool DAMP, int VW>
-__global__ __launch_bounds__(kBlock) void k_step(StepArgs a, int64_t step) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OP == kOpFan && !UNIFORM ? X_W : 1))) void k_step(StepArgs a, int64_t step) {
     int32_t row;
     int64_t s;
     bool active;
@@ -48,7 +63,14 @@ __global__ __launch_bounds__(kBlock) void k_step(StepArgs a, int64_t step) {
     if constexpr (UNIFORM) {
         if (a.order) row = a.order[row];
     }
-    step_row<OP, BETA, DAMP, VW>(a, row, s, active, step);
+    step_row<OP, UNIFORM, BETA, DAMP, VW>(a, row, s, active, step);
+}
+
+// The matrix-free step by node tiles (tile.h); the bits are those of k_step<kOpFan>.
+template <bool BETA, bool DAMP, int VW, int ELEMS, bool SMALL>
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void k_step_tile(StepArgs a, TileArgs t, int64_t step) {
+    tile_step<BETA, DAMP, VW, ELEMS, SMALL>(a, t, static_cast<uint32_t>(xcd_block()), step);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -374,7 +396,8 @@ int validate(const cvfes_system_t *sys, int method, const char *who) {
 
 RowArgs row_args(const cvfes_system_t *sys) {
     return RowArgs{sys->n_nodes, sys->n_smp, sys->indptr, sys->indices, sys->values,
-                   sys->cptr,    sys->celem, sys->khat,   sys->coef, sys->uvalues, sys->vblk};
+                   sys->cptr,    sys->celem, sys->khat,   sys->coef, sys->uvalues, sys->vblk,
+                   sys->nptr,    fan_entries(sys)};
 }
 
 // Dispatch helpers ------------------------------------------------------------------------------
@@ -403,11 +426,13 @@ void spmv_op(hipStream_t st, const StepArgs &a) {
 // Operator form of the generic row kernels: matrix-free, or the stored values in the storage
 // the system holds (full values when present, else the symmetric upper blocks).
 int row_op(const RowArgs &k, bool mf) {
-    return mf ? kOpMatfree : (k.values ? kOpStored : kOpSym);
+    if (mf) return k.fan ? kOpFan : kOpMatfree;
+    return k.values ? kOpStored : kOpSym;
 }
 
 void spmv_dispatch(hipStream_t st, bool mf, const StepArgs &a) {
     switch (row_op(a.k, mf)) {
+    case kOpFan: spmv_op<kOpFan>(st, a); break;
     case kOpMatfree: spmv_op<kOpMatfree>(st, a); break;
     case kOpStored: spmv_op<kOpStored>(st, a); break;
     default: spmv_op<kOpSym>(st, a); break;
@@ -438,6 +463,43 @@ void step_u(hipStream_t st, const StepArgs &a, int64_t step, bool beta, bool dam
         step_bd<OP, true, VW>(st, a, step, beta, damp);
     else
         step_bd<OP, false, VW>(st, a, step, beta, damp);
+}
+
+template <int VW, int ELEMS, bool SMALL>
+void launch_step_tile(hipStream_t st, const StepArgs &a, const TileArgs &t, const TileShape &h, int64_t step,
+                      bool beta, bool damp) {
+    const dim3 grid(tile_grid(t)), block(64 * h.waves);
+    const size_t lds = tile_lds(h.chunk, ELEMS);
+    if (beta) {
+        if (damp) hipLaunchKernelGGL((k_step_tile<true, true, VW, ELEMS, SMALL>), grid, block, lds, st, a, t, step);
+        else hipLaunchKernelGGL((k_step_tile<true, false, VW, ELEMS, SMALL>), grid, block, lds, st, a, t, step);
+    } else {
+        if (damp) hipLaunchKernelGGL((k_step_tile<false, true, VW, ELEMS, SMALL>), grid, block, lds, st, a, t, step);
+        else hipLaunchKernelGGL((k_step_tile<false, false, VW, ELEMS, SMALL>), grid, block, lds, st, a, t, step);
+    }
+}
+
+void step_tile(hipStream_t st, const cvfes_system_t *sys, const StepArgs &a, int64_t step, bool beta, bool damp) {
+    const TileShape h = tile_shape(sys->n_smp);
+    const TileArgs t = tile_args(sys, h);
+    const bool six = sys->max_node_elems <= 6, small = sys->n_smp <= kTileSmall;
+    if (h.vw == 2) {
+        if (small) {
+            if (six) launch_step_tile<2, 6, true>(st, a, t, h, step, beta, damp);
+            else launch_step_tile<2, 8, true>(st, a, t, h, step, beta, damp);
+        } else {
+            if (six) launch_step_tile<2, 6, false>(st, a, t, h, step, beta, damp);
+            else launch_step_tile<2, 8, false>(st, a, t, h, step, beta, damp);
+        }
+    } else {
+        if (small) {
+            if (six) launch_step_tile<1, 6, true>(st, a, t, h, step, beta, damp);
+            else launch_step_tile<1, 8, true>(st, a, t, h, step, beta, damp);
+        } else {
+            if (six) launch_step_tile<1, 6, false>(st, a, t, h, step, beta, damp);
+            else launch_step_tile<1, 8, false>(st, a, t, h, step, beta, damp);
+        }
+    }
 }
 
 template <int OP>
@@ -781,7 +843,12 @@ void step_dispatch(hipStream_t st, const cvfes_system_t *sys, bool mf, const Ste
     default:
         break;
     }
+    if (mf && a.k.fan && tiles_apply(sys)) {
+        step_tile(st, sys, a, step, beta, damp);
+        return;
+    }
     switch (row_op(a.k, mf)) {
+    case kOpFan: step_generic<kOpFan>(st, a, step, beta, damp); break;
     case kOpMatfree: step_generic<kOpMatfree>(st, a, step, beta, damp); break;
     case kOpStored: step_generic<kOpStored>(st, a, step, beta, damp); break;
     default: step_generic<kOpSym>(st, a, step, beta, damp); break;

@@ -71,9 +71,9 @@ inline unsigned occupancy_lds(int64_t w) {
 // that XCD k processes the k-th contiguous slice of the logical block range: consecutive block
 // rows then share one L2, which is where their common neighbour columns are cached.
 __device__ __forceinline__ int64_t xcd_block() {
-    const int64_t b = blockIdx.x;
-    const int64_t per = gridDim.x / kNumXcd;
-    return (b % kNumXcd) * per + b / kNumXcd;
+    const uint32_t b = blockIdx.x;
+    const uint32_t per = gridDim.x / kNumXcd;
+    return static_cast<int64_t>((b % kNumXcd) * per + b / kNumXcd);
 }
 
 template <int VW>
@@ -140,6 +140,18 @@ __device__ __forceinline__ void store_vec(CVFES_G double *__restrict__ p, const 
 #pragma unroll
         for (int k = 0; k < VW; ++k) p[k] = r.v[k];
     }
+}
+
+// VW consecutive doubles at a (usually wave-uniform) base and a 32-bit byte offset per lane: the
+// base stays in scalar registers and the lane needs one address register for all its loads.
+template <int VW>
+__device__ __forceinline__ Vec<VW> load_lane(const double *__restrict__ base, uint32_t lane) {
+    return load_vec<VW>(reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + lane));
+}
+
+template <int VW>
+__device__ __forceinline__ Vec<VW> load_lane(const CVFES_G double *__restrict__ base, uint32_t lane) {
+    return load_vec<VW>((const CVFES_G double *)((const CVFES_G char *)base + lane));
 }
 
 // Non-temporal stores of VW consecutive samples, as one 16-byte store for VW = 2 (two 8-byte

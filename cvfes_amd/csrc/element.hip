@@ -122,6 +122,48 @@ __global__ __launch_bounds__(kBlock) void k_lumped_mass_load(
     }
 }
 
+// Fan entries of one node per thread: the incident elements in list order, then sorted in place.
+// Each slot takes the first remaining entry whose p is the previous entry's q; where there is
+// none, the first remaining entry whose p no remaining entry leads to (the start of an open fan),
+// else simply the next.  Nodes have a handful of elements; beyond kFanSort they stay in list order.
+constexpr int kFanSort = 32;
+
+__global__ __launch_bounds__(kBlock) void k_node_fans(int64_t n_nodes, const int32_t *__restrict__ nptr,
+                                                      const int32_t *__restrict__ nent,
+                                                      const int32_t *__restrict__ elems,
+                                                      const int32_t *__restrict__ cpos, int4 *fan) {
+    const int64_t a = xcd_block() * kBlock + threadIdx.x;
+    if (a >= n_nodes) return;
+    const int32_t q0 = nptr[a], n = nptr[a + 1] - q0;
+    int4 *f = fan + q0;
+    for (int i = 0; i < n; ++i) {
+        const int32_t e = nent[q0 + i] / 3, la = nent[q0 + i] - 3 * e;
+        const int lp = (la + 1) % 3, lq = (la + 2) % 3;
+        const int32_t *c = cpos + 9 * static_cast<int64_t>(e) + 3 * la;
+        const int32_t c0 = 3 * q0;
+        f[i] = make_int4(elems[3 * static_cast<int64_t>(e) + lp], elems[3 * static_cast<int64_t>(e) + lq], e,
+                         (c[la] - c0) | (c[lp] - c0) << 10 | (c[lq] - c0) << 20);
+    }
+    if (n > kFanSort) return;
+    for (int i = 0; i < n; ++i) {
+        int take = -1, start = i;
+        for (int j = i; i > 0 && j < n && take < 0; ++j)
+            if (f[j].x == f[i - 1].y) take = j;
+        bool open = false;
+        for (int j = i; take < 0 && !open && j < n; ++j) {
+            open = true;
+            for (int m = i; m < n; ++m) open = open && f[m].y != f[j].x;
+            if (open) start = j;
+        }
+        const int j = take < 0 ? start : take;
+        const int4 t = f[j];
+        f[j] = f[i];
+        f[i] = t;
+    }
+    for (int i = n - 1; i > 0; --i)
+        if (f[i].x == f[i - 1].y) f[i].x = -1;
+}
+
 }  // namespace
 }  // namespace cvfes
 
@@ -172,4 +214,19 @@ extern "C" int cvfes_lumped_mass_load(void *stream, int64_t n_nodes, int64_t n_s
                        static_cast<hipStream_t>(stream), n_nodes, n_lm_smp, n_smp, nptr, nent,
                        elems, area, normal, vthick, thick_sstride, density, mass_scale, lm, f1);
     return check_launch("k_lumped_mass_load");
+}
+
+extern "C" int cvfes_node_fans(void *stream, int64_t n_nodes, int64_t max_node_elems,
+                               const int32_t *nptr, const int32_t *nent, const int32_t *elems,
+                               const int32_t *cpos, int32_t *fan) {
+    CVFES_REQUIRE(n_nodes >= 0, "cvfes_node_fans: n_nodes < 0");
+    if (n_nodes == 0) return CVFES_OK;
+    CVFES_REQUIRE(max_node_elems >= 1 && max_node_elems <= CVFES_FAN_MAX_ELEMS,
+                  "cvfes_node_fans: max_node_elems must be 1..%d", CVFES_FAN_MAX_ELEMS);
+    CVFES_REQUIRE(nptr && nent && elems && cpos && fan, "cvfes_node_fans: null pointer");
+    CVFES_REQUIRE(reinterpret_cast<uintptr_t>(fan) % 16 == 0, "cvfes_node_fans: fan must be 16-byte aligned");
+    hipLaunchKernelGGL(k_node_fans, dim3(grid_for(n_nodes)), dim3(kBlock), 0,
+                       static_cast<hipStream_t>(stream), n_nodes, nptr, nent, elems, cpos,
+                       reinterpret_cast<int4 *>(fan));
+    return check_launch("k_node_fans");
 }

@@ -49,9 +49,17 @@ inline int generic_vw(int64_t n_smp) {
 
 // Operator forms of the row functions (template argument OP): stored values in full storage,
 // matrix-free (element coefficients x unit element blocks), stored values in symmetric storage.
+// kOpFan is the matrix-free operator walked element by element around the row node
+// (cvfes_system_t.fan); kOpMatfree walks it block by block (systems without fan entries).
 constexpr int kOpStored = 0;
 constexpr int kOpMatfree = 1;
 constexpr int kOpSym = 2;
+constexpr int kOpFan = 3;
+
+// One fan entry: the element e incident to the row node, its two other nodes p and q, and the
+// positions of its blocks (row, row), (row, p), (row, q) among the row's contributions, 10 bits
+// each (`pk`).  p is -1 where it is the previous entry's q.
+typedef int32_t fan_t __attribute__((ext_vector_type(4)));
 
 // Stored operator: full storage `values` [nnzb][9][S], or, when `values` is null, symmetric
 // storage: the upper blocks `uvalues` [nnzu][9][S], block p of the row structure being
@@ -68,7 +76,20 @@ struct RowArgs {
     const double *coef;
     const double *uvalues;
     const int32_t *vblk;
+    const int32_t *nptr;
+    const fan_t *fan;      // null: the matrix-free operator is walked block by block
 };
+
+// The fan entries a kernel may use: the lane offsets of the fan product are 32-bit bytes.
+inline const fan_t *fan_entries(const cvfes_system_t *sys) {
+    return sys->nptr && sys->n_smp < (int64_t(1) << 28) ? reinterpret_cast<const fan_t *>(sys->fan) : nullptr;
+}
+
+// Node tiles (tile.h): rows per tile, column slots (39 of 64 samples and the unit blocks of 16
+// rows of 6 elements fit half a CU's LDS), and most elements around a node.
+constexpr int kTileRows = CVFES_TILE_ROWS;
+constexpr int kTileCols = CVFES_TILE_COLS;
+constexpr int kTileElems = CVFES_TILE_ELEMS;
 
 struct StepArgs {
     RowArgs k;
@@ -105,6 +126,8 @@ struct GRowArgs {
     const CVFES_G double *coef;
     const CVFES_G double *uvalues;
     const CVFES_K int32_t *vblk;
+    const CVFES_K int32_t *nptr;
+    const CVFES_K fan_t *fan;
 };
 
 struct GLoad {
@@ -247,72 +270,6 @@ __device__ __forceinline__ void block_apply2(const RA &k, int32_t p, bool tr, in
     }
 }
 
-// acc[i][v] = sum over the row's blocks of K_p (i, :) . x_col, with x = u + bdt (u - up) when BETA.
-template <int OP, bool BETA, int VW, class RA, class DP>
-__device__ __forceinline__ void row_product(const RA &k, DP u, DP up, double bdt, int32_t row,
-                                            int64_t s, double (&acc)[3][VW]) {
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int v = 0; v < VW; ++v) acc[i][v] = 0.0;
-    const int32_t p0 = k.indptr[row], p1 = k.indptr[row + 1];
-    for (int32_t p = p0; p < p1; ++p) {
-        const int64_t col = k.indices[p];
-        double x[3][VW];
-        state_column<BETA, VW>(u, up, bdt, col, k.n_smp, s, x);
-        block_apply<OP, VW>(k, p, col < row, s, x, acc);
-    }
-}
-
-// Central-difference update of one block row and VW consecutive samples from its product
-// acc = K x: load, damping, lumped mass and Dirichlet value; stores u_{n+1} when `active`.  Every
-// product and sum that could be contracted is an explicit fma, so the rounding is the same in
-// every kernel that uses it (single-mesh, batched, and the step fused with the adjoint).
-template <bool DAMP, int VW, class SA>
-__device__ __forceinline__ void step_update(const SA &a, int32_t row, int64_t s, bool active,
-                                            int64_t step, const double (&acc)[3][VW]) {
-    const double pn = a.load.p[step];
-    const double qa = a.load.ga ? a.load.qa[step] : 0.0;
-    const double qb = a.load.gb ? a.load.qb[step] : 0.0;
-    const bool fixed = a.fixed != nullptr && a.fixed[row] != 0;
-    const int64_t nsm = a.k.n_smp;
-    const auto *lmp = a.lm + (a.lm_sstride ? static_cast<int64_t>(row) * nsm + s : row);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const int64_t off = (static_cast<int64_t>(row) * 3 + i) * nsm + s;
-        const Vec<VW> uu = load_vec<VW>(a.u + off);
-        const Vec<VW> pp = load_vec<VW>(a.up + off);
-        const int64_t d = 3 * static_cast<int64_t>(row) + i;
-        double fi = pn * a.f1[d];
-        if (a.load.ga) fi = fma(qa, a.load.ga[d], fi);
-        if (a.load.gb) fi = fma(qb, a.load.gb[d], fi);
-        Vec<VW> o;
-#pragma unroll
-        for (int v = 0; v < VW; ++v) {
-            const double m = a.lm_sstride ? lmp[v] : lmp[0];
-            double force = fi;
-            if constexpr (DAMP) force = fma(-a.ddt, uu.v[v] - pp.v[v], force);
-            const double rhs = fma(a.dt2, force - acc[i][v], m * fma(2.0, uu.v[v], -pp.v[v]));
-            double un = m != 0.0 ? rhs / m : 0.0;
-            o.v[v] = fixed ? a.bdy_u : un;
-        }
-        // u_{n+1} is not read again in this launch: large outputs are streamed past L2 (stream_out)
-        if (active) {
-            if (a.nt_out) store_vec_nt<VW>(a.out + off, o);
-            else store_vec<VW>(a.out + off, o);
-        }
-    }
-}
-
-// Block-row product and central-difference update of one block row and VW consecutive samples.
-template <int OP, bool BETA, bool DAMP, int VW, class SA>
-__device__ __forceinline__ void step_row(const SA &a, int32_t row, int64_t s, bool active,
-                                         int64_t step) {
-    double acc[3][VW];
-    row_product<OP, BETA, VW>(a.k, a.u, a.up, a.bdt, row, s, acc);
-    step_update<DAMP, VW>(a, row, s, active, step, acc);
-}
-
 // ---------------------------------------------------------------------------------------------
 // Ext-vector forms (one value or two consecutive samples per lane) used by the row-load and
 // LDS-staged kernels.
@@ -368,6 +325,267 @@ __device__ __forceinline__ Vec<VW> to_vec(typename VecT<VW>::type t) {
     return r;
 }
 
+// The three components of a node's state, VW consecutive samples per lane at the lane's byte offset
+// `lane`.  Wave-uniform rows (UNI): buffer loads (below: one address register per lane).
+template <bool UNI, int VW, class DP>
+__device__ __forceinline__ void load_node(DP base, int32_t node, int64_t n_smp, uint32_t lane,
+                                          Vec<VW> (&r)[3]) {
+    if constexpr (UNI) {
+        const uint32_t sb = static_cast<uint32_t>(n_smp) * 8u;
+        const auto rs = buffer_rsrc((const double *)(base + static_cast<int64_t>(node) * 3 * n_smp), 3 * sb);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) r[j] = to_vec<VW>(ldb<VW, 0>(rs, lane, j * sb));
+    } else {
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            r[j] = load_lane<VW>(base + (static_cast<int64_t>(node) * 3 + j) * n_smp, lane);
+    }
+}
+
+// One value per sample of row `i` of an [..][S] array.
+template <bool UNI, int VW, class DP>
+__device__ __forceinline__ Vec<VW> load_entry(DP base, int64_t i, int64_t n_smp, uint32_t lane) {
+    if constexpr (UNI) {
+        const uint32_t sb = static_cast<uint32_t>(n_smp) * 8u;
+        return to_vec<VW>(ldb<VW, 0>(buffer_rsrc((const double *)(base + i * n_smp), sb), lane, 0));
+    } else {
+        return load_lane<VW>(base + i * n_smp, lane);
+    }
+}
+
+// Columns of the fan product: load() issues a node's loads, column() forms the column from them,
+// own() issues what the update of a row needs of its own node.  kCols columns share every
+// operator load (the fused forward + adjoint step applies two).
+template <bool UNI, bool BETA, int VW, class DP>
+struct StateCol {
+    static constexpr int kCols = 1;
+    struct Raw {
+        Vec<VW> u[3], up[3];
+    };
+    typedef Raw Own;
+    DP u, up;
+    double bdt;
+    int64_t n_smp;
+    uint32_t lane;          // the lane's byte offset in every row (its first sample)
+
+    __device__ __forceinline__ Raw load(int32_t node) const {
+        Raw r;
+        load_node<UNI, VW>(u, node, n_smp, lane, r.u);
+        if constexpr (BETA) load_node<UNI, VW>(up, node, n_smp, lane, r.up);
+        return r;
+    }
+    __device__ __forceinline__ Own own(int32_t node) const {
+        Own o;
+        load_node<UNI, VW>(u, node, n_smp, lane, o.u);
+        load_node<UNI, VW>(up, node, n_smp, lane, o.up);
+        return o;
+    }
+    __device__ __forceinline__ void column(const Raw &r, double (&x)[3][VW]) const {
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int v = 0; v < VW; ++v)
+                x[j][v] = BETA ? fma(bdt, r.u[j].v[v] - r.up[j].v[v], r.u[j].v[v]) : r.u[j].v[v];
+    }
+    __device__ __forceinline__ void value(const Raw &r, double (&x)[1][3][VW]) const { column(r, x[0]); }
+};
+
+// acc[c] = the row's matrix-free product with each column c: for every element e around the row
+// node a, with p and q its other nodes, acc += coef_e (khat_e(a,a) x_a + khat_e(a,p) x_p +
+// khat_e(a,q) x_q).  Compared with the walk over blocks, the coefficient is read and applied once
+// per element instead of once per contribution, and where the entries chain around the node each
+// neighbour is read once.  The next element's loads are issued before the current one is applied.
+// A row's contributions are contiguous, so its unit blocks start at contribution 3 nptr[row].
+template <bool UNI, int VW, class COL, class RA>
+__device__ __forceinline__ void fan_product(const RA &k, const COL &col, int32_t row,
+                                            double (&acc)[COL::kCols][3][VW]) {
+    constexpr int NC = COL::kCols;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int v = 0; v < VW; ++v) acc[c][i][v] = 0.0;
+    const int32_t q0 = k.nptr[row], q1 = k.nptr[row + 1];
+    if (q0 == q1) return;
+    const auto *kh0 = k.khat + 27 * static_cast<int64_t>(q0);
+    double xa[NC][3][VW], xp[NC][3][VW], xq[NC][3][VW];
+    fan_t e = k.fan[q0];
+    typename COL::Raw r = col.load(e.y);
+    Vec<VW> c = load_entry<UNI, VW>(k.coef, e.z, k.n_smp, col.lane);
+    {
+        const typename COL::Raw ra = col.load(row), rp = col.load(e.x);
+        col.value(ra, xa);
+        col.value(rp, xp);
+    }
+    for (int32_t q = q0 + 1;; ++q) {
+        const fan_t n = k.fan[q < q1 ? q : q1 - 1];
+        col.value(r, xq);
+        const Vec<VW> cf = c;
+        r = col.load(n.y);              // behind the last element: its own node again
+        c = load_entry<UNI, VW>(k.coef, n.z, k.n_smp, col.lane);
+        __builtin_amdgcn_sched_barrier(0);
+        const auto *ka = kh0 + 9 * (e.w & 1023);
+        const auto *kp = kh0 + 9 * ((e.w >> 10) & 1023);
+        const auto *kq = kh0 + 9 * ((e.w >> 20) & 1023);
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int m = 0; m < NC; ++m)
+#pragma unroll
+                for (int v = 0; v < VW; ++v) {
+                    double t = ka[3 * i] * xa[m][0][v];
+                    t = fma(ka[3 * i + 1], xa[m][1][v], t);
+                    t = fma(ka[3 * i + 2], xa[m][2][v], t);
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) t = fma(kp[3 * i + j], xp[m][j][v], t);
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) t = fma(kq[3 * i + j], xq[m][j][v], t);
+                    acc[m][i][v] = fma(cf.v[v], t, acc[m][i][v]);
+                }
+        if (q >= q1) break;
+        if (n.x >= 0) {
+            col.value(col.load(n.x), xp);
+        } else {
+#pragma unroll
+            for (int m = 0; m < NC; ++m)
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+#pragma unroll
+                    for (int v = 0; v < VW; ++v) xp[m][j][v] = xq[m][j][v];
+        }
+        e = n;
+    }
+}
+
+// acc[i][v] = sum over the row's blocks of K_p (i, :) . x_col, with x = u + bdt (u - up) when BETA.
+template <int OP, bool BETA, int VW, class RA, class DP>
+__device__ __forceinline__ void row_product(const RA &k, DP u, DP up, double bdt, int32_t row,
+                                            int64_t s, double (&acc)[3][VW]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int v = 0; v < VW; ++v) acc[i][v] = 0.0;
+    const int32_t p0 = k.indptr[row], p1 = k.indptr[row + 1];
+    for (int32_t p = p0; p < p1; ++p) {
+        const int64_t col = k.indices[p];
+        double x[3][VW];
+        state_column<BETA, VW>(u, up, bdt, col, k.n_smp, s, x);
+        block_apply<OP, VW>(k, p, col < row, s, x, acc);
+    }
+}
+
+// What the update of a row reads besides its states: unit load, lumped mass, whether the node is
+// fixed.
+template <int VW>
+struct RowLoad {
+    double f1[3];
+    Vec<VW> m;
+    bool fixed;
+};
+
+template <int VW, class SA>
+__device__ __forceinline__ RowLoad<VW> row_load(const SA &a, int32_t row, int64_t s) {
+    RowLoad<VW> r;
+    r.fixed = a.fixed != nullptr && a.fixed[row] != 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) r.f1[i] = a.f1[3 * static_cast<int64_t>(row) + i];
+    if (a.lm_sstride) {
+        const auto *lmp = a.lm + (static_cast<int64_t>(row) * a.k.n_smp + s);
+#pragma unroll
+        for (int v = 0; v < VW; ++v) r.m.v[v] = lmp[v];
+    } else {
+        const double mr = a.lm[row];
+#pragma unroll
+        for (int v = 0; v < VW; ++v) r.m.v[v] = mr;
+    }
+    return r;
+}
+
+// Central-difference update of one block row and VW consecutive samples from its product
+// acc = K x and its own state uu = u_n, pp = u_{n-1}: load, damping, lumped mass and Dirichlet
+// value; stores u_{n+1} when `active`.  Every product and sum that could be contracted is an
+// explicit fma, so the rounding is the same in every kernel that uses it (single-mesh, batched,
+// and the step fused with the adjoint).  Everything the update reads is read before its first
+// store: behind a store the compiler no longer takes the row's masses and loads through scalar
+// loads, and the three components would wait for memory one after the other.
+template <bool DAMP, int VW, class SA>
+__device__ __forceinline__ void step_update(const SA &a, int32_t row, int64_t s, bool active,
+                                            int64_t step, const RowLoad<VW> &r,
+                                            const double (&acc)[3][VW], const Vec<VW> (&uu)[3],
+                                            const Vec<VW> (&pp)[3]) {
+    const int64_t nsm = a.k.n_smp;
+    const double pn = a.load.p[step];
+    double fi[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) fi[i] = pn * r.f1[i];
+    if (a.load.ga) {
+        const double qa = a.load.qa[step];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) fi[i] = fma(qa, a.load.ga[3 * static_cast<int64_t>(row) + i], fi[i]);
+    }
+    if (a.load.gb) {
+        const double qb = a.load.qb[step];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) fi[i] = fma(qb, a.load.gb[3 * static_cast<int64_t>(row) + i], fi[i]);
+    }
+    Vec<VW> o[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+#pragma unroll
+        for (int v = 0; v < VW; ++v) {
+            double force = fi[i];
+            if constexpr (DAMP) force = fma(-a.ddt, uu[i].v[v] - pp[i].v[v], force);
+            const double rhs = fma(a.dt2, force - acc[i][v], r.m.v[v] * fma(2.0, uu[i].v[v], -pp[i].v[v]));
+            const double un = r.m.v[v] != 0.0 ? rhs / r.m.v[v] : 0.0;
+            o[i].v[v] = r.fixed ? a.bdy_u : un;
+        }
+    }
+    // u_{n+1} is not read again in this launch: large outputs are streamed past L2 (stream_out)
+    if (active) {
+        auto *out = a.out + static_cast<int64_t>(row) * 3 * nsm + s;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            if (a.nt_out) store_vec_nt<VW>(out + i * nsm, o[i]);
+            else store_vec<VW>(out + i * nsm, o[i]);
+        }
+    }
+}
+
+// The same with the row's own state read here.
+template <bool DAMP, int VW, class SA>
+__device__ __forceinline__ void step_update(const SA &a, int32_t row, int64_t s, bool active,
+                                            int64_t step, const double (&acc)[3][VW]) {
+    Vec<VW> uu[3], pp[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int64_t off = (static_cast<int64_t>(row) * 3 + i) * a.k.n_smp + s;
+        uu[i] = load_vec<VW>(a.u + off);
+        pp[i] = load_vec<VW>(a.up + off);
+    }
+    step_update<DAMP, VW>(a, row, s, active, step, row_load<VW>(a, row, s), acc, uu, pp);
+}
+
+// Block-row product and central-difference update of one block row and VW consecutive samples.
+// UNI: the row is wave-uniform.
+template <int OP, bool UNI, bool BETA, bool DAMP, int VW, class SA>
+__device__ __forceinline__ void step_row(const SA &a, int32_t row, int64_t s, bool active,
+                                         int64_t step) {
+    if constexpr (OP == kOpFan) {
+        typedef StateCol<UNI, BETA, VW, decltype(a.u)> Col;
+        const Col col{a.u, a.up, a.bdt, a.k.n_smp, static_cast<uint32_t>(s) * 8u};
+        double acc[1][3][VW];
+        fan_product<UNI, VW>(a.k, col, row, acc);
+        step_update<DAMP, VW>(a, row, s, active, step, acc[0]);
+    } else {
+        double acc[3][VW];
+        row_product<OP, BETA, VW>(a.k, a.u, a.up, a.bdt, row, s, acc);
+        step_update<DAMP, VW>(a, row, s, active, step, acc);
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Helpers of the row-load and LDS-staged kernels.
 template <int VW>
 __device__ __forceinline__ typename VecT<VW>::type splat(double x) {
     if constexpr (VW == 2) return dbl2{x, x};

@@ -1,0 +1,150 @@
+// Node tiles of the matrix-free tile kernels (tile.h): compact groups of at most kTileRows nodes
+// found on the host by recursive bisection of the node cloud, and the per-tile lists the kernels
+// read, built on the device from the fan entries.
+#include <algorithm>
+#include <limits>
+#include <vector>
+
+#include "rowops.h"
+
+namespace cvfes {
+namespace {
+
+// Distinct columns of the block rows ids[0..n), at most `most + 1` of them counted.
+int count_columns(const int32_t *ids, int n, const int32_t *indptr, const int32_t *indices, int most) {
+    int32_t seen[kTileCols + 1];
+    int m = 0;
+    for (int i = 0; i < n; ++i)
+        for (int32_t p = indptr[ids[i]]; p < indptr[ids[i] + 1]; ++p) {
+            int j = 0;
+            while (j < m && seen[j] != indices[p]) ++j;
+            if (j < m) continue;
+            if (m == most) return most + 1;
+            seen[m++] = indices[p];
+        }
+    return m;
+}
+
+// Halve the nodes across their longest extent, on a multiple of the tile size, until a part is a
+// tile; a tile with too many columns is halved again.
+int64_t bisect(const double *nodes, const int32_t *indptr, const int32_t *indices, int64_t n_nodes,
+               int32_t *rows, int64_t cap) {
+    std::vector<int32_t> ids(n_nodes);
+    for (int64_t i = 0; i < n_nodes; ++i) ids[i] = static_cast<int32_t>(i);
+    std::vector<std::pair<int64_t, int64_t>> todo{{0, n_nodes}};
+    int64_t n_tiles = 0;
+    while (!todo.empty()) {
+        const auto [a, b] = todo.back();
+        todo.pop_back();
+        const int64_t n = b - a;
+        const int most = kTileCols - kTileRows + static_cast<int>(n);      // its rows and the halo slots
+        if (n == 1 || (n <= kTileRows &&
+                       count_columns(&ids[a], static_cast<int>(n), indptr, indices, most) <= most)) {
+            if (n_tiles == cap) return -1;
+            std::sort(ids.begin() + a, ids.begin() + b);
+            for (int i = 0; i < kTileRows; ++i) rows[n_tiles * kTileRows + i] = i < n ? ids[a + i] : -1;
+            ++n_tiles;
+            continue;
+        }
+        double lo[3], hi[3];
+        for (int k = 0; k < 3; ++k) {
+            lo[k] = std::numeric_limits<double>::infinity();
+            hi[k] = -lo[k];
+            for (int64_t i = a; i < b; ++i) {
+                const double x = nodes[3 * static_cast<int64_t>(ids[i]) + k];
+                if (x < lo[k]) lo[k] = x;
+                if (x > hi[k]) hi[k] = x;
+            }
+        }
+        int ax = 0;
+        for (int k = 1; k < 3; ++k)
+            if (hi[k] - lo[k] > hi[ax] - lo[ax]) ax = k;
+        const int64_t whole = (n + kTileRows - 1) / kTileRows;
+        const int64_t h = n > kTileRows ? whole / 2 * kTileRows : n / 2;
+        const auto key = [&](int32_t i) {                  // NaN last: a strict order for any input
+            const double x = nodes[3 * static_cast<int64_t>(i) + ax];
+            return x == x ? x : std::numeric_limits<double>::infinity();
+        };
+        std::nth_element(ids.begin() + a, ids.begin() + a + h, ids.begin() + b, [&](int32_t i, int32_t j) {
+            const double x = key(i), y = key(j);
+            return x != y ? x < y : i < j;
+        });
+        todo.push_back({a + h, b});
+        todo.push_back({a, a + h});
+    }
+    return n_tiles;
+}
+
+// One wavefront per tile: lane c holds the node of column slot c (rows first, then the halo in the
+// order the entries name it); every node of the entries is looked up with a ballot.
+__global__ __launch_bounds__(kBlock) void k_tile_lists(int64_t n_tiles, const int32_t *__restrict__ rows,
+                                                       const int32_t *__restrict__ nptr,
+                                                       const fan_t *__restrict__ fan, int4 *__restrict__ head,
+                                                       int32_t *__restrict__ cols, int2 *__restrict__ ents) {
+    const int64_t t = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) >> 6;
+    const int lane = threadIdx.x & 63;
+    if (t >= n_tiles) return;
+    const int32_t mine = lane < kTileRows ? rows[t * kTileRows + lane] : -1;
+    int32_t held = mine;
+    int m = kTileRows;
+    for (int i = 0; i < kTileRows; ++i) {
+        const int32_t a = __shfl(mine, i);
+        const int32_t q0 = a >= 0 ? nptr[a] : 0;
+        const int32_t ne = a >= 0 ? min(nptr[a + 1] - q0, kTileElems) : 0;
+        if (lane == 0) head[t * kTileRows + i] = make_int4(a, q0, ne, 0);
+        int before = 0;
+        for (int k = 0; k < ne; ++k) {
+            const fan_t e = fan[q0 + k];
+            int slot[2] = {before, 0};
+            for (int s = e.x >= 0 ? 0 : 1; s < 2; ++s) {
+                const int32_t node = s == 0 ? e.x : e.y;
+                const unsigned long long hit = __ballot(held == node);
+                slot[s] = hit ? __ffsll(static_cast<long long>(hit)) - 1 : min(m++, kTileCols - 1);
+                if (lane == slot[s]) held = node;
+            }
+            before = slot[1];
+            if (lane == 0)
+                ents[(t * kTileRows + i) * kTileElems + k] = make_int2(
+                    e.z, slot[0] | slot[1] << 8 | (e.w & 31) << 16 | ((e.w >> 10) & 31) << 21 |
+                             ((e.w >> 20) & 31) << 26);
+        }
+        if (lane >= ne && lane < kTileElems) ents[(t * kTileRows + i) * kTileElems + lane] = make_int2(0, 0);
+    }
+    if (lane >= kTileRows && lane < kTileCols) cols[t * (kTileCols - kTileRows) + lane - kTileRows] = held;
+}
+
+}  // namespace
+}  // namespace cvfes
+
+using namespace cvfes;
+
+extern "C" int64_t cvfes_tile_rows(int64_t n_nodes, const double *nodes, const int32_t *indptr,
+                                   const int32_t *indices, int32_t *rows, int64_t cap) {
+    CVFES_REQUIRE(n_nodes >= 0 && n_nodes < (int64_t(1) << 31), "cvfes_tile_rows: bad sizes");
+    if (n_nodes == 0) return 0;
+    CVFES_REQUIRE(nodes && indptr && indices && rows, "cvfes_tile_rows: null pointer");
+    int64_t n = -1;
+    try {
+        n = bisect(nodes, indptr, indices, n_nodes, rows, cap);
+    } catch (...) {
+        return fail(CVFES_ERR_ARG, "cvfes_tile_rows: out of host memory");
+    }
+    CVFES_REQUIRE(n >= 0, "cvfes_tile_rows: more than %lld tiles", static_cast<long long>(cap));
+    return n;
+}
+
+extern "C" int cvfes_tile_lists(void *stream, int64_t n_tiles, const int32_t *rows, const int32_t *nptr,
+                                const int32_t *fan, int64_t max_node_elems, int32_t *head, int32_t *cols,
+                                int32_t *ents) {
+    CVFES_REQUIRE(n_tiles >= 0 && n_tiles < (int64_t(1) << 30), "cvfes_tile_lists: bad sizes");
+    if (n_tiles == 0) return CVFES_OK;
+    CVFES_REQUIRE(max_node_elems >= 1 && max_node_elems <= kTileElems,
+                  "cvfes_tile_lists: max_node_elems must be 1..%d", kTileElems);
+    CVFES_REQUIRE(rows && nptr && fan && head && cols && ents, "cvfes_tile_lists: null pointer");
+    const int64_t blocks = (n_tiles + kBlock / 64 - 1) / (kBlock / 64);
+    hipLaunchKernelGGL(k_tile_lists, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0,
+                       static_cast<hipStream_t>(stream), n_tiles, rows, nptr,
+                       reinterpret_cast<const fan_t *>(fan), reinterpret_cast<int4 *>(head), cols,
+                       reinterpret_cast<int2 *>(ents));
+    return check_launch("k_tile_lists");
+}

@@ -313,7 +313,7 @@ extern "C" int cvfes_step_updated(void *stream, const cvfes_system_t *sys, const
         const double *geom = upd->has_geometry ? (upd->interval == 1 ? cur : upd->ug) : nullptr;
         StepArgs a;
         a.k = RowArgs{sys->n_nodes, S, sys->indptr, sys->indices, sys->values, sys->cptr, sys->celem,
-                      sys->khat, sys->coef, sys->uvalues, sys->vblk};
+                      sys->khat, sys->coef, sys->uvalues, sys->vblk, sys->nptr, nullptr};
         a.u = cur;
         a.up = prev;
         a.out = nxt;

@@ -152,6 +152,17 @@ class MembraneSystem:
         S = self.n_smp
         with torch.cuda.device(dev):
             st = _lib.stream_handle(dev)
+            # --- the elements around each node, for the matrix-free row kernels ------------------
+            self.fan = None
+            if 1 <= self.max_node_elems <= _lib.FAN_MAX_ELEMS:
+                self.fan = torch.empty((3 * self.n_elms, 4), dtype=i32, device=dev)
+                check(self.lib.cvfes_node_fans(st, self.n_nodes, self.max_node_elems, ptr(self.nptr),
+                                               ptr(self.nent), ptr(self.elems), ptr(self.cpos),
+                                               ptr(self.fan)))
+            self.tile_head = self.tile_cols = self.tile_ents = None
+            self.n_tiles = 0
+            if self.fan is not None and self.max_node_elems <= _lib.TILE_ELEMS:
+                self._build_tiles(st)
             # --- element blocks ------------------------------------------------------------------
             self.khat = torch.empty((9 * self.n_elms, 9), dtype=f64, device=dev)
             self.area = torch.empty(self.n_elms, dtype=f64, device=dev)
@@ -207,6 +218,25 @@ class MembraneSystem:
         self.state = None
         self.update = None
         self.ug = None
+
+    def _build_tiles(self, st):
+        """Node tiles of the matrix-free kernels: the tiles' rows on the host, their lists on the
+        device."""
+        rows = np.empty((self.n_nodes, _lib.TILE_ROWS), np.int32)
+        ip, ix = self.indptr_h.astype(np.int32), self.indices_h.astype(np.int32)
+        xyz = np.ascontiguousarray(self._nodes_h)
+        n = int(self.lib.cvfes_tile_rows(self.n_nodes, xyz.ctypes.data, ip.ctypes.data, ix.ctypes.data,
+                                         rows.ctypes.data, self.n_nodes))
+        check(min(n, 0))
+        rows_d = _dev(rows[:n], torch.int32, self.device)
+        i32 = dict(dtype=torch.int32, device=self.device)
+        self.tile_head = torch.empty((n, _lib.TILE_ROWS, 4), **i32)
+        self.tile_cols = torch.empty((n, _lib.TILE_COLS - _lib.TILE_ROWS), **i32)
+        self.tile_ents = torch.empty((n, _lib.TILE_ROWS, _lib.TILE_ELEMS, 2), **i32)
+        check(self.lib.cvfes_tile_lists(st, n, ptr(rows_d), ptr(self.nptr), ptr(self.fan),
+                                        self.max_node_elems, ptr(self.tile_head), ptr(self.tile_cols),
+                                        ptr(self.tile_ents)))
+        self.n_tiles = n
 
     # ------------------------------------------------------------------------------------------
     def set_log_modulus(self, theta):
@@ -351,7 +381,9 @@ class MembraneSystem:
             color_elems=ptr(self.color_elems), elems=ptr(self.elems), cpos=ptr(self.cpos),
             n_colors=self.n_colors, max_color_elems=self.max_color_elems,
             waves_per_simd=self.waves_per_simd, row_records=ptr(self.row_records),
-            record_width=self.record_width, minv=ptr(self.minv))
+            record_width=self.record_width, minv=ptr(self.minv), fan=ptr(self.fan),
+            tile_head=ptr(self.tile_head), tile_cols=ptr(self.tile_cols),
+            tile_ents=ptr(self.tile_ents), n_tiles=self.n_tiles)
 
     def set_variant(self, variant):
         """Select the step kernel variant (names in ``_lib.VARIANTS``); the symmetric ones form the

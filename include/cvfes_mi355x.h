@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define CVFES_ABI_VERSION 12
+#define CVFES_ABI_VERSION 13
 
 #define CVFES_OK 0
 #define CVFES_ERR_ARG (-1)   /* invalid argument (null pointer, bad size)        */
@@ -106,6 +106,17 @@ typedef struct cvfes_system {
      * and gradient kernels scale by them (dt^2 * minv, nu_scale * minv) instead of dividing by lm
      * per column and sample; with NULL they divide.  The forward step kernels do not read it. */
     const double *minv;
+    /* Fan entries of the matrix-free row kernels (may be NULL: they then walk block by block):
+     * fan[3E][4], the entries nptr[a] .. nptr[a+1] of node a being its incident elements, ordered
+     * around the node, as cvfes_node_fans writes them. */
+    const int32_t *fan;
+    /* Node tiles of the matrix-free kernels (n_tiles = 0: none, they walk row by row), as
+     * cvfes_tile_rows and cvfes_tile_lists make them; they need fan and max_node_elems <=
+     * CVFES_TILE_ELEMS.  The results do not depend on them. */
+    const int32_t *tile_head;   /* [n_tiles][CVFES_TILE_ROWS][4]                                */
+    const int32_t *tile_cols;   /* [n_tiles][CVFES_TILE_COLS - CVFES_TILE_ROWS]                 */
+    const int32_t *tile_ents;   /* [n_tiles][CVFES_TILE_ROWS][CVFES_TILE_ELEMS][2]              */
+    int64_t n_tiles;
 } cvfes_system_t;
 
 /* Step kernel variants (cvfes_system_t.variant). */
@@ -170,6 +181,43 @@ int cvfes_stream_read(void *stream, const double *src, int64_t n_doubles, int no
                       double *partial);
 int cvfes_stream_copy(void *stream, const double *src, int64_t n_doubles, int nontemporal,
                       double *dst);
+
+/* Most elements around one node that cvfes_node_fans takes (10-bit block positions). */
+#define CVFES_FAN_MAX_ELEMS 341
+
+/*
+ * Fan entries of the matrix-free row kernels (cvfes_system_t.fan): for every node a its incident
+ * elements, ordered so that neighbouring entries share a node where the mesh allows it.  An entry
+ * is (p, q, e, pk): element e, its other nodes p and q (p = -1 where it is the previous entry's
+ * q), and the positions of e's blocks (a,a), (a,p), (a,q) among the row's contributions, 10 bits
+ * each from the lowest.  Needs max_node_elems <= CVFES_FAN_MAX_ELEMS.  fan is [3E][4], 16-byte
+ * aligned.  No counterpart in the reference.
+ */
+int cvfes_node_fans(void *stream, int64_t n_nodes, int64_t max_node_elems, const int32_t *nptr,
+                    const int32_t *nent, const int32_t *elems, const int32_t *cpos, int32_t *fan);
+
+/* Rows and column slots of a node tile, and most elements around a node of a tiled mesh. */
+#define CVFES_TILE_ROWS 16
+#define CVFES_TILE_COLS 39
+#define CVFES_TILE_ELEMS 8
+
+/*
+ * Node tiles: compact groups of at most CVFES_TILE_ROWS nodes whose block rows have at most
+ * CVFES_TILE_COLS distinct columns together, by recursive bisection of the node cloud.  Host only
+ * (host arrays): nodes [N][3], the block structure indptr/indices; rows [cap][CVFES_TILE_ROWS]
+ * receives the node ids of each tile, -1 padded.  Returns the number of tiles (at most N), or a
+ * negative code.  No counterpart in the reference.
+ */
+int64_t cvfes_tile_rows(int64_t n_nodes, const double *nodes, const int32_t *indptr,
+                        const int32_t *indices, int32_t *rows, int64_t cap);
+
+/*
+ * The lists of the tile kernels (cvfes_system_t.tile_head, tile_cols, tile_ents; device arrays,
+ * 16-byte aligned) from the tiles' rows and the fan entries.  No counterpart in the reference.
+ */
+int cvfes_tile_lists(void *stream, int64_t n_tiles, const int32_t *rows, const int32_t *nptr,
+                     const int32_t *fan, int64_t max_node_elems, int32_t *head, int32_t *cols,
+                     int32_t *ents);
 
 /*
  * Unit-coefficient element stiffness blocks, areas and normals.
@@ -406,6 +454,8 @@ typedef struct cvfes_batch_mesh {
     int64_t n_mtasks;      /* set by cvfes_batch_plan: wave tasks of the mesh                   */
     int64_t slice;         /* set by cvfes_batch_plan: tasks per XCD slice, ceil(n_mtasks / 8)  */
     int64_t xtask0;        /* set by cvfes_batch_plan: first item of the mesh in every XCD's list */
+    int64_t tiled;         /* 1 = cvfes_batch_step_tiles advances the mesh: cvfes_batch_plan then
+                              gives it no wave tasks                                          */
 } cvfes_batch_mesh_t;
 
 /* Device bytes cvfes_batch_plan writes for n_mesh meshes: the descriptors followed by a compact
@@ -423,7 +473,8 @@ int64_t cvfes_batch_plan_bytes(int n_mesh);
  * their L2).  n_tasks receives 8 x the slice items of all meshes (the size of the task space; one
  * wavefront per task is n_waves = n_tasks).  kinds receives the paths the ensemble needs (bit 0:
  * wave-uniform rows with two samples per lane, bit 1: one sample per lane, bit 2: a stored mesh,
- * bit 3: beta or damp, bit 4: packed rows with two samples per lane); pass it to cvfes_batch_step
+ * bit 3: beta or damp, bit 4: packed rows with two samples per lane, bit 10: a matrix-free mesh
+ * without fan entries); pass it to cvfes_batch_step
  * and cvfes_batch_graph_create, which then launch a kernel instance with only those paths (fewer
  * registers, more waves in flight; n_waves >= n_tasks selects the instance without the persistent
  * loop).  Blocks until the copy is done. */
@@ -441,6 +492,24 @@ int cvfes_batch_plan(void *stream, cvfes_batch_mesh_t *meshes, int n_mesh, void 
 int cvfes_batch_step(void *stream, const void *dev_meshes, int n_mesh, int64_t n_tasks, int phase,
                      const int64_t *counter, int64_t k_local, int64_t n_waves, int64_t kinds);
 
+/*
+ * Matrix-free meshes with node tiles (cvfes_system_t.n_tiles) advance in a launch of their own, a
+ * workgroup per tile and chunk of samples.  cvfes_batch_can_tile says whether a mesh qualifies
+ * (then set its `tiled` before cvfes_batch_plan).  cvfes_batch_plan_tiles numbers the workgroups of
+ * the tiled meshes, each mesh cut into 8 contiguous slices, one per XCD, and writes their table to
+ * dev_tiles (device, cvfes_batch_tile_bytes(n_mesh) bytes); n_blocks and shape are passed on to
+ * cvfes_batch_step_tiles.  Blocks until the copy is done.  cvfes_batch_step_tiles is one step of
+ * the tiled meshes (phase, counter and k_local as cvfes_batch_step); dev_meshes is the array
+ * cvfes_batch_plan copied.
+ */
+int cvfes_batch_can_tile(const cvfes_batch_mesh_t *mesh);
+int64_t cvfes_batch_tile_bytes(int n_mesh);
+int cvfes_batch_plan_tiles(void *stream, const cvfes_batch_mesh_t *meshes, int n_mesh, void *dev_tiles,
+                           int64_t *n_blocks, int64_t *shape);
+int cvfes_batch_step_tiles(void *stream, const void *dev_meshes, const void *dev_tiles, int n_mesh,
+                           int64_t n_blocks, int64_t shape, int phase, const int64_t *counter,
+                           int64_t k_local);
+
 /* counter[0] += by on the stream (a kernel, so that it can sit inside a captured graph). */
 int cvfes_counter_add(void *stream, int64_t *counter, int64_t by);
 
@@ -449,6 +518,12 @@ int cvfes_counter_add(void *stream, int64_t *counter, int64_t by);
 int cvfes_batch_graph_create(const void *dev_meshes, int n_mesh, int64_t n_tasks, int64_t *counter,
                              int64_t block_steps, int phase0, int64_t n_waves, int64_t kinds,
                              void **graph);
+/* The same for an ensemble with tiled meshes: every step launches the meshes with wave tasks (when
+ * n_tasks > 0), then the tiled ones. */
+int cvfes_batch_graph_create_tiles(const void *dev_meshes, int n_mesh, int64_t n_tasks,
+                                   int64_t *counter, int64_t block_steps, int phase0,
+                                   int64_t n_waves, int64_t kinds, const void *dev_tiles,
+                                   int64_t n_blocks, int64_t shape, void **graph);
 int cvfes_graph_launch(void *graph, void *stream);
 int cvfes_graph_destroy(void *graph);
 

@@ -1,0 +1,184 @@
+"""Matrix-free kernels by node tiles (GPU) and the tiles themselves (CPU).
+
+* every node sits in exactly one tile and a tile's columns fit its slots, for tubes, an irregular
+  wall, isolated nodes and coordinates that are not numbers (CPU);
+* the tile kernels (step, adjoint step) give the bits of the row kernels at sample counts around
+  the lane and chunk edges, per-node and per-sample masses, with and without damping, on meshes
+  with 6 and with 8 elements around a node, boundary fans and an isolated node; the row kernels
+  they are compared with follow the oracle (1e-10 relative max-norm, the bar of every step);
+* meshes with more elements around a node than a tile or a fan takes run the row kernels, within
+  the same bar, and walking block by block without fan entries agrees with the fans to rounding.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+from cvfes_amd import _lib
+from cvfes_amd.mesh import tube_geometry
+from cvfes_amd.sparse import block_structure
+from oracle import solid_oracle as so
+
+
+def wall(kind, seed=0):
+    """Nodes, triangles and fixed nodes of a test wall."""
+    rng = np.random.default_rng(seed)
+    if kind == "tube":
+        return tube_geometry(20, 9, 0.3, 2.0)
+    if kind == "isolated":                       # and a node in no element
+        nodes, el, bdy = tube_geometry(20, 9, 0.3, 2.0)
+        return np.vstack([nodes, [[4.0, 4.0, 4.0]]]), el, bdy
+    if kind.startswith("fan"):                   # a flat fan of n triangles about node 0, a grid beside it
+        n = int(kind[3:])
+        t = 2.0 * np.pi * np.arange(n) / n
+        nodes = np.vstack([[[0.0, 0.0, 0.1]], np.stack([np.cos(t), np.sin(t), 0.0 * t], 1)])
+        el = np.array([[0, 1 + i, 1 + (i + 1) % n] for i in range(n)])
+        el = el[rng.permutation(n)]
+        el = np.array([np.roll(e, rng.integers(3)) for e in el])
+        bdy = np.array([1])
+    else:                                        # "grid": a bumpy rectangle, diagonals at random
+        n = 13
+        x, y = np.meshgrid(np.arange(n), np.arange(n), indexing="ij")
+        nodes = np.stack([x, y, 0.3 * np.sin(x) * np.cos(0.7 * y)], -1).reshape(-1, 3) * 0.05
+        el = []
+        for i in range(n - 1):
+            for j in range(n - 1):
+                a, b, c, d = i * n + j, (i + 1) * n + j, (i + 1) * n + j + 1, i * n + j + 1
+                el += [[a, b, c], [a, c, d]] if (i + j) % 2 else [[a, b, d], [b, c, d]]
+        el = np.array(el)[rng.permutation(len(el))]
+        bdy = np.arange(n)
+    return nodes, el.astype(np.int64), bdy.astype(np.int64)
+
+
+def tile_rows(nodes, el):
+    ip, ix = block_structure(el, nodes.shape[0])
+    ip, ix = ip.astype(np.int32), ix.astype(np.int32)
+    xyz = np.ascontiguousarray(nodes, np.float64)
+    rows = np.full((nodes.shape[0], _lib.TILE_ROWS), -7, np.int32)
+    n = _lib.lib().cvfes_tile_rows(nodes.shape[0], xyz.ctypes.data, ip.ctypes.data, ix.ctypes.data,
+                                   rows.ctypes.data, nodes.shape[0])
+    assert n > 0
+    return rows[:n], ip, ix
+
+
+@pytest.mark.parametrize("kind", ["tube", "isolated", "grid", "fan8", "nan", "point"])
+def test_tiles_hold_every_node_once(kind):
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libcvfes_mi355x.so not built")
+    nodes, el, _ = wall("tube" if kind in ("nan", "point") else kind)
+    if kind == "nan":
+        nodes = nodes.copy()
+        nodes[::3] = np.nan
+    if kind == "point":
+        nodes = np.zeros_like(nodes)
+    rows, ip, ix = tile_rows(nodes, el)
+    assert np.array_equal(np.sort(rows[rows >= 0]), np.arange(nodes.shape[0]))
+    for r in rows:
+        own = r[r >= 0]
+        assert np.all(r[len(own):] == -1)
+        cols = np.unique(np.concatenate([ix[ip[a]:ip[a + 1]] for a in own] + [own]))
+        assert len(cols) - len(own) <= _lib.TILE_COLS - _lib.TILE_ROWS
+
+
+def build(kind, S, seed=0, thick_samples=False):
+    from cvfes_amd.system import MembraneSystem
+    nodes, el, bdy = wall(kind, seed)
+    rng = np.random.default_rng(seed)
+    E = 7e6 * np.exp(0.1 * rng.standard_normal((el.shape[0], S)))
+    n = nodes.shape[0]
+    h = 0.07 * rng.uniform(0.9, 1.1, (n, S)) if thick_samples else np.full(n, 0.07)
+    s = MembraneSystem(nodes, el, bdy, S, vthickness=h, elmE=E, density=1.0, nu=0.45, store_values=False)
+    return nodes, el, bdy, s
+
+
+def run(s, u0, dt, beta, damp, nsteps=6):
+    """Steps, then one adjoint step from the states, by the system's current matrix-free path."""
+    import torch
+    p = 1.33e4 * (1.0 + 0.1 * np.sin(np.arange(nsteps)))
+    s._sys = s._make_struct()
+    s.initial_state(u0, 0.0 * u0, s.loads(p), dt, beta=beta, damp=damp, method="matfree")
+    s.step(p, dt, beta=beta, damp=damp, method="matfree")
+    mu = torch.empty_like(s.u)
+    w = torch.linspace(0.5, 1.5, s.n_smp, dtype=torch.float64, device=s.device)
+    _lib.check(s.lib.cvfes_adjoint_step(s.stream, ctypes.byref(s._sys), _lib.METHOD_MATFREE, s.u.data_ptr(),
+                                        s.up.data_ptr(), mu.data_ptr(), s.state[2].data_ptr(), None,
+                                        w.data_ptr(), dt, beta, damp, 1))
+    return s.u.cpu().numpy(), mu.cpu().numpy(), p
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,S,beta,damp,thick", [
+    ("tube", 1, 1e-7, 0.0, False), ("isolated", 2, 0.0, 5.0, True), ("tube", 3, 1e-7, 5.0, False),
+    ("grid", 5, 0.0, 0.0, False), ("fan8", 7, 1e-7, 5.0, True), ("tube", 8, 0.0, 0.0, False), ("tube", 9, 1e-7, 0.0, False), ("tube", 31, 0.0, 5.0, True),
+    ("tube", 33, 1e-7, 5.0, False), ("tube", 64, 1e-7, 0.0, False), ("tube", 66, 0.0, 0.0, False),
+    ("isolated", 128, 1e-7, 5.0, False), ("isolated", 130, 0.0, 0.0, True), ("tube", 200, 1e-7, 5.0, True),
+    ("grid", 16, 1e-7, 5.0, True), ("grid", 97, 0.0, 0.0, False), ("fan7", 24, 1e-7, 5.0, False),
+    ("fan8", 34, 0.0, 5.0, True)])
+def test_tile_kernels_equal_row_kernels(require_gpu, kind, S, beta, damp, thick):
+    nodes, el, bdy, s = build(kind, S, seed=S, thick_samples=thick)
+    assert s.n_tiles > 0
+    dt = 1e-6
+    u0 = 1e-4 * np.random.default_rng(S).standard_normal(3 * nodes.shape[0])
+    u, mu, p = run(s, u0, dt, beta, damp)
+    tiles, s.n_tiles = s.n_tiles, 0
+    ur, mur, _ = run(s, u0, dt, beta, damp)
+    s.n_tiles = tiles
+    assert np.all(np.isfinite(u)) and np.max(np.abs(mu)) > 0
+    assert np.array_equal(u, ur) and np.array_equal(mu, mur)
+    ref = oracle_run(nodes, el, bdy, s, u0, p, dt, beta, damp)
+    assert np.max(np.abs(u.reshape(-1, S) - ref)) < 1e-10 * np.max(np.abs(ref))
+
+
+def oracle_run(nodes, el, bdy, s, u0, p, dt, beta, damp):
+    ip, ix = so.sparse_info_loops(el, nodes.shape[0])
+    h = np.broadcast_to(s.vthick.cpu().numpy().reshape(nodes.shape[0], -1), (nodes.shape[0], s.n_smp))
+    gth = so.gauss_properties(np.ones_like(h), h, el)[1]
+    _, K, f1, LM = so.assemble_reference(nodes, el, 1.0, so.d_matrix(0.45), s.coef.cpu().numpy(), gth, 1.0, ip, ix)
+    bd = (3 * bdy[:, None] + np.arange(3)).ravel()
+    return so.run(ip, ix, K, LM, f1, p, u0, 0.0 * u0, dt, beta=beta, damp=damp, bdy_dofs=bd)[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,S", [("fan9", 16), ("fan40", 5), ("fan9", 3)])
+def test_untiled_meshes_and_block_walk(require_gpu, kind, S):
+    """More elements around a node than a tile takes (9, and 40: beyond the sorted fans)."""
+    nodes, el, bdy, s = build(kind, S, seed=3)
+    dt, beta, damp = 1e-6, 1e-7, 5.0
+    assert s.fan is not None and s.n_tiles == 0
+    u0 = 1e-4 * np.random.default_rng(1).standard_normal(3 * nodes.shape[0])
+    u, mu, p = run(s, u0, dt, beta, damp)
+    ref = oracle_run(nodes, el, bdy, s, u0, p, dt, beta, damp)
+    assert np.max(np.abs(u.reshape(-1, S) - ref)) < 1e-10 * np.max(np.abs(ref))
+    fan, s.fan = s.fan, None
+    ub, mub, _ = run(s, u0, dt, beta, damp)
+    s.fan = fan
+    # the two walks sum the same products in another order: a few ulp per step of the largest value
+    assert np.max(np.abs(u - ub)) < 1e-13 * np.max(np.abs(ub))
+    assert np.max(np.abs(mu - mub)) < 1e-12 * np.max(np.abs(mub))
+
+
+@pytest.mark.gpu
+def test_batched_tiles_and_rows_in_one_ensemble(require_gpu):
+    """Tiled meshes of three shapes beside meshes with wave tasks: eager and replayed steps give the
+    single-mesh bits."""
+    from cvfes_amd.batch import BatchedEnsemble
+    n = 24
+    specs = [("tube", 64, 1e-7, 5.0), ("tube", 5, 0.0, 0.0), ("fan8", 33, 0.0, 5.0), ("grid", 12, 0.0, 0.0),
+             ("fan9", 16, 1e-7, 0.0)]
+    systems = [build(k, S, seed=S)[3] for k, S, _, _ in specs]
+    loads = [s.loads(np.full(n, 1.33e4)) for s in systems]
+    u0s = [1e-4 * np.random.default_rng(i).standard_normal(3 * s.n_nodes) for i, s in enumerate(systems)]
+    outs = []
+    for mode in ("single", "eager", "graph"):
+        ens = BatchedEnsemble(systems, loads, dts=1e-6, methods="matfree", betas=[c[2] for c in specs],
+                              damps=[c[3] for c in specs])
+        ens.initial_state(u0s=u0s)
+        assert [int(m.tiled) for m in ens.host_meshes] == [1, 0, 1, 1, 0]
+        if mode == "single":
+            ens.run_per_mesh(n)
+        else:
+            ens.run(n, graph=mode == "graph", block=6)
+        outs.append([s.u.cpu().numpy() for s in systems])
+    for o in outs[1:]:
+        for a, b in zip(outs[0], o):
+            assert np.all(np.isfinite(a)) and np.array_equal(a, b)
