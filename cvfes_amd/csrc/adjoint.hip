@@ -240,7 +240,7 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_step(AdjArgs a) {
         const int64_t col = a.k.indices[p];
         double x[3][VW];
         adj_column<BETA, VW>(a, col, s, x);
-        block_apply<OP, VW>(a.k, p, col < row, s, x, acc);
+        block_apply<OP, VW>(a.k, p, static_cast<int>(col) - row, s, x, acc);
     }
     adj_finish<DAMP, VW>(a, row, s, active, acc);
 }
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(kBlock) void k_fused_step(StepArgs f, AdjArgs a, in
         double xf[3][VW], xa[3][VW];
         state_column<BETA, VW>(f.u, f.up, f.bdt, col, f.k.n_smp, s, xf);
         adj_column<BETA, VW>(a, col, s, xa);
-        block_apply2<OP, VW>(f.k, p, col < row, s, xf, accf, xa, acca);
+        block_apply2<OP, VW>(f.k, p, static_cast<int>(col) - row, s, xf, accf, xa, acca);
     }
     step_update<DAMP, VW>(f, row, s, active, step, accf);
     adj_finish<DAMP, VW>(a, row, s, active, acca);

@@ -254,7 +254,7 @@ __global__ __launch_bounds__(kBlock) void k_step_sym(StepArgs a, const double *_
             const bool valid = b < nb;
             const int32_t pb = p0 + (valid ? b : nb - 1);
             const int32_t col = REC ? r[2 + b] : k.indices[pb];
-            const bool tr = col < row;
+            const int side = col - row;
             V w[3];
             const auto cu = buffer_rsrc(a.u + static_cast<int64_t>(col) * 3 * S, 3 * sb);
             const auto cp = buffer_rsrc(a.up + static_cast<int64_t>(col) * 3 * S, 3 * sb);
@@ -271,13 +271,14 @@ __global__ __launch_bounds__(kBlock) void k_step_sym(StepArgs a, const double *_
             const int64_t ub = REC ? r[2 + MAXB + b] : vblk[pb];
             const auto rv = buffer_rsrc(uvalues + ub * 9 * S, 9 * sb);
             V kv[9];
-            if (NT == 2 && tr) {
+            if (NT == 2 && side < 0) {
 #pragma unroll
-                for (int ij = 0; ij < 9; ++ij) kv[ij] = ldb<VW, kAuxNT>(rv, lo, (3 * (ij % 3) + ij / 3) * sb);
+                for (int ij = 0; ij < 9; ++ij) kv[ij] = ldb<VW, kAuxNT>(rv, lo, sym_entry(ij, -1) * sb);
             } else {
 #pragma unroll
                 for (int ij = 0; ij < 9; ++ij)
-                    kv[ij] = ldb<VW, AUX_FIRST>(rv, lo, (tr ? 3 * (ij % 3) + ij / 3 : ij) * sb);
+                    kv[ij] = ldb<VW, AUX_FIRST>(
+                        rv, lo, (side < 0 ? sym_entry(ij, -1) : (side == 0 ? sym_entry(ij, 0) : ij)) * sb);
             }
 #pragma unroll
             for (int i = 0; i < 3; ++i)

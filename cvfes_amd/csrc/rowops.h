@@ -151,10 +151,19 @@ struct GStepArgs {
     bool nt_out;
 };
 
+// Entry of a stored upper block that gives entry ij of the block a row needs: `side` < 0 the block's
+// column precedes its row (read transposed), 0 it is the row's diagonal block, > 0 neither.  The
+// diagonal block of a symmetric matrix is symmetric itself, so only its upper six entries are read:
+// a quarter of the stored blocks are diagonal ones, which is 8 % of the stream of values.
+__device__ __forceinline__ constexpr int sym_entry(int ij, int side) {
+    const int i = ij / 3, j = ij % 3;
+    return side < 0 || (side == 0 && i > j) ? 3 * j + i : ij;
+}
+
 // Stored block p of the row: kv[ij][v] = K_p[ij] of sample s + v.  SYM: symmetric storage, the
-// block is the upper block vblk[p], transposed when `tr` (its column precedes its row).
+// block is the upper block vblk[p] (`side`: sym_entry).
 template <bool SYM, int VW, class RA>
-__device__ __forceinline__ void stored_block(const RA &k, int32_t p, bool tr, int64_t s,
+__device__ __forceinline__ void stored_block(const RA &k, int32_t p, int side, int64_t s,
                                              double (&kv)[9][VW]) {
     if constexpr (!SYM) {
         const auto *base = k.values + (static_cast<int64_t>(p) * 9) * k.n_smp + s;
@@ -168,7 +177,7 @@ __device__ __forceinline__ void stored_block(const RA &k, int32_t p, bool tr, in
         const auto *base = k.uvalues + (static_cast<int64_t>(k.vblk[p]) * 9) * k.n_smp + s;
 #pragma unroll
         for (int ij = 0; ij < 9; ++ij) {
-            const int src = tr ? 3 * (ij % 3) + ij / 3 : ij;
+            const int src = side < 0 ? sym_entry(ij, -1) : (side == 0 ? sym_entry(ij, 0) : ij);
             const Vec<VW> t = load_vec<VW>(base + src * k.n_smp);
 #pragma unroll
             for (int v = 0; v < VW; ++v) kv[ij][v] = t.v[v];
@@ -180,13 +189,13 @@ __device__ __forceinline__ void stored_block(const RA &k, int32_t p, bool tr, in
 // K_p = sum over the block's element contributions c of coef_e(c) * khat_c, applied as
 // acc += coef_e (khat_c x), so the block itself is never formed and only the three sums per
 // sample are live (khat_c is wave-uniform for wave-uniform rows: scalar loads).
-// `tr`: the block's column precedes its row (symmetric storage reads it transposed).
+// `side`: the block's column less its row, for the symmetric storage (sym_entry).
 template <int OP, int VW, class RA>
-__device__ __forceinline__ void block_apply(const RA &k, int32_t p, bool tr, int64_t s,
+__device__ __forceinline__ void block_apply(const RA &k, int32_t p, int side, int64_t s,
                                             const double (&x)[3][VW], double (&acc)[3][VW]) {
     if constexpr (OP != kOpMatfree) {
         double kv[9][VW];
-        stored_block<OP == kOpSym, VW>(k, p, tr, s, kv);
+        stored_block<OP == kOpSym, VW>(k, p, side, s, kv);
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -234,12 +243,12 @@ __device__ __forceinline__ void state_column(DP u, DP up, double bdt, int64_t co
 // block_apply for two columns at once (the block is loaded once): acc += K_p x and acc2 += K_p x2,
 // each with exactly the operations block_apply performs.
 template <int OP, int VW, class RA>
-__device__ __forceinline__ void block_apply2(const RA &k, int32_t p, bool tr, int64_t s,
+__device__ __forceinline__ void block_apply2(const RA &k, int32_t p, int side, int64_t s,
                                              const double (&x)[3][VW], double (&acc)[3][VW],
                                              const double (&x2)[3][VW], double (&acc2)[3][VW]) {
     if constexpr (OP != kOpMatfree) {
         double kv[9][VW];
-        stored_block<OP == kOpSym, VW>(k, p, tr, s, kv);
+        stored_block<OP == kOpSym, VW>(k, p, side, s, kv);
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -471,7 +480,7 @@ __device__ __forceinline__ void row_product(const RA &k, DP u, DP up, double bdt
         const int64_t col = k.indices[p];
         double x[3][VW];
         state_column<BETA, VW>(u, up, bdt, col, k.n_smp, s, x);
-        block_apply<OP, VW>(k, p, col < row, s, x, acc);
+        block_apply<OP, VW>(k, p, static_cast<int>(col) - row, s, x, acc);
     }
 }
 
