@@ -289,6 +289,23 @@ __global__ __launch_bounds__(kBlock) void k_step_sym(StepArgs a, const double *_
     finish_row<DAMP, VW, NT != 0>(a, row, s, active, step, uo, po, acc);
 }
 
+// The generic step on the symmetric storage with row records, for any sample count (sym_product; the
+// bits are those of k_step<kOpSym>).
+template <bool UNIFORM, bool BETA, bool DAMP, int VW, int MAXB>
+__global__ __launch_bounds__(kBlock) void k_step_symrec(StepArgs a, const int32_t *__restrict__ rec, int64_t step) {
+    int32_t row;
+    int64_t s;
+    bool active;
+    if (!row_and_sample<UNIFORM, VW>(a.k.n_nodes, a.k.n_smp, row, s, active)) return;
+    const int32_t *r = rec + static_cast<int64_t>(row) * (2 + 2 * MAXB);
+    row = r[0];
+    typedef StateCol<UNIFORM, BETA, VW, const double *> Col;
+    const Col col{a.u, a.up, a.bdt, a.k.n_smp, static_cast<uint32_t>(s) * 8u};
+    double acc[1][3][VW];
+    sym_product<UNIFORM, VW, MAXB>(a.k, r, col, row, acc);
+    step_update<DAMP, VW>(a, row, s, active, step, acc[0]);
+}
+
 // Matrix-free step with the row's coefficients loaded once per row (step_row_cached); one
 // wavefront per (row, 64*VW samples), so rows must be wave-uniform.
 template <bool BETA, bool DAMP, int VW, int MAXE>
@@ -573,6 +590,30 @@ void launch_sym(hipStream_t st, const cvfes_system_t *sys, const StepArgs &a, in
         launch_sym_rec<NT, MAXB, false>(st, sys, a, step, beta, damp);
 }
 
+template <bool UNI, int VW, int MAXB>
+void launch_symrec(hipStream_t st, const StepArgs &a, const int32_t *rec, int64_t step, bool beta, bool damp) {
+    const dim3 g(grid_for(a.k.n_nodes * lanes_per_row<UNI, VW>(a.k.n_smp))), b(kBlock);
+    if (beta) {
+        if (damp) hipLaunchKernelGGL((k_step_symrec<UNI, true, true, VW, MAXB>), g, b, a.occ_lds, st, a, rec, step);
+        else hipLaunchKernelGGL((k_step_symrec<UNI, true, false, VW, MAXB>), g, b, a.occ_lds, st, a, rec, step);
+    } else {
+        if (damp) hipLaunchKernelGGL((k_step_symrec<UNI, false, true, VW, MAXB>), g, b, a.occ_lds, st, a, rec, step);
+        else hipLaunchKernelGGL((k_step_symrec<UNI, false, false, VW, MAXB>), g, b, a.occ_lds, st, a, rec, step);
+    }
+}
+
+template <int MAXB>
+void step_symrec(hipStream_t st, const StepArgs &a, const int32_t *rec, int64_t step, bool beta, bool damp) {
+    const int64_t S = a.k.n_smp;
+    if (generic_vw(S) == 2) {
+        if (use_uniform<2>(S)) launch_symrec<true, 2, MAXB>(st, a, rec, step, beta, damp);
+        else launch_symrec<false, 2, MAXB>(st, a, rec, step, beta, damp);
+    } else {
+        if (use_uniform<1>(S)) launch_symrec<true, 1, MAXB>(st, a, rec, step, beta, damp);
+        else launch_symrec<false, 1, MAXB>(st, a, rec, step, beta, damp);
+    }
+}
+
 template <int VW, int MAXE>
 void launch_cached(hipStream_t st, const StepArgs &a, const LdsArgs &l, int64_t step, bool beta,
                    bool damp) {
@@ -852,7 +893,13 @@ void step_dispatch(hipStream_t st, const cvfes_system_t *sys, bool mf, const Ste
     case kOpFan: step_generic<kOpFan>(st, a, step, beta, damp); break;
     case kOpMatfree: step_generic<kOpMatfree>(st, a, step, beta, damp); break;
     case kOpStored: step_generic<kOpStored>(st, a, step, beta, damp); break;
-    default: step_generic<kOpSym>(st, a, step, beta, damp); break;
+    default:
+        switch (record_slots(sys)) {
+        case 7: step_symrec<7>(st, a, sys->row_records, step, beta, damp); break;
+        case 10: step_symrec<10>(st, a, sys->row_records, step, beta, damp); break;
+        default: step_generic<kOpSym>(st, a, step, beta, damp); break;
+        }
+        break;
     }
 }
 

@@ -85,6 +85,15 @@ inline const fan_t *fan_entries(const cvfes_system_t *sys) {
     return sys->nptr && sys->n_smp < (int64_t(1) << 28) ? reinterpret_cast<const fan_t *>(sys->fan) : nullptr;
 }
 
+// Block slots of the system's row records if the kernels that read the symmetric storage by them
+// apply, else 0 (byte offsets inside a block are 32-bit: 72 S).
+inline int record_slots(const cvfes_system_t *sys) {
+    if (!sys->row_records || !sys->uvalues || 72 * sys->n_smp > INT32_MAX) return 0;
+    for (int maxb : {7, 10})
+        if (sys->record_width == 2 + 2 * maxb && sys->max_row_blocks >= 1 && sys->max_row_blocks <= maxb) return maxb;
+    return 0;
+}
+
 // Node tiles (tile.h): rows per tile, column slots (39 of 64 samples and the unit blocks of 16
 // rows of 6 elements fit half a CU's LDS), and most elements around a node.
 constexpr int kTileRows = CVFES_TILE_ROWS;
@@ -464,6 +473,67 @@ __device__ __forceinline__ void fan_product(const RA &k, const COL &col, int32_t
                     for (int v = 0; v < VW; ++v) xp[m][j][v] = xq[m][j][v];
         }
         e = n;
+    }
+}
+
+// acc[c] = the row's product with each column c from the symmetric storage, the row's structure
+// coming from its record `r` (cvfes_system_t.row_records): the operations of block_apply, block by
+// block in the same order, with the next block's loads issued before the current one is applied.  The walk over
+// indptr, indices and vblk puts two dependent loads in front of every block's values.  Slots behind
+// the row's last block repeat it and are not added.
+template <bool UNI, int VW, int MAXB, class COL>
+__device__ __forceinline__ void sym_product(const RowArgs &k, const int32_t *r, const COL &col, int32_t row,
+                                            double (&acc)[COL::kCols][3][VW]) {
+    constexpr int NC = COL::kCols;
+    const int32_t nb = r[1];
+    const int64_t S = k.n_smp;
+    const uint32_t sb = static_cast<uint32_t>(S) * 8u;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int v = 0; v < VW; ++v) acc[c][i][v] = 0.0;
+    // blocks in flight, this one included: as many as leave two waves per SIMD (one sample per lane:
+    // 166 registers; all of a row's blocks at once, which is what the compiler makes of the plain
+    // loop, run at one wave per SIMD)
+    constexpr int D = VW == 1 ? (NC == 1 ? 6 : 4) : (NC == 1 ? 3 : 2);
+    typename COL::Raw x[D];
+    Vec<VW> kv[D][9];
+    auto issue = [&](int b) {
+        const int32_t node = r[2 + b];
+        const int side = node - row;
+        const double *base = k.uvalues + static_cast<int64_t>(r[2 + MAXB + b]) * 9 * S;
+        x[b % D] = col.load(node);
+#pragma unroll
+        for (int ij = 0; ij < 9; ++ij) {
+            const uint32_t src = side < 0 ? sym_entry(ij, -1) : (side == 0 ? sym_entry(ij, 0) : ij);
+            if constexpr (UNI) kv[b % D][ij] = to_vec<VW>(ldb<VW, 0>(buffer_rsrc(base, 9 * sb), col.lane, src * sb));
+            else kv[b % D][ij] = load_lane<VW>(base, src * sb + col.lane);
+        }
+    };
+#pragma unroll
+    for (int b = 0; b < D - 1; ++b) issue(b);
+#pragma unroll
+    for (int b = 0; b < MAXB; ++b) {
+        if (b + D - 1 < MAXB) issue(b + D - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        double xv[NC][3][VW];
+        col.value(x[b % D], xv);
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int v = 0; v < VW; ++v) {
+                    double t = acc[c][i][v];
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) t = fma(kv[b % D][3 * i + j].v[v], xv[c][j][v], t);
+                    acc[c][i][v] = b < nb ? t : acc[c][i][v];
+                    // the sums stay here: they would be moved behind the loads of all blocks
+                    asm volatile("" : "+v"(acc[c][i][v]));
+                }
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 

@@ -161,8 +161,8 @@ class MembraneSystem:
                                                ptr(self.fan)))
             self.tile_head = self.tile_cols = self.tile_ents = None
             self.n_tiles = 0
-            if self.fan is not None and self.max_node_elems <= _lib.TILE_ELEMS:
-                self._build_tiles(st)
+            if not store_values:
+                self._ensure_tiles()
             # --- element blocks ------------------------------------------------------------------
             self.khat = torch.empty((9 * self.n_elms, 9), dtype=f64, device=dev)
             self.area = torch.empty(self.n_elms, dtype=f64, device=dev)
@@ -219,9 +219,11 @@ class MembraneSystem:
         self.update = None
         self.ug = None
 
-    def _build_tiles(self, st):
-        """Node tiles of the matrix-free kernels: the tiles' rows on the host, their lists on the
-        device."""
+    def _ensure_tiles(self):
+        """Node tiles of the matrix-free kernels, on first use: the tiles' rows on the host, their
+        lists on the device."""
+        if self.tile_head is not None or self.fan is None or self.max_node_elems > _lib.TILE_ELEMS:
+            return
         rows = np.empty((self.n_nodes, _lib.TILE_ROWS), np.int32)
         ip, ix = self.indptr_h.astype(np.int32), self.indices_h.astype(np.int32)
         xyz = np.ascontiguousarray(self._nodes_h)
@@ -233,10 +235,12 @@ class MembraneSystem:
         self.tile_head = torch.empty((n, _lib.TILE_ROWS, 4), **i32)
         self.tile_cols = torch.empty((n, _lib.TILE_COLS - _lib.TILE_ROWS), **i32)
         self.tile_ents = torch.empty((n, _lib.TILE_ROWS, _lib.TILE_ELEMS, 2), **i32)
-        check(self.lib.cvfes_tile_lists(st, n, ptr(rows_d), ptr(self.nptr), ptr(self.fan),
+        check(self.lib.cvfes_tile_lists(self.stream, n, ptr(rows_d), ptr(self.nptr), ptr(self.fan),
                                         self.max_node_elems, ptr(self.tile_head), ptr(self.tile_cols),
                                         ptr(self.tile_ents)))
         self.n_tiles = n
+        if hasattr(self, "_sys"):
+            self._sys = self._make_struct()
 
     # ------------------------------------------------------------------------------------------
     def set_log_modulus(self, theta):
@@ -584,6 +588,8 @@ class MembraneSystem:
         load at the start time.
         """
         f64 = torch.float64
+        if self.method_id(method) == _lib.METHOD_MATFREE:
+            self._ensure_tiles()
         if not isinstance(load, LoadTables):
             load = self.loads(load)
         shp = self.state_shape()
