@@ -27,6 +27,7 @@ struct GeomArgs {
     const int32_t *nptr;     // [N+1]
     const int32_t *nent;     // [3E]
     double nu, g, gk, inv_1mnu2;
+    const fan_t *fan;        // [3E] (rowops.h); null: the elements are walked by nent
 };
 
 __device__ __forceinline__ void moved_points(const GeomArgs &g, const int32_t (&ids)[3], int64_t S,
@@ -152,6 +153,167 @@ __global__ __launch_bounds__(kBlock) void k_step_updated(StepArgs a, GeomArgs g,
     }
 }
 
+__device__ __forceinline__ double dot(const double (&x)[3], const double (&y)[3]) {
+    return fma(x[2], y[2], fma(x[1], y[1], x[0] * y[0]));
+}
+
+__device__ __forceinline__ void cross(const double (&x)[3], const double (&y)[3], double (&z)[3]) {
+    z[0] = fma(x[1], y[2], -(x[2] * y[1]));
+    z[1] = fma(x[2], y[0], -(x[0] * y[2]));
+    z[2] = fma(x[0], y[1], -(x[1] * y[0]));
+}
+
+// The same product by the fan entries and without element frames.  With the row's node a as origin,
+// e_p and e_q the moved edges to an element's other nodes, n = e_p x e_q (twice the area vector) and
+// G_p = e_q x n, G_q = n x e_p, G_a = -(G_p + G_q) the gradients of the shape functions times n.n,
+// the in-plane isotropic law and the transverse shear, both independent of the direction of the
+// in-plane axes, give the force of the relative displacements y_p, y_q on a as
+//   f_a = coef / (1 - nu^2) / (2 |n|) [ g w + ((gk - g) (n.w) n + nu tau G_a + g (G_p (y_p.G_a) +
+//         G_q (y_q.G_a))) / n.n ],
+//   w = (e_p.d) y_q - (e_q.d) y_p,  d = e_q - e_p,  tau = y_p.G_p + y_q.G_q,
+// and the unit-pressure load as n / 6.  That is one reciprocal square root and about 100 FP64
+// instructions per element and sample; the frames (two square roots, three divisions, the local
+// coordinates and the nine 3 x 3 blocks' rows) took about 250, and FP64 issue bounds this kernel.
+// Neighbours chain around the node, so each is read once, its loads in flight while the element
+// before is applied.  65,920 nodes x 200 samples, every step re-formed: 939 -> 560 us a step.
+template <bool UNIFORM, bool BETA, bool DAMP, bool GEO_U, int VW>
+__global__ __launch_bounds__(kBlock) void k_step_moved(StepArgs a, GeomArgs g, int64_t step) {
+    int32_t row;
+    int64_t s;
+    bool active;
+    if (!row_and_sample<UNIFORM, VW>(a.k.n_nodes, a.k.n_smp, row, s, active)) return;
+    const int64_t S = a.k.n_smp;
+    const uint32_t lane = static_cast<uint32_t>(s) * 8u;
+    // y = x relative to the row's node is all the product needs of the displacement, and with
+    // GEO_U and no beta the moved edge is the reference edge plus y
+    constexpr bool ONE = GEO_U && !BETA;
+    struct Raw {
+        Vec<VW> u[3], up[3], ug[3];
+        double ref[3];
+    };
+    struct Rel {
+        double e[3][VW], y[3][VW], ee[VW];
+    };
+    auto load = [&](int32_t node) {
+        Raw r;
+        load_node<UNIFORM, VW>(a.u, node, S, lane, r.u);
+        if constexpr (BETA) load_node<UNIFORM, VW>(a.up, node, S, lane, r.up);
+        if constexpr (!GEO_U) {
+            if (g.ug) load_node<UNIFORM, VW>(g.ug, node, S, lane, r.ug);
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) r.ref[k] = g.nodes[3 * static_cast<int64_t>(node) + k];
+        return r;
+    };
+    auto disp = [&](const Raw &r, int k, int v) {
+        return BETA ? fma(a.bdt, r.u[k].v[v] - r.up[k].v[v], r.u[k].v[v]) : r.u[k].v[v];
+    };
+    auto move = [&](const Raw &r, int k, int v) {
+        if constexpr (GEO_U) return r.u[k].v[v];
+        else return g.ug ? r.ug[k].v[v] : 0.0;
+    };
+    const Raw own = load(row);
+    auto relative = [&](const Raw &r, Rel &o) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int v = 0; v < VW; ++v) {
+                o.y[k][v] = disp(r, k, v) - disp(own, k, v);
+                o.e[k][v] = (r.ref[k] - own.ref[k]) + (ONE ? o.y[k][v] : move(r, k, v) - move(own, k, v));
+            }
+#pragma unroll
+        for (int v = 0; v < VW; ++v)
+            o.ee[v] = fma(o.e[2][v], o.e[2][v], fma(o.e[1][v], o.e[1][v], o.e[0][v] * o.e[0][v]));
+    };
+    double acc[3][VW] = {};
+    double fl[3][VW] = {};        // six times the unit-traction load of the row's node
+    const double cg = g.g, cs = g.gk - g.g, half = 0.5 * g.inv_1mnu2;
+    auto apply = [&](const Rel &p, const Rel &q, const Vec<VW> &cf) {
+#pragma unroll
+        for (int v = 0; v < VW; ++v) {
+            const double ep[3] = {p.e[0][v], p.e[1][v], p.e[2][v]}, eq[3] = {q.e[0][v], q.e[1][v], q.e[2][v]};
+            const double yp[3] = {p.y[0][v], p.y[1][v], p.y[2][v]}, yq[3] = {q.y[0][v], q.y[1][v], q.y[2][v]};
+            double n[3], Gp[3], Gq[3];
+            cross(ep, eq, n);
+            const double r = rsqrt(dot(n, n));
+            cross(eq, n, Gp);
+            cross(n, ep, Gq);
+            const double pq = dot(ep, eq), cp = q.ee[v] - pq, cq = pq - p.ee[v];
+            double w[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) w[k] = fma(cq, yq[k], -(cp * yp[k]));
+            // nu tau G_a + g (G_p (y_p.G_a) + G_q (y_q.G_a)) = fp G_p + fq G_q
+            const double ypp = dot(yp, Gp), yqq = dot(yq, Gq), t = g.nu * (ypp + yqq);
+            const double fp = -fma(cg, ypp + dot(yp, Gq), t), fq = -fma(cg, yqq + dot(yq, Gp), t);
+            const double nw = cs * dot(n, w), sc = half * cf.v[v] * r, s1 = sc * cg, s2 = sc * (r * r);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const double in = fma(nw, n[k], fma(fp, Gp[k], fq * Gq[k]));
+                acc[k][v] = fma(s2, in, fma(s1, w[k], acc[k][v]));
+                fl[k][v] += n[k];
+            }
+        }
+    };
+    const int32_t q0 = g.nptr[row], q1 = g.nptr[row + 1];
+    if (q0 != q1) {
+        Rel x0, x1;                     // the p and q columns, taking turns
+        const fan_t e = g.fan[q0];
+        fan_t n = g.fan[q0 + 1 < q1 ? q0 + 1 : q0];        // one entry ahead of the loads it names
+        Raw rq = load(e.y);
+        Vec<VW> c = load_entry<UNIFORM, VW>(a.k.coef, e.z, S, lane);
+        int32_t q = q0 + 1;
+        relative(load(e.x), x0);
+        // one element: its q column into xq, the next one's loads, then the element itself; true
+        // behind the last one
+        auto element = [&](Rel &xp, Rel &xq) {
+            relative(rq, xq);
+            const Vec<VW> cf = c;
+            const int32_t apart = n.x;
+            rq = load(n.y);             // behind the last element: its own node again
+            c = load_entry<UNIFORM, VW>(a.k.coef, n.z, S, lane);
+            n = g.fan[q + 1 < q1 ? q + 1 : q1 - 1];
+            __builtin_amdgcn_sched_barrier(0);
+            apply(xp, xq, cf);
+            if (q++ >= q1) return true;
+            if (apart >= 0) relative(load(apart), xq);
+            return false;
+        };
+        while (!element(x0, x1) && !element(x1, x0)) {}
+    }
+    Vec<VW> pp[3];
+    if constexpr (BETA) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) pp[k] = own.up[k];
+    } else {
+        load_node<UNIFORM, VW>(a.up, row, S, lane, pp);
+    }
+    const RowLoad<VW> rl = row_load<VW>(a, row, s);
+    const double pn = a.load.p[step];
+    const double qa = a.load.ga ? a.load.qa[step] : 0.0;
+    const double qb = a.load.gb ? a.load.qb[step] : 0.0;
+    Vec<VW> o[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int64_t d = 3 * static_cast<int64_t>(row) + k;
+        double more = 0.0;
+        if (a.load.ga) more = qa * a.load.ga[d];
+        if (a.load.gb) more = fma(qb, a.load.gb[d], more);
+#pragma unroll
+        for (int v = 0; v < VW; ++v) {
+            double force = fma(pn, (1.0 / 6.0) * fl[k][v], more);
+            if constexpr (DAMP) force -= a.ddt * (own.u[k].v[v] - pp[k].v[v]);
+            const double m = rl.m.v[v];
+            const double rhs = fma(a.dt2, force - acc[k][v], m * fma(2.0, own.u[k].v[v], -pp[k].v[v]));
+            const double un = m != 0.0 ? rhs / m : 0.0;
+            o[k].v[v] = rl.fixed ? a.bdy_u : un;
+        }
+    }
+    if (active) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) store_vec<VW>(a.out + (static_cast<int64_t>(row) * 3 + k) * S + s, o[k]);
+    }
+}
+
 __global__ __launch_bounds__(kBlock) void k_element_stress(int64_t n_elms, int64_t S, GeomArgs g,
                                                            const double *__restrict__ u,
                                                            const double *__restrict__ ave_E,
@@ -212,6 +374,7 @@ GeomArgs geom_args(const cvfes_geometry_t *geo, const cvfes_system_t *sys, const
     g.ug = ug;
     g.nptr = sys ? sys->nptr : nullptr;
     g.nent = sys ? sys->nent : nullptr;
+    g.fan = sys ? fan_entries(sys) : nullptr;
     g.nu = geo->nu;
     g.g = 0.5 * (1.0 - geo->nu);
     g.gk = 0.5 * geo->kshear * (1.0 - geo->nu);
@@ -233,6 +396,24 @@ void launch_updated_inst(hipStream_t st, const StepArgs &a, const GeomArgs &g, i
     }
 }
 
+template <bool UNIFORM, bool GEO_U, int VW>
+void launch_moved_inst(hipStream_t st, const StepArgs &a, const GeomArgs &g, int64_t step, bool beta, bool damp) {
+    const dim3 grid(grid_for(a.k.n_nodes * lanes_per_row<UNIFORM, VW>(a.k.n_smp))), block(kBlock);
+    if (beta) {
+        if (damp) hipLaunchKernelGGL((k_step_moved<UNIFORM, true, true, GEO_U, VW>), grid, block, 0, st, a, g, step);
+        else hipLaunchKernelGGL((k_step_moved<UNIFORM, true, false, GEO_U, VW>), grid, block, 0, st, a, g, step);
+    } else {
+        if (damp) hipLaunchKernelGGL((k_step_moved<UNIFORM, false, true, GEO_U, VW>), grid, block, 0, st, a, g, step);
+        else hipLaunchKernelGGL((k_step_moved<UNIFORM, false, false, GEO_U, VW>), grid, block, 0, st, a, g, step);
+    }
+}
+
+template <bool GEO_U, int VW>
+void launch_moved(hipStream_t st, const StepArgs &a, const GeomArgs &g, int64_t step, bool beta, bool damp) {
+    if (use_uniform<VW>(a.k.n_smp)) launch_moved_inst<true, GEO_U, VW>(st, a, g, step, beta, damp);
+    else launch_moved_inst<false, GEO_U, VW>(st, a, g, step, beta, damp);
+}
+
 template <bool FAST, bool GEO_U, int VW>
 void launch_updated_u(hipStream_t st, const StepArgs &a, const GeomArgs &g, int64_t step, bool beta,
                       bool damp) {
@@ -241,14 +422,24 @@ void launch_updated_u(hipStream_t st, const StepArgs &a, const GeomArgs &g, int6
 }
 
 // Updated-geometry kernel forms (sys->variant): GENERIC the divided frames with one sample per
-// lane; ROWLOAD1 reciprocal frames, one sample per lane; ROWLOAD (and AUTO) reciprocal frames, two
-// samples per lane for even sample counts.  geo_u: the geometry displacement is the current u.
+// lane; ROWLOAD1 one sample per lane, ROWLOAD (and AUTO) two for even sample counts, without frames
+// by the fan entries (65,920 nodes x 200 samples: 560 us a step for two samples per lane, 564 for
+// one), with reciprocal frames (939 us) for systems that hold none.  geo_u: the geometry
+// displacement is the current u.
 void launch_updated(hipStream_t st, const StepArgs &a, const GeomArgs &g, int64_t step, bool beta,
                     bool damp, int64_t variant, bool geo_u) {
     const bool two = (variant == CVFES_VARIANT_AUTO || variant == CVFES_VARIANT_ROWLOAD) &&
                      a.k.n_smp % 2 == 0;
     if (variant == CVFES_VARIANT_GENERIC) {
         launch_updated_u<false, false, 1>(st, a, g, step, beta, damp);
+    } else if (g.fan) {
+        if (two) {
+            if (geo_u) launch_moved<true, 2>(st, a, g, step, beta, damp);
+            else launch_moved<false, 2>(st, a, g, step, beta, damp);
+        } else {
+            if (geo_u) launch_moved<true, 1>(st, a, g, step, beta, damp);
+            else launch_moved<false, 1>(st, a, g, step, beta, damp);
+        }
     } else if (two) {
         if (geo_u) launch_updated_u<true, true, 2>(st, a, g, step, beta, damp);
         else launch_updated_u<true, false, 2>(st, a, g, step, beta, damp);
