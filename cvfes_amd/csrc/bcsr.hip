@@ -330,7 +330,19 @@ __global__ __launch_bounds__(kBlock) void k_step_lds(StepArgs a, LdsArgs l, int6
     step_row_lds<BETA, DAMP, VW, MAXB, MAXE>(a, l, s_row[threadIdx.x / 64], row, s, active, step);
 }
 
-// values[p][ij][s] = sum_c coef[celem[c]][s] * khat[c][ij]; one thread per (block, sample).
+// lane `i`'s value, i wave-uniform
+__device__ __forceinline__ double lane_value(double x, int i) {
+    const int2 w = __builtin_bit_cast(int2, x);
+    return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_readlane(w.x, i), __builtin_amdgcn_readlane(w.y, i)));
+}
+
+// values[p][ij][s] = sum_c coef[celem[c]][s] * khat[c][ij].  The values written bound it (nine per
+// block and sample against a coefficient per contribution), so a lane holds two samples and stores
+// 16 bytes past L2: the step that follows reads more than L2 holds.  With wave-uniform rows the unit
+// blocks of up to seven contributions, which lie next to each other, come in by one load of 63
+// lanes and are broadcast from its registers; scalar loads would miss their cache on every block.
+// 131,072 upper blocks x 128 samples (1.2 GB): 337 -> 230 us.
+template <bool UNIFORM, int VW>
 __global__ __launch_bounds__(kBlock) void k_assemble(int64_t nnzb, int64_t n_smp,
                                                       const int32_t *__restrict__ bmap,
                                                       const int32_t *__restrict__ cptr,
@@ -338,23 +350,45 @@ __global__ __launch_bounds__(kBlock) void k_assemble(int64_t nnzb, int64_t n_smp
                                                       const double *__restrict__ khat,
                                                       const double *__restrict__ coef,
                                                       double *__restrict__ values) {
-    const int64_t g = xcd_block() * kBlock + threadIdx.x;
-    if (g >= nnzb * n_smp) return;
-    const int64_t p = g / n_smp;                  // output block
-    const int64_t s = g - p * n_smp;
-    const int64_t b = bmap ? bmap[p] : p;         // block of the full structure
-    double kv[9];
+    int32_t row;
+    int64_t s;
+    bool active;
+    if (!row_and_sample<UNIFORM, VW>(nnzb, n_smp, row, s, active)) return;
+    const int64_t p = static_cast<uint32_t>(row);   // output block
+    const int64_t b = bmap ? bmap[p] : p;           // block of the full structure
+    const int32_t c0 = cptr[b], c1 = cptr[b + 1];
+    Vec<VW> kv[9] = {};
+    if constexpr (UNIFORM) {
+        const int lane = threadIdx.x % 64;
+        for (int32_t c = c0; c < c1; c += 7) {
+            const int n = c1 - c < 7 ? c1 - c : 7;
+            const double mine = khat[9 * static_cast<int64_t>(c) + (lane < 9 * n ? lane : 0)];
+            Vec<VW> cf = load_vec<VW>(coef + static_cast<int64_t>(celem[c]) * n_smp + s);
+            for (int i = 0; i < n; ++i) {
+                const Vec<VW> t = cf;
+                if (i + 1 < n) cf = load_vec<VW>(coef + static_cast<int64_t>(celem[c + i + 1]) * n_smp + s);
 #pragma unroll
-    for (int ij = 0; ij < 9; ++ij) kv[ij] = 0.0;
-    for (int32_t c = cptr[b]; c < cptr[b + 1]; ++c) {
-        const double cf = coef[static_cast<int64_t>(celem[c]) * n_smp + s];
-        const double *kh = khat + 9 * static_cast<int64_t>(c);
+                for (int ij = 0; ij < 9; ++ij) {
+                    const double kh = lane_value(mine, 9 * i + ij);
 #pragma unroll
-        for (int ij = 0; ij < 9; ++ij) kv[ij] = fma(cf, kh[ij], kv[ij]);
+                    for (int v = 0; v < VW; ++v) kv[ij].v[v] = fma(t.v[v], kh, kv[ij].v[v]);
+                }
+            }
+        }
+    } else {
+        for (int32_t c = c0; c < c1; ++c) {
+            const Vec<VW> cf = load_vec<VW>(coef + static_cast<int64_t>(celem[c]) * n_smp + s);
+            const double *kh = khat + 9 * static_cast<int64_t>(c);
+#pragma unroll
+            for (int ij = 0; ij < 9; ++ij)
+#pragma unroll
+                for (int v = 0; v < VW; ++v) kv[ij].v[v] = fma(cf.v[v], kh[ij], kv[ij].v[v]);
+        }
     }
+    if (!active) return;
     double *out = values + p * 9 * n_smp + s;
 #pragma unroll
-    for (int ij = 0; ij < 9; ++ij) out[ij * n_smp] = kv[ij];
+    for (int ij = 0; ij < 9; ++ij) store_vec_nt<VW>(out + ij * n_smp, kv[ij]);
 }
 
 // x[n][j][s] = u0[3n+j] + beta * du0[3n+j]  (tile a sample-independent vector over samples)
@@ -914,15 +948,37 @@ extern "C" int64_t cvfes_step_kernel(const cvfes_system_t *sys, int method) {
     return resolve_variant(sys, method == CVFES_METHOD_MATFREE);
 }
 
+namespace {
+
+template <int VW>
+void assemble_vw(hipStream_t st, int64_t nnzb, int64_t S, const int32_t *bmap, const int32_t *cptr,
+                 const int32_t *celem, const double *khat, const double *coef, double *values) {
+    // padding the rows to whole wavefronts may not push the launch past 2^32 threads
+    if (use_uniform<VW>(S) && nnzb < (int64_t(1) << 31) / lanes_per_row<true, VW>(S))
+        hipLaunchKernelGGL((k_assemble<true, VW>), dim3(grid_for(nnzb * lanes_per_row<true, VW>(S))), dim3(kBlock),
+                           0, st, nnzb, S, bmap, cptr, celem, khat, coef, values);
+    else
+        hipLaunchKernelGGL((k_assemble<false, VW>), dim3(grid_for(nnzb * lanes_per_row<false, VW>(S))),
+                           dim3(kBlock), 0, st, nnzb, S, bmap, cptr, celem, khat, coef, values);
+}
+
+// two samples per lane and 16-byte accesses where the count and both arrays allow it
+void assemble(hipStream_t st, int64_t nnzb, int64_t S, const int32_t *bmap, const int32_t *cptr,
+              const int32_t *celem, const double *khat, const double *coef, double *values) {
+    const uintptr_t any = reinterpret_cast<uintptr_t>(coef) | reinterpret_cast<uintptr_t>(values);
+    if (S % 2 == 0 && any % 16 == 0) assemble_vw<2>(st, nnzb, S, bmap, cptr, celem, khat, coef, values);
+    else assemble_vw<1>(st, nnzb, S, bmap, cptr, celem, khat, coef, values);
+}
+
+}  // namespace
+
 extern "C" int cvfes_assemble_bcsr(void *stream, int64_t nnzb, int64_t n_smp, const int32_t *cptr,
                                    const int32_t *celem, const double *khat, const double *coef,
                                    double *values) {
     CVFES_REQUIRE(nnzb >= 0 && n_smp >= 1, "cvfes_assemble_bcsr: bad sizes");
     if (nnzb == 0) return CVFES_OK;
     CVFES_REQUIRE(cptr && celem && khat && coef && values, "cvfes_assemble_bcsr: null pointer");
-    hipLaunchKernelGGL(k_assemble, dim3(grid_for(nnzb * n_smp)), dim3(kBlock), 0,
-                       static_cast<hipStream_t>(stream), nnzb, n_smp, nullptr, cptr, celem, khat,
-                       coef, values);
+    assemble(static_cast<hipStream_t>(stream), nnzb, n_smp, nullptr, cptr, celem, khat, coef, values);
     return check_launch("k_assemble");
 }
 
@@ -932,9 +988,7 @@ extern "C" int cvfes_assemble_upper(void *stream, int64_t nnzu, int64_t n_smp, c
     CVFES_REQUIRE(nnzu >= 0 && n_smp >= 1, "cvfes_assemble_upper: bad sizes");
     if (nnzu == 0) return CVFES_OK;
     CVFES_REQUIRE(ublk && cptr && celem && khat && coef && uvalues, "cvfes_assemble_upper: null pointer");
-    hipLaunchKernelGGL(k_assemble, dim3(grid_for(nnzu * n_smp)), dim3(kBlock), 0,
-                       static_cast<hipStream_t>(stream), nnzu, n_smp, ublk, cptr, celem, khat,
-                       coef, uvalues);
+    assemble(static_cast<hipStream_t>(stream), nnzu, n_smp, ublk, cptr, celem, khat, coef, uvalues);
     return check_launch("k_assemble");
 }
 

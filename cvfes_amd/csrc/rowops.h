@@ -20,10 +20,12 @@ __host__ __device__ __forceinline__ int64_t lanes_per_row(int64_t n_smp) {
 template <bool UNIFORM, int VW>
 __device__ __forceinline__ bool row_and_sample(int64_t n_nodes, int64_t n_smp, int32_t &row,
                                                int64_t &s, bool &active) {
-    const int64_t lpr = lanes_per_row<UNIFORM, VW>(n_smp);
-    const int64_t g = xcd_block() * kBlock + threadIdx.x;
-    int64_t r = g / lpr;
-    s = (g - r * lpr) * VW;
+    // a launch has fewer than 2^32 threads, so the division is one of 32 bits (of 64 it took some
+    // hundred instructions of each short kernel)
+    const uint32_t lpr = static_cast<uint32_t>(lanes_per_row<UNIFORM, VW>(n_smp));
+    const uint32_t g = static_cast<uint32_t>(xcd_block() * kBlock + threadIdx.x);
+    uint32_t r = g / lpr;
+    s = static_cast<int64_t>(g - r * lpr) * VW;
     active = s < n_smp;
     if (!active) s = n_smp - VW;
     if constexpr (UNIFORM) r = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(r));
