@@ -82,9 +82,9 @@ struct RowArgs {
     const fan_t *fan;      // null: the matrix-free operator is walked block by block
 };
 
-// The fan entries a kernel may use: the lane offsets of the fan product are 32-bit bytes.
+// The fan entries a kernel may use: the byte offsets inside a node's samples are 31 bits.
 inline const fan_t *fan_entries(const cvfes_system_t *sys) {
-    return sys->nptr && sys->n_smp < (int64_t(1) << 28) ? reinterpret_cast<const fan_t *>(sys->fan) : nullptr;
+    return sys->nptr && sys->n_smp < (int64_t(1) << 31) / 24 ? reinterpret_cast<const fan_t *>(sys->fan) : nullptr;
 }
 
 // Block slots of the system's row records if the kernels that read the symmetric storage by them
@@ -360,6 +360,12 @@ __device__ __forceinline__ void load_node(DP base, int32_t node, int64_t n_smp, 
         for (int j = 0; j < 3; ++j)
             r[j] = load_lane<VW>(base + (static_cast<int64_t>(node) * 3 + j) * n_smp, lane);
     }
+}
+
+// lane `i`'s value, i wave-uniform
+__device__ __forceinline__ double lane_value(double x, int i) {
+    const int2 w = __builtin_bit_cast(int2, x);
+    return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_readlane(w.x, i), __builtin_amdgcn_readlane(w.y, i)));
 }
 
 // One value per sample of row `i` of an [..][S] array.
