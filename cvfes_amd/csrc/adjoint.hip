@@ -346,163 +346,167 @@ struct GradArgs {
     double *grad;
 };
 
-// sum_{a,b} nu_a^T khat_e(a,b) x_b over the element's 9 x 9 unit block; `kh(ab)` gives the 9
-// entries of unit block ab.
-template <class KH>
-__device__ __forceinline__ double grad_form(const double (&nu)[9], const double (&x)[9], KH kh) {
-    double acc = 0.0;
+// sum_{a,b} nu_a^T khat_e(a,b) x_b over the element's nodes, by the vectors relative to its node 0:
+// an element's rows and columns sum to zero and its block is symmetric, so three of the nine 3 x 3
+// unit blocks, (1,1), (1,2) and (2,2), 27 of the 81 entries, hold the form.
+constexpr int kGradKh = 27;
+
+__device__ __forceinline__ int grad_block(int r) { return r < 9 ? 4 : (r < 18 ? 5 : 8); }
+
+template <int VW, class KH>
+__device__ __forceinline__ void grad_form(const double (&nu)[2][3][VW], const double (&x)[2][3][VW], KH kh,
+                                          double (&acc)[VW]) {
+    double y[2][3][VW];
 #pragma unroll
-    for (int p = 0; p < 3; ++p) {
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int b = 0; b < 3; ++b) {
-            const auto *h = kh(3 * p + b);
+        for (int v = 0; v < VW; ++v) y[0][i][v] = y[1][i][v] = 0.0;
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                double t = 0.0;
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-                for (int j = 0; j < 3; ++j) t = fma(h[3 * i + j], x[3 * b + j], t);
-                acc = fma(nu[3 * p + i], t, acc);
+        for (int j = 0; j < 3; ++j) {
+            const double pp = kh(3 * i + j), pq = kh(9 + 3 * i + j), qq = kh(18 + 3 * i + j);
+#pragma unroll
+            for (int v = 0; v < VW; ++v) {
+                y[0][i][v] = fma(pp, x[0][j][v], y[0][i][v]);
+                y[0][i][v] = fma(pq, x[1][j][v], y[0][i][v]);
+                y[1][i][v] = fma(qq, x[1][j][v], y[1][i][v]);
+                y[1][j][v] = fma(pq, x[0][i][v], y[1][j][v]);
             }
         }
+#pragma unroll
+    for (int v = 0; v < VW; ++v) {
+        acc[v] = 0.0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) acc[v] = fma(nu[0][i][v], y[0][i][v], fma(nu[1][i][v], y[1][i][v], acc[v]));
     }
-    return acc;
 }
 
-// grad[e,s] = fma(-coef[e,s], sum_{a,b} nu_a^T khat_e(a,b) x_b, grad[e,s]) for the thread's
-// (element e, sample s), with nu = nu_scale * mu / m (nu_scale * minv with the inverse masses) and
-// x = xc + bdt (xc - xp) (x = xc when xp is NULL).
-template <class KH>
-__device__ __forceinline__ void grad_update(const GradArgs &a, int64_t e, int64_t s, KH kh) {
-    double nu[9], x[9];
+__device__ __forceinline__ double grad_scale(const GradArgs &a, double m) {
+    return a.minv ? a.nu_scale * m : (m != 0.0 ? a.nu_scale / m : 0.0);
+}
+
+// grad[e,s] = fma(-coef[e,s], sum_{a,b} nu_a^T khat_e(a,b) x_b, grad[e,s]) for the lane's element e
+// and VW samples at s, with nu = nu_scale * mu / m (nu_scale * minv with the inverse masses) and
+// x = xc + bdt (xc - xp) (x = xc when xp is NULL).  `sc` holds nu_scale / m of the three nodes where
+// the mass has no sample axis.
+template <int VW, class KH>
+__device__ __forceinline__ void grad_update(const GradArgs &a, int64_t e, int64_t s, const int32_t (&ids)[3],
+                                            const double (&sc)[3], KH kh) {
+    double nu0[3][VW], x0[3][VW], dn[2][3][VW], dx[2][3][VW], f[VW];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-        const int64_t nd = a.elems[3 * e + q];
-        const int64_t mi = a.lm_sstride ? nd * a.n_smp + s : nd;
-        double sc;
-        if (a.minv) {
-            sc = a.nu_scale * a.minv[mi];
-        } else {
-            const double m = a.lm[mi];
-            sc = m != 0.0 ? a.nu_scale / m : 0.0;
-        }
+        const int64_t nd = ids[q];
+        Vec<VW> m;
+        if (a.lm_sstride) m = load_vec<VW>((a.minv ? a.minv : a.lm) + nd * a.n_smp + s);
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             const int64_t off = (nd * 3 + j) * a.n_smp + s;
-            nu[3 * q + j] = sc * a.mu[off];
-            const double c = a.xc[off];
-            x[3 * q + j] = a.xp ? fma(a.bdt, c - a.xp[off], c) : c;
-        }
-    }
-    const int64_t idx = e * a.n_smp + s;
-    a.grad[idx] = fma(-a.coef[idx], grad_form(nu, x, kh), a.grad[idx]);
-}
-
-// The same for two consecutive samples per lane (16-byte loads; the element's node scales and
-// unit blocks serve 128 samples per wave).
-template <class KH>
-__device__ __forceinline__ void grad_update2(const GradArgs &a, int64_t e, int64_t s, KH kh) {
-    double nu[2][9], x[2][9];
+            const Vec<VW> mu = load_vec<VW>(a.mu + off), c = load_vec<VW>(a.xc + off);
+            Vec<VW> p;
+            if (a.xp) p = load_vec<VW>(a.xp + off);
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        const int64_t nd = a.elems[3 * e + q];
-        double sc[2];
-        if (a.lm_sstride) {
-            const Vec<2> m = load_vec<2>((a.minv ? a.minv : a.lm) + nd * a.n_smp + s);
-#pragma unroll
-            for (int v = 0; v < 2; ++v)
-                sc[v] = a.minv ? a.nu_scale * m.v[v] : (m.v[v] != 0.0 ? a.nu_scale / m.v[v] : 0.0);
-        } else {
-            const double m = a.minv ? a.minv[nd] : a.lm[nd];
-            sc[0] = sc[1] = a.minv ? a.nu_scale * m : (m != 0.0 ? a.nu_scale / m : 0.0);
-        }
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int64_t off = (nd * 3 + j) * a.n_smp + s;
-            const Vec<2> mu = load_vec<2>(a.mu + off);
-            const Vec<2> c = load_vec<2>(a.xc + off);
-            Vec<2> p;
-            if (a.xp) p = load_vec<2>(a.xp + off);
-#pragma unroll
-            for (int v = 0; v < 2; ++v) {
-                nu[v][3 * q + j] = sc[v] * mu.v[v];
-                x[v][3 * q + j] = a.xp ? fma(a.bdt, c.v[v] - p.v[v], c.v[v]) : c.v[v];
+            for (int v = 0; v < VW; ++v) {
+                // products and differences as written, so that every form gives the same bits
+                const double scale = a.lm_sstride ? grad_scale(a, m.v[v]) : sc[q];
+                const double x = a.xp ? fma(a.bdt, c.v[v] - p.v[v], c.v[v]) : c.v[v];
+                if (q == 0) {
+                    nu0[j][v] = scale * mu.v[v];
+                    x0[j][v] = x;
+                } else {
+                    dn[q - 1][j][v] = fma(scale, mu.v[v], -nu0[j][v]);
+                    dx[q - 1][j][v] = x - x0[j][v];
+                }
             }
         }
     }
     const int64_t idx = e * a.n_smp + s;
-    const Vec<2> cf = load_vec<2>(a.coef + idx);
-    Vec<2> g = load_vec<2>(a.grad + idx);
+    const Vec<VW> cf = load_vec<VW>(a.coef + idx);
+    Vec<VW> g = load_vec<VW>(a.grad + idx);
+    grad_form<VW>(dn, dx, kh, f);
 #pragma unroll
-    for (int v = 0; v < 2; ++v) g.v[v] = fma(-cf.v[v], grad_form(nu[v], x[v], kh), g.v[v]);
-    store_vec<2>(a.grad + idx, g);
+    for (int v = 0; v < VW; ++v) g.v[v] = fma(-cf.v[v], f[v], g.v[v]);
+    store_vec<VW>(a.grad + idx, g);
 }
 
-// Sample counts that are multiples of 128: each wave one element and 128 of its samples, two per
-// lane, waves sample group first as below.  124 VGPRs (4 waves per SIMD; a 5-wave target spills):
-// 5.02 ms against 6.24 ms for one sample per lane on the 512,000-node tube with 256 samples.
-__global__ __launch_bounds__(kBlock) void k_grad_accum_vw2(GradArgs a) {
-    const int64_t g = xcd_block() * kBlock + threadIdx.x;
-    if (g >= a.n_elms * a.n_smp / 2) return;
-    const int64_t w = g >> 6, group = w / a.n_elms;
-    const int64_t e = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(w - group * a.n_elms));
-    const int64_t s = (group * 64 + (g & 63)) * 2;
-    grad_update2(a, e, s, [&](int ab) {
-        return a.khat + 9 * static_cast<int64_t>(a.cpos[9 * e + ab]);
-    });
-}
-
-// One thread per (element, sample), unit blocks read from memory.  UNI (sample count a multiple
-// of 64): every wave holds one element and 64 of its samples, so its node ids and unit blocks are
-// scalar loads, and the waves run sample group first (all elements for samples 0-63, then
-// 64-127, ...), which keeps the gathered node data of one group in L2 between the elements that
-// share it.  At most 80 registers (6 waves per SIMD or more): left alone, the compiler hoists all
-// 81 unit-block loads and runs at 3 waves per SIMD.  (A form that applies two consecutive steps'
-// terms in one pass, reading u_{n-1}, coef and grad once, needs 123 registers and measured 10 %
-// slower per step.)
-template <bool UNI>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_grad_accum(GradArgs a) {
-    const int64_t g = xcd_block() * kBlock + threadIdx.x;
-    if (g >= a.n_elms * a.n_smp) return;
-    int64_t e, s;
-    if constexpr (UNI) {
-        const int64_t w = g >> 6, group = w / a.n_elms;
-        e = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(w - group * a.n_elms));
-        s = group * 64 + (g & 63);
-    } else {
-        e = g / a.n_smp;
-        s = g - e * a.n_smp;
+// Sample counts that are multiples of 64: each wave one element and 64 VW of its samples.  What the
+// samples share, node ids, node scales and unit blocks, comes in by one vector load each (lane r the
+// r-th entry) and is broadcast from the registers: scalar loads of 648 B an element missed their
+// cache ten times each and bound the kernel.  Waves run sample group first (all elements for the
+// first 64 VW samples, then the next), which keeps the gathered node data of one group in L2 between
+// the elements that share it.  65,536 elements x 64 samples: 114 -> 98 us.
+template <int VW>
+__global__ __launch_bounds__(kBlock) void k_grad_accum(GradArgs a) {
+    const uint32_t w = static_cast<uint32_t>(xcd_block() * kBlock + threadIdx.x) >> 6;
+    const uint32_t group = w / static_cast<uint32_t>(a.n_elms);
+    if (group >= a.n_smp / (64 * VW)) return;
+    const int64_t e = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(w - group * static_cast<uint32_t>(a.n_elms)));
+    const int lane = threadIdx.x & 63;
+    const int64_t s = (static_cast<int64_t>(group) * 64 + lane) * VW;
+    const int r = lane < kGradKh ? lane : 0;
+    const int32_t id = a.elems[3 * e + (lane < 3 ? lane : 0)];
+    const double kh = a.khat[9 * static_cast<int64_t>(a.cpos[9 * e + grad_block(r)]) + r % 9];
+    const double m = a.lm_sstride ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[id]);
+    int32_t ids[3];
+    double sc[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        ids[q] = __builtin_amdgcn_readlane(id, q);
+        sc[q] = lane_value(m, q);
     }
-    grad_update(a, e, s, [&](int ab) {
-        return a.khat + 9 * static_cast<int64_t>(a.cpos[9 * e + ab]);
-    });
+    grad_update<VW>(a, e, s, ids, sc, [&](int i) { return lane_value(kh, i); });
 }
 
-// The same with the unit blocks of the workgroup's elements staged in LDS first (cooperative
-// loads, about 3 per thread at 32 samples), for sample counts that put several elements in a
-// wave: the lanes of one element then read its 81 entries from LDS instead of issuing 81 vector
-// loads each.  Needs n_smp >= kGradLdsMinSmp (at most kGradLdsElems elements per workgroup).
-constexpr int kGradLdsMinSmp = 8;
-constexpr int kGradLdsElems = (kBlock - 1) / kGradLdsMinSmp + 2;   // 33
+// Any other sample count: lanes packed, VW samples of one element each, the ids, scales and unit
+// blocks of the workgroup's elements staged in LDS first.  The staging and the gather's latency
+// bound it.  Two samples per lane for even counts from kGradPair, one for 8 samples up (at most
+// kGradElems elements per workgroup).  98,304 elements x 32 samples: 80 -> 67 us.
+constexpr int kGradMin = 8, kGradPair = 16;
+constexpr int kGradElems = (kBlock - 1) / kGradMin + 2;   // 33
 
+template <int VW>
 __global__ __launch_bounds__(kBlock) void k_grad_accum_lds(GradArgs a) {
-    __shared__ double sk[kGradLdsElems * 81];
-    const int64_t g0 = xcd_block() * kBlock;
-    const int64_t total = a.n_elms * a.n_smp;
-    const int64_t e0 = g0 / a.n_smp;
-    int64_t e1 = (g0 + kBlock - 1) / a.n_smp;
-    if (e1 > a.n_elms - 1) e1 = a.n_elms - 1;
-    const int nel = e0 <= e1 ? static_cast<int>(e1 - e0 + 1) : 0;    // <= kGradLdsElems
-    for (int q = threadIdx.x; q < nel * 81; q += kBlock) {
-        const int le = q / 81, r = q - le * 81, ab = r / 9, ij = r - ab * 9;
-        sk[q] = a.khat[9 * static_cast<int64_t>(a.cpos[9 * (e0 + le) + ab]) + ij];
+    __shared__ double sk[kGradElems * kGradKh];
+    __shared__ double ssc[kGradElems * 3];
+    __shared__ int32_t sid[kGradElems * 3];
+    const uint32_t lpr = static_cast<uint32_t>(a.n_smp / VW), g0 = static_cast<uint32_t>(xcd_block() * kBlock);
+    const uint32_t e0 = g0 / lpr;
+    uint32_t e1 = (g0 + (kBlock - 1)) / lpr;
+    if (e1 >= a.n_elms) e1 = static_cast<uint32_t>(a.n_elms) - 1;
+    const int nel = e0 <= e1 ? static_cast<int>(e1 - e0 + 1) : 0;    // <= kGradElems
+    for (int q = threadIdx.x; q < nel * 3; q += kBlock) {
+        const int32_t id = a.elems[3 * static_cast<int64_t>(e0) + q];
+        sid[q] = id;
+        ssc[q] = a.lm_sstride ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[id]);
+    }
+    for (int q = threadIdx.x; q < nel * kGradKh; q += kBlock) {
+        const int le = q / kGradKh, r = q - le * kGradKh;
+        sk[q] = a.khat[9 * static_cast<int64_t>(a.cpos[9 * static_cast<int64_t>(e0 + le) + grad_block(r)]) + r % 9];
     }
     __syncthreads();
-    const int64_t g = g0 + threadIdx.x;
-    if (g >= total) return;
+    const uint32_t g = g0 + threadIdx.x, e = g / lpr;
+    if (e >= a.n_elms) return;
+    const int le = static_cast<int>(e - e0);
+    const int32_t ids[3] = {sid[3 * le], sid[3 * le + 1], sid[3 * le + 2]};
+    const double sc[3] = {ssc[3 * le], ssc[3 * le + 1], ssc[3 * le + 2]};
+    grad_update<VW>(a, e, static_cast<int64_t>(g - e * lpr) * VW, ids, sc,
+                    [&](int i) { return sk[kGradKh * le + i]; });
+}
+
+// Fewer than 8 samples: everything read per lane.
+__global__ __launch_bounds__(kBlock) void k_grad_accum_lane(GradArgs a) {
+    const int64_t g = xcd_block() * kBlock + threadIdx.x;
+    if (g >= a.n_elms * a.n_smp) return;
     const int64_t e = g / a.n_smp;
-    const int64_t s = g - e * a.n_smp;
-    const double *ske = sk + (e - e0) * 81;
-    grad_update(a, e, s, [&](int ab) { return ske + 9 * ab; });
+    const int32_t ids[3] = {a.elems[3 * e], a.elems[3 * e + 1], a.elems[3 * e + 2]};
+    double sc[3];
+    const double *kh[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        sc[q] = a.lm_sstride ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[ids[q]]);
+        kh[q] = a.khat + 9 * static_cast<int64_t>(a.cpos[9 * e + grad_block(9 * q)]);
+    }
+    grad_update<1>(a, e, g - e * a.n_smp, ids, sc, [&](int i) { return kh[i / 9][i % 9]; });
 }
 
 template <int MF, bool UNI, int VW>
@@ -783,16 +787,21 @@ extern "C" int cvfes_grad_accum(void *stream, const cvfes_system_t *sys, const i
     CVFES_REQUIRE(dt > 0.0, "cvfes_grad_accum: dt must be positive");
     const GradArgs a{sys->n_elms, sys->n_smp, elems, cpos, sys->khat, sys->coef, sys->lm,
                      sys->lm_sstride, sys->minv, mu, x_cur, x_prev, beta / dt, nu_scale, grad};
-    const dim3 grid(grid_for(sys->n_elms * sys->n_smp)), block(kBlock);
+    const int64_t S = sys->n_smp, work = sys->n_elms * S;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (sys->n_smp % 128 == 0)
-        hipLaunchKernelGGL(k_grad_accum_vw2, dim3(grid_for(sys->n_elms * sys->n_smp / 2)), block, 0, st, a);
-    else if (sys->n_smp % 64 == 0)
-        hipLaunchKernelGGL(k_grad_accum<true>, grid, block, 0, st, a);
-    else if (sys->n_smp >= kGradLdsMinSmp)
-        hipLaunchKernelGGL(k_grad_accum_lds, grid, block, 0, st, a);
-    else
-        hipLaunchKernelGGL(k_grad_accum<false>, grid, block, 0, st, a);
+    // two samples per lane need 16-byte alignment of every array with a sample axis
+    const uintptr_t any = reinterpret_cast<uintptr_t>(mu) | reinterpret_cast<uintptr_t>(x_cur) |
+                          reinterpret_cast<uintptr_t>(x_prev) | reinterpret_cast<uintptr_t>(grad) |
+                          reinterpret_cast<uintptr_t>(a.coef) | reinterpret_cast<uintptr_t>(a.minv ? a.minv : a.lm);
+    const bool pairs = S % 2 == 0 && any % 16 == 0;
+    auto launch = [&](auto kernel, int vw) {
+        hipLaunchKernelGGL(kernel, dim3(grid_for(work / vw)), dim3(kBlock), 0, st, a);
+    };
+    if (S % 128 == 0 && pairs) launch(k_grad_accum<2>, 2);
+    else if (S % 64 == 0) launch(k_grad_accum<1>, 1);
+    else if (S >= kGradPair && pairs) launch(k_grad_accum_lds<2>, 2);
+    else if (S >= kGradMin) launch(k_grad_accum_lds<1>, 1);
+    else launch(k_grad_accum_lane, 1);
     return check_launch("k_grad_accum");
 }
 
