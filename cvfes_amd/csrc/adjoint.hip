@@ -388,65 +388,72 @@ __device__ __forceinline__ double grad_scale(const GradArgs &a, double m) {
 
 // grad[e,s] = fma(-coef[e,s], sum_{a,b} nu_a^T khat_e(a,b) x_b, grad[e,s]) for the lane's element e
 // and VW samples at s, with nu = nu_scale * mu / m (nu_scale * minv with the inverse masses) and
-// x = xc + bdt (xc - xp) (x = xc when xp is NULL).  `sc` holds nu_scale / m of the three nodes where
-// the mass has no sample axis.
-template <int VW, class KH>
+// x = xc + bdt (xc - xp) (PREV; else x = xc).  `sc` holds nu_scale / m of the three nodes where the
+// mass has no sample axis.  All loads are issued before the first is used.
+template <bool PREV, bool LMS, int VW, class KH>
 __device__ __forceinline__ void grad_update(const GradArgs &a, int64_t e, int64_t s, const int32_t (&ids)[3],
                                             const double (&sc)[3], KH kh) {
-    double nu0[3][VW], x0[3][VW], dn[2][3][VW], dx[2][3][VW], f[VW];
+    Vec<VW> mu[3][3], c[3][3], p[3][3], m[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
         const int64_t nd = ids[q];
-        Vec<VW> m;
-        if (a.lm_sstride) m = load_vec<VW>((a.minv ? a.minv : a.lm) + nd * a.n_smp + s);
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             const int64_t off = (nd * 3 + j) * a.n_smp + s;
-            const Vec<VW> mu = load_vec<VW>(a.mu + off), c = load_vec<VW>(a.xc + off);
-            Vec<VW> p;
-            if (a.xp) p = load_vec<VW>(a.xp + off);
-#pragma unroll
-            for (int v = 0; v < VW; ++v) {
-                // products and differences as written, so that every form gives the same bits
-                const double scale = a.lm_sstride ? grad_scale(a, m.v[v]) : sc[q];
-                const double x = a.xp ? fma(a.bdt, c.v[v] - p.v[v], c.v[v]) : c.v[v];
-                if (q == 0) {
-                    nu0[j][v] = scale * mu.v[v];
-                    x0[j][v] = x;
-                } else {
-                    dn[q - 1][j][v] = fma(scale, mu.v[v], -nu0[j][v]);
-                    dx[q - 1][j][v] = x - x0[j][v];
-                }
-            }
+            mu[q][j] = load_vec<VW>(a.mu + off);
+            c[q][j] = load_vec<VW>(a.xc + off);
+            if constexpr (PREV) p[q][j] = load_vec<VW>(a.xp + off);
         }
+        if constexpr (LMS) m[q] = load_vec<VW>((a.minv ? a.minv : a.lm) + nd * a.n_smp + s);
     }
     const int64_t idx = e * a.n_smp + s;
     const Vec<VW> cf = load_vec<VW>(a.coef + idx);
     Vec<VW> g = load_vec<VW>(a.grad + idx);
+    __builtin_amdgcn_sched_barrier(0);
+    double nu0[3][VW], x0[3][VW], dn[2][3][VW], dx[2][3][VW], f[VW];
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int v = 0; v < VW; ++v) {
+            const double scale = LMS ? grad_scale(a, m[q].v[v]) : sc[q];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                // products and differences as written, so that every form gives the same bits
+                const double u = c[q][j].v[v], x = PREV ? fma(a.bdt, u - p[q][j].v[v], u) : u;
+                if (q == 0) {
+                    nu0[j][v] = scale * mu[q][j].v[v];
+                    x0[j][v] = x;
+                } else {
+                    dn[q - 1][j][v] = fma(scale, mu[q][j].v[v], -nu0[j][v]);
+                    dx[q - 1][j][v] = x - x0[j][v];
+                }
+            }
+        }
     grad_form<VW>(dn, dx, kh, f);
 #pragma unroll
     for (int v = 0; v < VW; ++v) g.v[v] = fma(-cf.v[v], f[v], g.v[v]);
     store_vec<VW>(a.grad + idx, g);
 }
 
-// Sample counts that are multiples of 64: each wave one element and 64 VW of its samples.  What the
-// samples share, node ids, node scales and unit blocks, comes in by one vector load each (lane r the
-// r-th entry) and is broadcast from the registers: scalar loads of 648 B an element missed their
-// cache ten times each and bound the kernel.  Waves run sample group first (all elements for the
-// first 64 VW samples, then the next), which keeps the gathered node data of one group in L2 between
-// the elements that share it.  65,536 elements x 64 samples: 114 -> 98 us.
-template <int VW>
+// Sample counts that are multiples of 128: each wave one element and 128 of its samples, two per
+// lane.  What the samples share, node ids, node scales and unit blocks, comes in by one vector load
+// each (lane r the r-th entry) and is broadcast from the registers: scalar loads of 648 B an element
+// missed their cache ten times each and bound the kernel.  Waves run sample group first (all
+// elements for samples 0-127, then 128-255, ...), which keeps the gathered node data of one group in
+// L2 between the elements that share it.  The gather bounds it: the address unit takes a vector
+// load's lanes at 4 a clock whatever their width, hence 16 bytes each.
+template <bool PREV, bool LMS>
 __global__ __launch_bounds__(kBlock) void k_grad_accum(GradArgs a) {
     const uint32_t w = static_cast<uint32_t>(xcd_block() * kBlock + threadIdx.x) >> 6;
     const uint32_t group = w / static_cast<uint32_t>(a.n_elms);
-    if (group >= a.n_smp / (64 * VW)) return;
+    if (group >= a.n_smp / 128) return;
     const int64_t e = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(w - group * static_cast<uint32_t>(a.n_elms)));
     const int lane = threadIdx.x & 63;
-    const int64_t s = (static_cast<int64_t>(group) * 64 + lane) * VW;
+    const int64_t s = (static_cast<int64_t>(group) * 64 + lane) * 2;
     const int r = lane < kGradKh ? lane : 0;
     const int32_t id = a.elems[3 * e + (lane < 3 ? lane : 0)];
     const double kh = a.khat[9 * static_cast<int64_t>(a.cpos[9 * e + grad_block(r)]) + r % 9];
-    const double m = a.lm_sstride ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[id]);
+    const double m = LMS ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[id]);
     int32_t ids[3];
     double sc[3];
 #pragma unroll
@@ -454,18 +461,20 @@ __global__ __launch_bounds__(kBlock) void k_grad_accum(GradArgs a) {
         ids[q] = __builtin_amdgcn_readlane(id, q);
         sc[q] = lane_value(m, q);
     }
-    grad_update<VW>(a, e, s, ids, sc, [&](int i) { return lane_value(kh, i); });
+    grad_update<PREV, LMS, 2>(a, e, s, ids, sc, [&](int i) { return lane_value(kh, i); });
 }
 
 // Any other sample count: lanes packed, VW samples of one element each, the ids, scales and unit
-// blocks of the workgroup's elements staged in LDS first.  The staging and the gather's latency
-// bound it.  Two samples per lane for even counts from kGradPair, one for 8 samples up (at most
-// kGradElems elements per workgroup).  98,304 elements x 32 samples: 80 -> 67 us.
+// blocks of the workgroup's elements staged in LDS first.  Two samples per lane for even counts from
+// kGradPair (a workgroup then still has at most kGradElems elements; four waves per SIMD: a fifth
+// waits on fewer registers, 56 us), one from kGradMin.  98,304 elements x 32 samples: 80 -> 52 us;
+// 65,536 x 64 with the damped state: 114 -> 72 us (one wave an element with one sample per lane 89).
 constexpr int kGradMin = 8, kGradPair = 16;
 constexpr int kGradElems = (kBlock - 1) / kGradMin + 2;   // 33
 
-template <int VW>
-__global__ __launch_bounds__(kBlock) void k_grad_accum_lds(GradArgs a) {
+template <bool PREV, bool LMS, int VW>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(VW == 2 && !LMS ? 4 : 1))) void
+k_grad_accum_lds(GradArgs a) {
     __shared__ double sk[kGradElems * kGradKh];
     __shared__ double ssc[kGradElems * 3];
     __shared__ int32_t sid[kGradElems * 3];
@@ -477,7 +486,7 @@ __global__ __launch_bounds__(kBlock) void k_grad_accum_lds(GradArgs a) {
     for (int q = threadIdx.x; q < nel * 3; q += kBlock) {
         const int32_t id = a.elems[3 * static_cast<int64_t>(e0) + q];
         sid[q] = id;
-        ssc[q] = a.lm_sstride ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[id]);
+        ssc[q] = LMS ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[id]);
     }
     for (int q = threadIdx.x; q < nel * kGradKh; q += kBlock) {
         const int le = q / kGradKh, r = q - le * kGradKh;
@@ -489,11 +498,12 @@ __global__ __launch_bounds__(kBlock) void k_grad_accum_lds(GradArgs a) {
     const int le = static_cast<int>(e - e0);
     const int32_t ids[3] = {sid[3 * le], sid[3 * le + 1], sid[3 * le + 2]};
     const double sc[3] = {ssc[3 * le], ssc[3 * le + 1], ssc[3 * le + 2]};
-    grad_update<VW>(a, e, static_cast<int64_t>(g - e * lpr) * VW, ids, sc,
+    grad_update<PREV, LMS, VW>(a, e, static_cast<int64_t>(g - e * lpr) * VW, ids, sc,
                     [&](int i) { return sk[kGradKh * le + i]; });
 }
 
 // Fewer than 8 samples: everything read per lane.
+template <bool PREV, bool LMS>
 __global__ __launch_bounds__(kBlock) void k_grad_accum_lane(GradArgs a) {
     const int64_t g = xcd_block() * kBlock + threadIdx.x;
     if (g >= a.n_elms * a.n_smp) return;
@@ -503,10 +513,10 @@ __global__ __launch_bounds__(kBlock) void k_grad_accum_lane(GradArgs a) {
     const double *kh[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-        sc[q] = a.lm_sstride ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[ids[q]]);
+        sc[q] = LMS ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[ids[q]]);
         kh[q] = a.khat + 9 * static_cast<int64_t>(a.cpos[9 * e + grad_block(9 * q)]);
     }
-    grad_update<1>(a, e, g - e * a.n_smp, ids, sc, [&](int i) { return kh[i / 9][i % 9]; });
+    grad_update<PREV, LMS, 1>(a, e, g - e * a.n_smp, ids, sc, [&](int i) { return kh[i / 9][i % 9]; });
 }
 
 template <int MF, bool UNI, int VW>
@@ -794,14 +804,18 @@ extern "C" int cvfes_grad_accum(void *stream, const cvfes_system_t *sys, const i
                           reinterpret_cast<uintptr_t>(x_prev) | reinterpret_cast<uintptr_t>(grad) |
                           reinterpret_cast<uintptr_t>(a.coef) | reinterpret_cast<uintptr_t>(a.minv ? a.minv : a.lm);
     const bool pairs = S % 2 == 0 && any % 16 == 0;
-    auto launch = [&](auto kernel, int vw) {
-        hipLaunchKernelGGL(kernel, dim3(grid_for(work / vw)), dim3(kBlock), 0, st, a);
+    auto run = [&](auto prev, auto lms) {
+        constexpr bool PREV = decltype(prev)::value, LMS = decltype(lms)::value;
+        auto launch = [&](auto kernel, int vw) {
+            hipLaunchKernelGGL(kernel, dim3(grid_for(work / vw)), dim3(kBlock), 0, st, a);
+        };
+        if (S % 128 == 0 && pairs) launch(k_grad_accum<PREV, LMS>, 2);
+        else if (S >= kGradPair && pairs) launch(k_grad_accum_lds<PREV, LMS, 2>, 2);
+        else if (S >= kGradMin) launch(k_grad_accum_lds<PREV, LMS, 1>, 1);
+        else launch(k_grad_accum_lane<PREV, LMS>, 1);
     };
-    if (S % 128 == 0 && pairs) launch(k_grad_accum<2>, 2);
-    else if (S % 64 == 0) launch(k_grad_accum<1>, 1);
-    else if (S >= kGradPair && pairs) launch(k_grad_accum_lds<2>, 2);
-    else if (S >= kGradMin) launch(k_grad_accum_lds<1>, 1);
-    else launch(k_grad_accum_lane, 1);
+    if (x_prev) a.lm_sstride ? run(std::true_type{}, std::true_type{}) : run(std::true_type{}, std::false_type{});
+    else a.lm_sstride ? run(std::false_type{}, std::true_type{}) : run(std::false_type{}, std::false_type{});
     return check_launch("k_grad_accum");
 }
 
