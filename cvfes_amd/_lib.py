@@ -13,7 +13,7 @@ from pathlib import Path
 import torch  # noqa: F401  (load torch's HIP runtime first)
 
 LIB_PATH = Path(__file__).resolve().parent / "libcvfes_mi355x.so"
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 METHOD_STORED = 0
 METHOD_MATFREE = 1
@@ -111,6 +111,8 @@ _SIGNATURES = {
                                           ctypes.POINTER(CvfesLoad), _f64, _f64, _f64, _vp, _vp]),
     "cvfes_step": (_int, [_vp, ctypes.POINTER(CvfesSystem), _int, ctypes.POINTER(_vp),
                           ctypes.POINTER(CvfesLoad), _i64, _f64, _f64, _f64]),
+    "cvfes_step_pressure": (_int, [_vp, ctypes.POINTER(CvfesSystem), _int, ctypes.POINTER(_vp),
+                                   _f64, _f64, _f64, _f64]),
     "cvfes_adjoint_step": (_int, [_vp, ctypes.POINTER(CvfesSystem), _int, _vp, _vp, _vp, _vp, _vp,
                                   _vp, _f64, _f64, _f64, _int]),
     "cvfes_grad_accum": (_int, [_vp, ctypes.POINTER(CvfesSystem), _vp, _vp, _vp, _vp, _vp, _f64,
@@ -191,4 +193,6 @@ def ptr(t) -> int | None:
 
 def stream_handle(device=None) -> int:
     """Raw ``hipStream_t`` of torch's current stream on ``device``."""
+    if isinstance(device, torch.device) and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)   # without a Stream object
     return torch.cuda.current_stream(device).cuda_stream

@@ -1148,11 +1148,11 @@ extern "C" int cvfes_initial_state_static(void *stream, const cvfes_system_t *sy
                               beta, damp, u, up, work);
 }
 
-extern "C" int cvfes_step(void *stream, const cvfes_system_t *sys, int method, double **state,
-                          const cvfes_load_t *load, int64_t nsteps, double dt, double beta,
-                          double damp) {
-    if (int rc = validate(sys, method, "cvfes_step")) return rc;
-    if (int rc = validate_load(load, "cvfes_step")) return rc;
+namespace {
+
+// nsteps steps under `load`, or one under the pressure p0 alone (load null).
+int run_steps(void *stream, const cvfes_system_t *sys, int method, double **state, const cvfes_load_t *load, double p0,
+              int64_t nsteps, double dt, double beta, double damp) {
     CVFES_REQUIRE(state && state[0] && state[1] && state[2], "cvfes_step: null state buffer");
     CVFES_REQUIRE(state[0] != state[1] && state[1] != state[2] && state[0] != state[2],
                   "cvfes_step: state buffers must be distinct");
@@ -1169,7 +1169,8 @@ extern "C" int cvfes_step(void *stream, const cvfes_system_t *sys, int method, d
     a.lm_sstride = sys->lm_sstride;
     a.f1 = sys->f1;
     a.fixed = sys->fixed;
-    a.load = *load;
+    if (load) a.load = *load;
+    a.p0 = p0;
     a.bdy_u = sys->bdy_u;
     a.dt2 = dt * dt;
     a.bdt = beta / dt;
@@ -1194,4 +1195,20 @@ extern "C" int cvfes_step(void *stream, const cvfes_system_t *sys, int method, d
     state[1] = prev;
     state[2] = nxt;
     return CVFES_OK;
+}
+
+}  // namespace
+
+extern "C" int cvfes_step(void *stream, const cvfes_system_t *sys, int method, double **state,
+                          const cvfes_load_t *load, int64_t nsteps, double dt, double beta,
+                          double damp) {
+    if (int rc = validate(sys, method, "cvfes_step")) return rc;
+    if (int rc = validate_load(load, "cvfes_step")) return rc;
+    return run_steps(stream, sys, method, state, load, 0.0, nsteps, dt, beta, damp);
+}
+
+extern "C" int cvfes_step_pressure(void *stream, const cvfes_system_t *sys, int method, double **state,
+                                   double pressure, double dt, double beta, double damp) {
+    if (int rc = validate(sys, method, "cvfes_step_pressure")) return rc;
+    return run_steps(stream, sys, method, state, nullptr, pressure, 1, dt, beta, damp);
 }

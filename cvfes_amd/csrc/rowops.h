@@ -111,7 +111,8 @@ struct StepArgs {
     int64_t lm_sstride;
     const double *f1;
     const uint8_t *fixed;
-    cvfes_load_t load;
+    cvfes_load_t load;    // load.p null: the pressure is p0
+    double p0;
     double bdy_u;
     double dt2;
     double bdt;           // beta / dt
@@ -589,6 +590,18 @@ __device__ __forceinline__ RowLoad<VW> row_load(const SA &a, int32_t row, int64_
     return r;
 }
 
+// Pressure of a step: from its table, or (the single-mesh step only) with the launch.  One load in
+// either case, of an address that holds: behind a branch it would wait for the row's product.
+__device__ __forceinline__ double step_pressure(const StepArgs &a, int64_t step) {
+    const double p = *(a.load.p ? a.load.p + step : a.f1);
+    return a.load.p ? p : a.p0;
+}
+
+template <class SA>
+__device__ __forceinline__ double step_pressure(const SA &a, int64_t step) {
+    return a.load.p[step];
+}
+
 // Central-difference update of one block row and VW consecutive samples from its product
 // acc = K x and its own state uu = u_n, pp = u_{n-1}: load, damping, lumped mass and Dirichlet
 // value; stores u_{n+1} when `active`.  Every product and sum that could be contracted is an
@@ -602,7 +615,7 @@ __device__ __forceinline__ void step_update(const SA &a, int32_t row, int64_t s,
                                             const double (&acc)[3][VW], const Vec<VW> (&uu)[3],
                                             const Vec<VW> (&pp)[3]) {
     const int64_t nsm = a.k.n_smp;
-    const double pn = a.load.p[step];
+    const double pn = step_pressure(a, step);
     double fi[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) fi[i] = pn * r.f1[i];
@@ -695,7 +708,7 @@ __device__ __forceinline__ void finish_row(const StepArgs &a, int32_t row, int64
                                            const typename VecT<VW>::type (&acc)[3]) {
     typedef typename VecT<VW>::type V;
     const int64_t S = a.k.n_smp;
-    const double pn = a.load.p[step];
+    const double pn = step_pressure(a, step);
     const double qa = a.load.ga ? a.load.qa[step] : 0.0;
     const double qb = a.load.gb ? a.load.qb[step] : 0.0;
     const bool fixed = a.fixed != nullptr && a.fixed[row] != 0;

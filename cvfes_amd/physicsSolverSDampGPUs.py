@@ -204,14 +204,17 @@ class GPUSolidSolver(PhysicsSolver):
     def Solve(self, t, dt):
         """One step of all samples with the load set by the last ``RefreshContext``."""
         if self.traction is None:
-            # one resident single-step table; the pressure is set by a fill on the launch stream,
-            # so there is no allocation and no host-to-device copy per step
+            # one resident single-step table; the pressure goes with the step's launch, so there
+            # is no allocation, no host-to-device copy and no second launch per step
             if self._solve_tables is None:
                 self._solve_tables = self.system.loads(np.zeros(1))
             tables = self._solve_tables
         else:
             tables = self._load_tables(np.array([self.t]))[0][1]
-        tables.p.fill_(self.pressure)
+        if self.traction is None and isinstance(tables, LoadTables):
+            tables.set_pressure(self.pressure)
+        else:
+            tables.p.fill_(self.pressure)
         self._advance(tables, dt)
         self._step_load = tables
         self._nSolve += 1

@@ -30,13 +30,17 @@ def _dev(a, dtype, device):
     return torch.as_tensor(np.ascontiguousarray(a), dtype=dtype).to(device)
 
 
+_STATE = ctypes.c_void_p * 3
+
+
 class LoadTables:
     """Device load tables ``f_n = p[n] f1 + qa[n] ga + qb[n] gb`` for a run of steps."""
 
     def __init__(self, p, device, ga=None, qa=None, gb=None, qb=None, n_nodes=None):
         f64 = torch.float64
-        self.p = p.to(device, f64).contiguous() if isinstance(p, torch.Tensor) else _dev(np.atleast_1d(np.asarray(p, np.float64)), f64, device)
-        self.n = int(self.p.numel())
+        self.value = None           # set_pressure: not yet in the table
+        self._p = p.to(device, f64).contiguous() if isinstance(p, torch.Tensor) else _dev(np.atleast_1d(np.asarray(p, np.float64)), f64, device)
+        self.n = int(self._p.numel())
         self.ga = self._field(ga, device)
         self.gb = self._field(gb, device)
         self.qa = None if qa is None else _dev(np.asarray(qa, np.float64).reshape(-1), f64, device)
@@ -51,6 +55,21 @@ class LoadTables:
         for g in (self.ga, self.gb):
             if g is not None and n_nodes is not None and tuple(g.shape) != (int(n_nodes), 3):
                 raise ValueError(f"traction field of shape {tuple(g.shape)}, expected ({n_nodes}, 3)")
+
+    @property
+    def p(self):
+        """Pressure table on the device."""
+        if self.value is not None:
+            self._p.fill_(self.value)
+            self.value = None
+        return self._p
+
+    def set_pressure(self, value):
+        """New pressure of a one-entry table without tractions.  :meth:`MembraneSystem.step` passes
+        it with its launch; the table itself is filled when something reads it."""
+        if self.n != 1 or self.ga is not None or self.gb is not None:
+            raise ValueError("set_pressure needs a one-entry table without tractions")
+        self.value = float(value)
 
     @staticmethod
     def _field(g, device):
@@ -618,8 +637,15 @@ class MembraneSystem:
         n = load.n - offset if nsteps is None else int(nsteps)
         if offset < 0 or n < 0 or offset + n > load.n:
             raise ValueError("steps exceed the load tables")
+        if load.value is not None and n == 1:
+            u, up, work = self.state
+            arr = _STATE(u.data_ptr(), up.data_ptr(), work.data_ptr())
+            check(self.lib.cvfes_step_pressure(self.stream, ctypes.byref(self._sys), self.method_id(method), arr,
+                                               load.value, float(dt), float(beta), float(damp)))
+            self.state = [work, u, up]
+            return work
         ls = load.struct(offset)
-        arr = (ctypes.c_void_p * 3)(*[b.data_ptr() for b in self.state])
+        arr = _STATE(*[b.data_ptr() for b in self.state])
         check(self.lib.cvfes_step(self.stream, ctypes.byref(self._sys), self.method_id(method), arr,
                                   ctypes.byref(ls), n, float(dt), float(beta), float(damp)))
         addr = {b.data_ptr(): b for b in self.state}

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define CVFES_ABI_VERSION 13
+#define CVFES_ABI_VERSION 14
 
 #define CVFES_OK 0
 #define CVFES_ERR_ARG (-1)   /* invalid argument (null pointer, bad size)        */
@@ -333,6 +333,14 @@ int cvfes_initial_state_static(void *stream, const cvfes_system_t *sys, int meth
  */
 int cvfes_step(void *stream, const cvfes_system_t *sys, int method, double **state,
                const cvfes_load_t *load, int64_t nsteps, double dt, double beta, double damp);
+
+/*
+ * One step of cvfes_step under the pressure `pressure` alone (no traction fields), which travels
+ * with the launch: the coupled solver's step sets a new pressure every time, and a table in device
+ * memory takes a launch of its own to set.
+ */
+int cvfes_step_pressure(void *stream, const cvfes_system_t *sys, int method, double **state,
+                        double pressure, double dt, double beta, double damp);
 
 /*
  * The step kernel cvfes_step launches for this system and method (CVFES_VARIANT_*, with AUTO and
