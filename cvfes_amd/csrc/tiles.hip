@@ -2,6 +2,7 @@
 // found on the host by recursive bisection of the node cloud, and the per-tile lists the kernels
 // read, built on the device from the fan entries.
 #include <algorithm>
+#include <cmath>
 #include <limits>
 #include <vector>
 
@@ -31,6 +32,16 @@ int64_t bisect(const double *nodes, const int32_t *indptr, const int32_t *indice
                int32_t *rows, int64_t cap) {
     std::vector<int32_t> ids(n_nodes);
     for (int64_t i = 0; i < n_nodes; ++i) ids[i] = static_cast<int32_t>(i);
+    // Extents are counted in edges: on a wall whose mesh is finer along one axis than along the
+    // others, parts of equal sides would be long strips of nodes with too many columns.
+    double edge[3] = {0.0, 0.0, 0.0};
+    for (int64_t i = 0; i < n_nodes; ++i)
+        for (int32_t p = indptr[i]; p < indptr[i + 1]; ++p)
+            for (int k = 0; k < 3; ++k) {
+                const double d = std::abs(nodes[3 * static_cast<int64_t>(indices[p]) + k] - nodes[3 * i + k]);
+                if (d < std::numeric_limits<double>::infinity()) edge[k] += d;
+            }
+    for (double &d : edge) d = d > 0.0 ? 1.0 / d : 0.0;
     std::vector<std::pair<int64_t, int64_t>> todo{{0, n_nodes}};
     int64_t n_tiles = 0;
     while (!todo.empty()) {
@@ -58,7 +69,7 @@ int64_t bisect(const double *nodes, const int32_t *indptr, const int32_t *indice
         }
         int ax = 0;
         for (int k = 1; k < 3; ++k)
-            if (hi[k] - lo[k] > hi[ax] - lo[ax]) ax = k;
+            if (edge[k] * (hi[k] - lo[k]) > edge[ax] * (hi[ax] - lo[ax])) ax = k;
         const int64_t whole = (n + kTileRows - 1) / kTileRows;
         const int64_t h = n > kTileRows ? whole / 2 * kTileRows : n / 2;
         const auto key = [&](int32_t i) {                  // NaN last: a strict order for any input
