@@ -417,11 +417,18 @@ struct StateCol {
     __device__ __forceinline__ void value(const Raw &r, double (&x)[1][3][VW]) const { column(r, x[0]); }
 };
 
+// a - b as it stands: a column that is itself a product would else be fused into the difference in
+// the kernels that form it in registers, and not in those that read it back from LDS.
+__device__ __forceinline__ double minus(double a, double b) {
+#pragma clang fp contract(off)
+    return a - b;
+}
+
 // acc[c] = the row's matrix-free product with each column c: for every element e around the row
-// node a, with p and q its other nodes, acc += coef_e (khat_e(a,a) x_a + khat_e(a,p) x_p +
-// khat_e(a,q) x_q).  Compared with the walk over blocks, the coefficient is read and applied once
-// per element instead of once per contribution, and where the entries chain around the node each
-// neighbour is read once.  The next element's loads are issued before the current one is applied.
+// node a, with p and q its other nodes, acc += coef_e (khat_e(a,p) (x_p - x_a) + khat_e(a,q) (x_q -
+// x_a)): an element's rows sum to zero, so its block (a,a) is neither read nor applied.  Compared
+// with the walk over blocks, the coefficient is read and applied once per element instead of once
+// per contribution, and where the entries chain around the node each neighbour is read once.  The next element's loads are issued before the current one is applied.
 // A row's contributions are contiguous, so its unit blocks start at contribution 3 nptr[row].
 template <bool UNI, int VW, class COL, class RA>
 __device__ __forceinline__ void fan_product(const RA &k, const COL &col, int32_t row,
@@ -436,23 +443,31 @@ __device__ __forceinline__ void fan_product(const RA &k, const COL &col, int32_t
     const int32_t q0 = k.nptr[row], q1 = k.nptr[row + 1];
     if (q0 == q1) return;
     const auto *kh0 = k.khat + 27 * static_cast<int64_t>(q0);
-    double xa[NC][3][VW], xp[NC][3][VW], xq[NC][3][VW];
+    double xa[NC][3][VW], xp[NC][3][VW], xq[NC][3][VW];     // xp, xq less xa
+    auto relative = [&](const typename COL::Raw &raw, double (&x)[NC][3][VW]) {
+        col.value(raw, x);
+#pragma unroll
+        for (int m = 0; m < NC; ++m)
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+#pragma unroll
+                for (int v = 0; v < VW; ++v) x[m][j][v] = minus(x[m][j][v], xa[m][j][v]);
+    };
     fan_t e = k.fan[q0];
     typename COL::Raw r = col.load(e.y);
     Vec<VW> c = load_entry<UNI, VW>(k.coef, e.z, k.n_smp, col.lane);
     {
         const typename COL::Raw ra = col.load(row), rp = col.load(e.x);
         col.value(ra, xa);
-        col.value(rp, xp);
+        relative(rp, xp);
     }
     for (int32_t q = q0 + 1;; ++q) {
         const fan_t n = k.fan[q < q1 ? q : q1 - 1];
-        col.value(r, xq);
+        relative(r, xq);
         const Vec<VW> cf = c;
         r = col.load(n.y);              // behind the last element: its own node again
         c = load_entry<UNI, VW>(k.coef, n.z, k.n_smp, col.lane);
         __builtin_amdgcn_sched_barrier(0);
-        const auto *ka = kh0 + 9 * (e.w & 1023);
         const auto *kp = kh0 + 9 * ((e.w >> 10) & 1023);
         const auto *kq = kh0 + 9 * ((e.w >> 20) & 1023);
 #pragma unroll
@@ -461,18 +476,16 @@ __device__ __forceinline__ void fan_product(const RA &k, const COL &col, int32_t
             for (int m = 0; m < NC; ++m)
 #pragma unroll
                 for (int v = 0; v < VW; ++v) {
-                    double t = ka[3 * i] * xa[m][0][v];
-                    t = fma(ka[3 * i + 1], xa[m][1][v], t);
-                    t = fma(ka[3 * i + 2], xa[m][2][v], t);
+                    double t = kp[3 * i] * xp[m][0][v];
 #pragma unroll
-                    for (int j = 0; j < 3; ++j) t = fma(kp[3 * i + j], xp[m][j][v], t);
+                    for (int j = 1; j < 3; ++j) t = fma(kp[3 * i + j], xp[m][j][v], t);
 #pragma unroll
                     for (int j = 0; j < 3; ++j) t = fma(kq[3 * i + j], xq[m][j][v], t);
                     acc[m][i][v] = fma(cf.v[v], t, acc[m][i][v]);
                 }
         if (q >= q1) break;
         if (n.x >= 0) {
-            col.value(col.load(n.x), xp);
+            relative(col.load(n.x), xp);
         } else {
 #pragma unroll
             for (int m = 0; m < NC; ++m)

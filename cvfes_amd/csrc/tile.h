@@ -28,10 +28,10 @@ typedef int32_t word4_t __attribute__((ext_vector_type(4)));
 constexpr int kTileThreads = 32 * kTileRows;      // half a wavefront per row at most
 
 struct TileArgs {
-    const CVFES_G word4_t *head;    // [T][kTileRows] node (-1: none), first fan entry, fan entries
+    const CVFES_G word4_t *head;    // [T][kTileRows] node (-1: none), first fan entry, fan entries, cut | skip << 16
     const CVFES_G int32_t *cols;    // [T][kTileCols - kTileRows] halo nodes (-1: none)
     const CVFES_G word4_t *ents;    // [T][kTileRows][kTileElems / 2] two entries each: element; slots
-                                    // p, q and block positions
+                                    // p, q and where its blocks (a,p), (a,q) start
     int32_t chunks;        // chunks of the samples
     int32_t chunk;         // samples per chunk (a multiple of the lane width)
     int32_t lanes;         // lanes per row, chunk / VW
@@ -57,9 +57,13 @@ inline TileShape tile_shape(int64_t n_smp) {
     return t;
 }
 
+// Unit block values staged per row: the blocks (a,p) and (a,q) of its elements, and up to two values
+// of the skipped blocks (a,a) (k_tile_lists keeps the copies in aligned pairs).
+__host__ __device__ constexpr int tile_kh(int elems) { return 18 * elems + 2; }
+
 inline size_t tile_lds(int chunk, int elems) {
     return sizeof(double) * (static_cast<size_t>(kTileCols) * 3 * chunk +
-                             static_cast<size_t>(kTileRows) * 27 * elems);
+                             static_cast<size_t>(kTileRows) * tile_kh(elems));
 }
 
 inline TileArgs tile_args(const cvfes_system_t *sys, const TileShape &h) {
@@ -93,8 +97,8 @@ __device__ __forceinline__ void tile_product(const RA &k, const TileArgs &t, con
                                              int i, int l, bool in, word4_t rw, double (&acc)[3][VW], EARLY early) {
     extern __shared__ double s_tile[];
     const int pitch = 3 * t.chunk;                      // doubles per column
-    double *s_kh = s_tile + i * 27 * ELEMS;
-    double *s_x = s_tile + kTileRows * 27 * ELEMS;
+    double *s_kh = s_tile + i * tile_kh(ELEMS);
+    double *s_x = s_tile + kTileRows * tile_kh(ELEMS);
     int32_t ew[ELEMS];
     Vec<VW> cf[ELEMS];
     const int32_t node = rw.x >= 0 ? rw.x : 0;
@@ -106,7 +110,7 @@ __device__ __forceinline__ void tile_product(const RA &k, const TileArgs &t, con
     // Unit blocks, two values a round, kAhead rounds in flight at a time: by the lanes of the row (all
     // its rounds at once when the row has half a wavefront), or, with one or two samples, by the
     // wavefront's lanes shared out over its rows.
-    constexpr int kAhead = SMALL ? 11 : (ELEMS + 1) / 2;
+    constexpr int kAhead = SMALL ? 14 : (tile_kh(ELEMS) / 2 + 31) / 32;
     int si = i, l0 = 2 * l, ls = 2 * t.lanes;
     word4_t sw = rw;
     if constexpr (SMALL) {
@@ -119,14 +123,17 @@ __device__ __forceinline__ void tile_product(const RA &k, const TileArgs &t, con
         if (lane / n < t.groups && si < kTileRows) sw = t.head[static_cast<int64_t>(tile) * kTileRows + si];
         else si = 0;
     }
-    const int nk = 27 * sw.z - 2;       // the last round's first value; negative: nothing to stage
+    // values from `cut` on are those `skip` further on in the row's blocks (k_tile_lists)
+    const int cut = sw.w & 0xffff, skip = sw.w >> 16;
+    const int nk = 27 * sw.z - skip - 2;       // the last round's first value; negative: nothing to stage
     const auto *kh = k.khat + 27 * static_cast<int64_t>(sw.y);
-    double *s_st = s_tile + si * 27 * ELEMS;
+    double *s_st = s_tile + si * tile_kh(ELEMS);
     double kv[kAhead][2];
     auto fetch = [&](int at) {
 #pragma unroll
         for (int j = 0; j < kAhead; ++j) {
-            const auto *p = kh + min(at + j * ls, nk);
+            const int to = min(at + j * ls, nk);
+            const auto *p = kh + (to < cut ? to : to + skip);
             kv[j][0] = p[0];
             kv[j][1] = p[1];
         }
@@ -196,25 +203,22 @@ __device__ __forceinline__ void tile_product(const RA &k, const TileArgs &t, con
         for (int j = 0; j < 3; ++j) {
             const Vec<VW> r = load_vec<VW>(d + j * t.chunk);
 #pragma unroll
-            for (int v = 0; v < VW; ++v) x[j][v] = r.v[v];
+            for (int v = 0; v < VW; ++v) x[j][v] = minus(r.v[v], xa[j][v]);
         }
     };
-    // element e with its p column in x0; its q column goes to x1
+    // element e with its p column (less the row's own) in x0; its q column goes to x1
     auto apply = [&](int e, int before, double (&x0)[3][VW], double (&x1)[3][VW]) {
         const int w = ew[e];
         if ((w & 255) != before) get(w & 255, x0);
         get((w >> 8) & 255, x1);
-        const double *ka = s_kh + 9 * ((w >> 16) & 31), *kp = s_kh + 9 * ((w >> 21) & 31),
-                     *kq = s_kh + 9 * ((static_cast<uint32_t>(w) >> 26) & 31);
+        const double *kp = s_kh + ((w >> 16) & 255), *kq = s_kh + (static_cast<uint32_t>(w) >> 24);
 #pragma unroll
         for (int r = 0; r < 3; ++r)
 #pragma unroll
             for (int v = 0; v < VW; ++v) {
-                double y = ka[3 * r] * xa[0][v];
-                y = fma(ka[3 * r + 1], xa[1][v], y);
-                y = fma(ka[3 * r + 2], xa[2][v], y);
+                double y = kp[3 * r] * x0[0][v];
 #pragma unroll
-                for (int j = 0; j < 3; ++j) y = fma(kp[3 * r + j], x0[j][v], y);
+                for (int j = 1; j < 3; ++j) y = fma(kp[3 * r + j], x0[j][v], y);
 #pragma unroll
                 for (int j = 0; j < 3; ++j) y = fma(kq[3 * r + j], x1[j][v], y);
                 acc[r][v] = fma(cf[e].v[v], y, acc[r][v]);

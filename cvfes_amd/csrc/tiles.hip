@@ -102,7 +102,15 @@ __global__ __launch_bounds__(kBlock) void k_tile_lists(int64_t n_tiles, const in
         const int32_t a = __shfl(mine, i);
         const int32_t q0 = a >= 0 ? nptr[a] : 0;
         const int32_t ne = a >= 0 ? min(nptr[a + 1] - q0, kTileElems) : 0;
-        if (lane == 0) head[t * kTileRows + i] = make_int4(a, q0, ne, 0);
+        // The row's contributions lie block by block, the ne of its own block (a,a) next to each other
+        // from d0 on.  The kernels stage them in aligned pairs of values without those: as they lie up
+        // to `cut`, then from `skip` further on, both even, so up to two values of (a,a) stay.
+        int d0 = 3 * kTileElems;
+        for (int k = 0; k < ne; ++k) d0 = min(d0, fan[q0 + k].w & 1023);
+        const int cut = ne ? (9 * d0 + 1) & ~1 : 0;
+        const int skip = ne ? (9 * (d0 + ne) & ~1) - cut : 0;
+        const auto at = [&](int pos) { return 9 * pos - (pos > d0 ? skip : 0); };
+        if (lane == 0) head[t * kTileRows + i] = make_int4(a, q0, ne, cut | skip << 16);
         int before = 0;
         for (int k = 0; k < ne; ++k) {
             const fan_t e = fan[q0 + k];
@@ -116,8 +124,8 @@ __global__ __launch_bounds__(kBlock) void k_tile_lists(int64_t n_tiles, const in
             before = slot[1];
             if (lane == 0)
                 ents[(t * kTileRows + i) * kTileElems + k] = make_int2(
-                    e.z, slot[0] | slot[1] << 8 | (e.w & 31) << 16 | ((e.w >> 10) & 31) << 21 |
-                             ((e.w >> 20) & 31) << 26);
+                    e.z, static_cast<int32_t>(slot[0] | slot[1] << 8 | at((e.w >> 10) & 1023) << 16 |
+                                              static_cast<uint32_t>(at((e.w >> 20) & 1023)) << 24));
         }
         if (lane >= ne && lane < kTileElems) ents[(t * kTileRows + i) * kTileElems + lane] = make_int2(0, 0);
     }

@@ -47,7 +47,9 @@ typedef struct cvfes_system {
     const double *values;     /* [nnzb][9][S] stored values                                    */
     const int32_t *cptr;      /* [nnzb+1] contribution ranges per block                        */
     const int32_t *celem;     /* [9E] element of each contribution                             */
-    const double *khat;       /* [9E][9] unit-coefficient element block of each contribution   */
+    const double *khat;       /* [9E][9] unit-coefficient element block of each contribution; the
+                                 kernels by fan entries, by tiles and of the gradient take an
+                                 element's rows to sum to zero and its block to be symmetric     */
     const double *coef;       /* [E][S] stiffness coefficient per element and sample           */
     const double *lm;         /* lumped mass, [N][S] (lm_sstride = 1) or [N] (lm_sstride = 0)  */
     int64_t lm_sstride;
@@ -111,8 +113,8 @@ typedef struct cvfes_system {
      * around the node, as cvfes_node_fans writes them. */
     const int32_t *fan;
     /* Node tiles of the matrix-free kernels (n_tiles = 0: none, they walk row by row), as
-     * cvfes_tile_rows and cvfes_tile_lists make them; they need fan and max_node_elems <=
-     * CVFES_TILE_ELEMS.  The results do not depend on them. */
+     * cvfes_tile_rows and cvfes_tile_lists make them; they need fan, max_node_elems <=
+     * CVFES_TILE_ELEMS and elements of three distinct nodes.  The results do not depend on them. */
     const int32_t *tile_head;   /* [n_tiles][CVFES_TILE_ROWS][4]                                */
     const int32_t *tile_cols;   /* [n_tiles][CVFES_TILE_COLS - CVFES_TILE_ROWS]                 */
     const int32_t *tile_ents;   /* [n_tiles][CVFES_TILE_ROWS][CVFES_TILE_ELEMS][2]              */
