@@ -1,7 +1,7 @@
 """The kernels with a row per element or block at every lane width, row mapping and alignment: the
 stresses against the oracle (some 100 roundings of 1.1e-16 and gradients no worse conditioned than
 10: 1e-12 of the largest), the assembled blocks against the contributions summed in 64 bits (at most
-40 products and sums: 1e-14 of the sum of magnitudes)."""
+40 products and sums: 1e-14 of the sum of magnitudes), the coefficients against NumPy."""
 import numpy as np
 import pytest
 import torch
@@ -65,3 +65,23 @@ def test_assembled_rows(require_gpu, kind, S, symmetric, by):
     for i, b in enumerate(blocks):
         terms = kh[cp[b]:cp[b + 1], :, None] * cf[ce[cp[b]:cp[b + 1]], None, :]
         assert np.all(np.abs(got[i] - terms.sum(0)) <= 1e-14 * np.abs(terms).sum(0))
+
+
+@pytest.mark.parametrize("S", [1, 2, 33, 64, 97, 100, 130])
+@pytest.mark.parametrize("thick_samples,node_field,log,by", [
+    (False, False, False, 0), (True, False, True, 0), (True, True, False, 1), (False, True, False, 0)])
+def test_coefficient_rows(require_gpu, S, thick_samples, node_field, log, by):
+    from cvfes_amd import _lib
+    nodes, el, E, s = system("grid", 2)
+    n, rng, p = nodes.shape[0], np.random.default_rng(S), _lib.ptr
+    h = 0.07 * rng.uniform(0.5, 1.5, (n, S) if thick_samples else (n, 1))
+    E = np.exp(rng.standard_normal((n if node_field else el.shape[0], S)))
+    out = shifted(np.full((el.shape[0], S), np.nan), by)
+    hd, Ed = shifted(h, by), shifted(np.log(E) if log else E, by)
+    _lib.check(s.lib.cvfes_element_coef(s.stream, el.shape[0], S, p(s.elems), p(hd), int(thick_samples),
+                                        p(Ed) if node_field else None, None if node_field else p(Ed), int(log), p(out)))
+    i, j = el[:, [0, 0, 1]], el[:, [1, 2, 2]]
+    Eq = 0.5 * (E[i] + E[j]) if node_field else E[:, None]
+    ref = (0.5 * (h[i] + h[j]) * Eq).sum(1) / 3.0
+    # a dozen roundings, and with the logarithm an argument off by an ulp and exp's own
+    assert np.all(np.abs(out.cpu().numpy() - ref) <= 1e-14 * ref)
