@@ -64,6 +64,10 @@ class LoadTables:
             self.value = None
         return self._p
 
+    @p.setter
+    def p(self, table):
+        self._p, self.value = table, None
+
     def set_pressure(self, value):
         """New pressure of a one-entry table without tractions.  :meth:`MembraneSystem.step` passes
         it with its launch; the table itself is filled when something reads it."""
@@ -289,7 +293,7 @@ class MembraneSystem:
                                                ptr(self.celem), ptr(self.khat), ptr(self.coef),
                                                ptr(self.values)))
         if self.storage == "sym" or self.uvalues is not None:
-            self.assemble_upper()
+            self._form_upper()
         if hasattr(self, "_sys"):
             self._sys = self._make_struct()
 
@@ -306,6 +310,11 @@ class MembraneSystem:
     def assemble_upper(self):
         """Form (or re-form) the symmetric storage ``uvalues [nnzu][9][S]`` (upper blocks only) used
         by the ``sym`` step variants."""
+        self._form_upper()
+        if hasattr(self, "_sys"):
+            self._sys = self._make_struct()
+
+    def _form_upper(self):
         S = self.n_smp
         if self.uvalues is None:
             self.uvalues = torch.empty((self.nnzu, 9, S), dtype=torch.float64, device=self.device)
@@ -314,8 +323,6 @@ class MembraneSystem:
                                             ptr(self.uvalues)))
         if self.row_records is None:
             self._build_records()
-        if hasattr(self, "_sys"):
-            self._sys = self._make_struct()
 
     def _record_slots(self):
         """Block slots of the symmetric kernels for this structure (as the C side picks them), or

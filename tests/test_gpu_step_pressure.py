@@ -31,6 +31,8 @@ def test_pressure_with_the_launch(require_gpu, S, method, variant, storage):
             s.step(load, dt, beta=1e-7, damp=5.0, method=method)
         got.append([t.cpu() for t in s.state[:2]])
         assert float(load.p[0]) == pressures[-1]
+        load.p = torch.full_like(load.p, 7.0)
+        assert load.value is None and load.struct(0).p == load.p.data_ptr()
     assert all(torch.equal(a, b) and bool(a.abs().max() > 0) for a, b in zip(*got))
 
 
