@@ -12,10 +12,10 @@
 // gather every column from L1/L2 for each of its about 7 rows, 77 KB per row and 128 samples, which
 // keeps the L1 path 73 % busy.  A tile of 16 rows has about 35 columns, so a row costs 2.2 column
 // loads instead of 8, and one wait for memory instead of one per element; the unit blocks are
-// coalesced loads.  The step at 102,400 nodes: 505 -> 358 us with 128 samples (1.77 GB of traffic,
-// 4.9 TB/s), 99 -> 50 us with 32 on 49,152 nodes, 52 -> 37 us with 1.  What bounds it now is the
-// wait for memory at the start of a workgroup: two of 512 threads and 80 KB fit a CU (128 registers,
-// 16 rows x 64 samples), and 67 % of their cycles are waits.  Tiles of 8 rows (three workgroups) and
+// coalesced loads.  The step at 102,400 nodes: 505 -> 328 us with 128 samples, 99 -> 41 us with 32 on
+// 49,152 nodes, 52 -> 26 us with 1.  What bounds it now is memory traffic (1.4 GB with the columns
+// that neighbouring tiles share) and the wait for it at the start of a workgroup: two of 512 threads
+// and 74 KB fit a CU (128 registers, 16 rows x 64 samples), two thirds of whose cycles are waits.  Tiles of 8 rows (three workgroups) and
 // chunks of 32 samples measured 4 % and 45 % slower.
 #pragma once
 
@@ -79,8 +79,9 @@ inline unsigned tile_grid(const TileArgs &t) {
 }
 
 // Up to this many samples a wavefront holds so many rows that each has few lanes to stage its unit
-// blocks with; they are then staged by all lanes of the wavefront (SMALL), 11 rounds in flight
-// (102,400 nodes: 1 sample 37 us, 5 samples 48, 8 samples 52, against 55, 53 and 58 without).
+// blocks with; they are then staged by all lanes of the wavefront (SMALL), 14 rounds in flight
+// (102,400 nodes: 1 sample 26 us, 5 samples 33, 8 samples 42; with all 27 values an element 37, 48
+// and 52, against 55, 53 and 58 staged by the row's lanes).
 constexpr int kTileSmall = 8;
 
 // Whether the matrix-free kernels of this system run by tiles.
