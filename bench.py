@@ -64,9 +64,13 @@ def algorithmic_bytes(sysm, method):
     if getattr(sysm, "row_order", None) is not None:
         small += 4 * N                                 # the visiting order
     if method == "stored" and reads_upper_blocks(sysm):                  # symmetric storage
-        op = sysm.nnzu * 9 * S * 8 + 4 * nnzb                          # upper values, vblk
+        # upper values (six of a diagonal block's nine entries), vblk
+        op = (sysm.nnzu * 9 - 3 * N) * S * 8 + 4 * nnzb
     elif method == "stored":
         op = nnzb * 9 * S * 8
+    elif sysm.n_tiles:                                                   # node tiles
+        # coef, two unit blocks of three per element and node, the tiles' lists
+        op = E * S * 8 + 6 * E * 9 * 8 + sum(x.numel() * 4 for x in (sysm.tile_head, sysm.tile_cols, sysm.tile_ents))
     else:
         op = E * S * 8 + 9 * E * 9 * 8 + 4 * 9 * E + 4 * (nnzb + 1)   # coef, khat, celem, cptr
     return state + lm + small + op
@@ -522,10 +526,12 @@ def run_batch(args):
 
 
 # FP64 operations of the updated-geometry step per (row node, sample, incident element), FMA = 2,
-# square root and division = 1 each: frame (edge vectors 6, two normalisations 2 x (5 + 1 + 1 + 3),
+# roots and divisions = 1 each.  Without frames: the normal 9 + 5 + 1, two gradients 18, edge products
+# 7, the shear vector 9, four projections 20, the factors 19, sums 30, and per neighbour the relative
+# edge and displacement 14.  The generic form: frame (edge vectors 6, two normalisations 2 x (5 + 1 + 1 + 3),
 # projection 5 + 6, cross product 9), local coordinates 30, area 12, edge terms 6, element scale 4,
 # three blocks applied in the local frame 3 x 46, accumulation 21, follower load 9.
-UPDATED_FLOPS_PER_ROW_ELEMENT = 272
+UPDATED_FLOPS_PER_ROW_ELEMENT = {"generic": 272, "rowload1": 132, "rowload": 132}
 UPDATED_FLOPS_PER_ROW = 20          # the central-difference update of the row (3 components)
 
 
@@ -562,7 +568,6 @@ def run_updated(args):
     steps = 100 if args.steps is None else args.steps
     warm = 5 if args.warmup is None else args.warmup
     load = sysm.loads(case.pressures(0, 2 * (warm + steps) + 10, dt))
-    flops = (UPDATED_FLOPS_PER_ROW_ELEMENT * 3 * E + UPDATED_FLOPS_PER_ROW * N) * S
     st = torch.cuda.current_stream()
     res = {}
     for interval in (1, 10):
@@ -581,6 +586,7 @@ def run_updated(args):
             if not bool(torch.isfinite(sysm.u).all()):
                 raise RuntimeError(f"updated step ({form}): non-finite displacement")
             ms = e0.elapsed_time(e1) / steps
+            flops = (UPDATED_FLOPS_PER_ROW_ELEMENT[form] * 3 * E + UPDATED_FLOPS_PER_ROW * N) * S
             abytes = updated_algorithmic_bytes(sysm, interval)
             res[f"interval{interval}-{form}"] = {
                 "kernel_ms": ms, "sample_steps_per_s": S / (ms * 1e-3),
@@ -602,7 +608,7 @@ def run_updated(args):
                       "beta": beta, "dt": dt},
            "roofline": {"bound": "fp64", "achieved": best["fp64"]["achieved_TFLOPs"],
                         "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": best["fp64"]["frac"],
-                        "hbm_frac": best["hbm"]["frac"], "flops_per_launch": flops},
+                        "hbm_frac": best["hbm"]["frac"], "flops_per_launch": best["fp64"]["flops_per_launch"]},
            "forms": res}
     print(json.dumps(out), flush=True)
 

@@ -13,7 +13,7 @@
 // keeps the L1 path 73 % busy.  A tile of 16 rows has about 35 columns, so a row costs 2.2 column
 // loads instead of 8, and one wait for memory instead of one per element; the unit blocks are
 // coalesced loads.  The step at 102,400 nodes: 505 -> 328 us with 128 samples, 99 -> 41 us with 32 on
-// 49,152 nodes, 52 -> 26 us with 1.  What bounds it now is memory traffic (1.4 GB with the columns
+// 49,152 nodes, 52 -> 26 us with 1.  What bounds it now is memory traffic (1.51 GB with the columns
 // that neighbouring tiles share) and the wait for it at the start of a workgroup: two of 512 threads
 // and 74 KB fit a CU (128 registers, 16 rows x 64 samples), two thirds of whose cycles are waits.  Tiles of 8 rows (three workgroups) and
 // chunks of 32 samples measured 4 % and 45 % slower.
