@@ -38,3 +38,27 @@ def test_moved_equals_frames(require_gpu, kind, S, interval, beta, damp, form):
     assert top > 0 and all(np.all(np.isfinite(g)) for g in got)
     assert np.max(np.abs(got[1] - got[0])) < 1e-12 * top
     assert np.max(np.abs(got[1] - got[2])) < 1e-12 * top
+
+
+@pytest.mark.parametrize("S,interval,beta", [(200, 1, 1e-7), (255, 3, 0.0)])
+def test_rows_by_tiles_equal_natural_order(require_gpu, S, interval, beta):
+    """Systems large enough for the tiles' row order give the bits of the natural order."""
+    from cvfes_amd.mesh import tube_geometry
+    from cvfes_amd.system import MembraneSystem
+    nodes, el, bdy = tube_geometry(96, 97, 0.3, 2.0)
+    assert 24 * nodes.shape[0] * S > 32 << 20
+    E = 7e6 * np.exp(0.1 * np.random.default_rng(S).standard_normal((el.shape[0], S)))
+    u0 = 1e-3 * np.random.default_rng(1).standard_normal(3 * nodes.shape[0])
+    s = MembraneSystem(nodes, el, bdy, S, vthickness=np.full(nodes.shape[0], 0.07), elmE=E, density=1.0, nu=0.45,
+                       store_values=False)
+    got, tiles = [], s.n_tiles
+    assert tiles > 0
+    for n in (tiles, 0):
+        s.n_tiles = n
+        s._sys = s._make_struct()
+        ls = s.loads(np.full(5, 1.33e4))
+        s.initial_state(u0, 0.0 * u0, ls, 1e-6, beta=beta, damp=5.0, method="matfree")
+        s.step_updated(ls, 1e-6, interval, beta=beta, damp=5.0)
+        got.append(s.u.cpu().numpy())
+    # the initial product runs by rows either way
+    assert np.max(np.abs(got[0])) > 0 and np.array_equal(got[0], got[1])
