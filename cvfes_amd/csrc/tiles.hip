@@ -11,23 +11,26 @@
 namespace cvfes {
 namespace {
 
-// Distinct columns of the block rows ids[0..n), at most `most + 1` of them counted.
-int count_columns(const int32_t *ids, int n, const int32_t *indptr, const int32_t *indices, int most) {
-    int32_t seen[kTileCols + 1];
-    int m = 0;
+// Distinct columns of the block rows ids[0..n) that are not themselves among ids, at most `most + 1`
+// of them counted: the halo columns of a tile of these rows.  (A node of no element has an empty
+// row and is no column of it, so the halo is not the row's columns less n.)
+int count_halo(const int32_t *ids, int n, const int32_t *indptr, const int32_t *indices, int most) {
+    int32_t seen[kTileCols];
+    for (int i = 0; i < n; ++i) seen[i] = ids[i];
+    int m = n;
     for (int i = 0; i < n; ++i)
         for (int32_t p = indptr[ids[i]]; p < indptr[ids[i] + 1]; ++p) {
             int j = 0;
             while (j < m && seen[j] != indices[p]) ++j;
             if (j < m) continue;
-            if (m == most) return most + 1;
+            if (m - n == most) return most + 1;
             seen[m++] = indices[p];
         }
-    return m;
+    return m - n;
 }
 
 // Halve the nodes across their longest extent, on a multiple of the tile size, until a part is a
-// tile; a tile with too many columns is halved again.
+// tile; a tile with too many halo columns is halved again.
 int64_t bisect(const double *nodes, const int32_t *indptr, const int32_t *indices, int64_t n_nodes,
                int32_t *rows, int64_t cap) {
     std::vector<int32_t> ids(n_nodes);
@@ -48,9 +51,9 @@ int64_t bisect(const double *nodes, const int32_t *indptr, const int32_t *indice
         const auto [a, b] = todo.back();
         todo.pop_back();
         const int64_t n = b - a;
-        const int most = kTileCols - kTileRows + static_cast<int>(n);      // its rows and the halo slots
+        const int halo = kTileCols - kTileRows;
         if (n == 1 || (n <= kTileRows &&
-                       count_columns(&ids[a], static_cast<int>(n), indptr, indices, most) <= most)) {
+                       count_halo(&ids[a], static_cast<int>(n), indptr, indices, halo) <= halo)) {
             if (n_tiles == cap) return -1;
             std::sort(ids.begin() + a, ids.begin() + b);
             for (int i = 0; i < kTileRows; ++i) rows[n_tiles * kTileRows + i] = i < n ? ids[a + i] : -1;
@@ -86,6 +89,9 @@ int64_t bisect(const double *nodes, const int32_t *indptr, const int32_t *indice
     return n_tiles;
 }
 
+// Last column slot of a tile whose rows name more columns or elements than the slots hold.
+constexpr int32_t kTileOver = -2;
+
 // One wavefront per tile: lane c holds the node of column slot c (rows first, then the halo in the
 // order the entries name it); every node of the entries is looked up with a ballot.
 __global__ __launch_bounds__(kBlock) void k_tile_lists(int64_t n_tiles, const int32_t *__restrict__ rows,
@@ -98,10 +104,12 @@ __global__ __launch_bounds__(kBlock) void k_tile_lists(int64_t n_tiles, const in
     const int32_t mine = lane < kTileRows ? rows[t * kTileRows + lane] : -1;
     int32_t held = mine;
     int m = kTileRows;
+    bool over = false;
     for (int i = 0; i < kTileRows; ++i) {
         const int32_t a = __shfl(mine, i);
         const int32_t q0 = a >= 0 ? nptr[a] : 0;
         const int32_t ne = a >= 0 ? min(nptr[a + 1] - q0, kTileElems) : 0;
+        over |= a >= 0 && nptr[a + 1] - q0 > kTileElems;
         // The row's contributions lie block by block, the ne of its own block (a,a) next to each other
         // from d0 on.  The kernels stage them in aligned pairs of values without those: as they lie up
         // to `cut`, then from `skip` further on, both even, so up to two values of (a,a) stay.
@@ -129,7 +137,9 @@ __global__ __launch_bounds__(kBlock) void k_tile_lists(int64_t n_tiles, const in
         }
         if (lane >= ne && lane < kTileElems) ents[(t * kTileRows + i) * kTileElems + lane] = make_int2(0, 0);
     }
-    if (lane >= kTileRows && lane < kTileCols) cols[t * (kTileCols - kTileRows) + lane - kTileRows] = held;
+    over |= m > kTileCols;
+    if (lane >= kTileRows && lane < kTileCols)
+        cols[t * (kTileCols - kTileRows) + lane - kTileRows] = over && lane == kTileCols - 1 ? kTileOver : held;
 }
 
 }  // namespace
@@ -165,5 +175,23 @@ extern "C" int cvfes_tile_lists(void *stream, int64_t n_tiles, const int32_t *ro
                        static_cast<hipStream_t>(stream), n_tiles, rows, nptr,
                        reinterpret_cast<const fan_t *>(fan), reinterpret_cast<int4 *>(head), cols,
                        reinterpret_cast<int2 *>(ents));
-    return check_launch("k_tile_lists");
+    if (int rc = check_launch("k_tile_lists")) return rc;
+    // a tile that does not fit is refused here: its rows would read another node's column
+    const int64_t halo = kTileCols - kTileRows;
+    std::vector<int32_t> held;
+    try {
+        held.resize(n_tiles * halo);
+    } catch (...) {
+        return fail(CVFES_ERR_ARG, "cvfes_tile_lists: out of host memory");
+    }
+    hipError_t err = hipMemcpyAsync(held.data(), cols, sizeof(int32_t) * held.size(), hipMemcpyDeviceToHost,
+                                    static_cast<hipStream_t>(stream));
+    if (err == hipSuccess) err = hipStreamSynchronize(static_cast<hipStream_t>(stream));
+    if (err != hipSuccess) return fail(CVFES_ERR_HIP, "cvfes_tile_lists: %s", hipGetErrorString(err));
+    for (int64_t t = 0; t < n_tiles; ++t)
+        CVFES_REQUIRE(held[(t + 1) * halo - 1] != kTileOver,
+                      "cvfes_tile_lists: the rows of tile %lld name more than %lld halo columns or a node of more than "
+                      "%d elements",
+                      static_cast<long long>(t), static_cast<long long>(halo), kTileElems);
+    return CVFES_OK;
 }

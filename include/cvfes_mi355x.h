@@ -205,7 +205,8 @@ int cvfes_node_fans(void *stream, int64_t n_nodes, int64_t max_node_elems, const
 
 /*
  * Node tiles: compact groups of at most CVFES_TILE_ROWS nodes whose block rows have at most
- * CVFES_TILE_COLS distinct columns together, by recursive bisection of the node cloud.  Host only
+ * CVFES_TILE_COLS - CVFES_TILE_ROWS columns outside the group, by recursive bisection of the node
+ * cloud.  Host only
  * (host arrays): nodes [N][3], the block structure indptr/indices; rows [cap][CVFES_TILE_ROWS]
  * receives the node ids of each tile, -1 padded.  Returns the number of tiles (at most N), or a
  * negative code.  No counterpart in the reference.
@@ -215,7 +216,9 @@ int64_t cvfes_tile_rows(int64_t n_nodes, const double *nodes, const int32_t *ind
 
 /*
  * The lists of the tile kernels (cvfes_system_t.tile_head, tile_cols, tile_ents; device arrays,
- * 16-byte aligned) from the tiles' rows and the fan entries.  No counterpart in the reference.
+ * 16-byte aligned) from the tiles' rows and the fan entries.  Blocks until they are written, and
+ * fails where the rows of a tile have more halo columns (columns that are not themselves rows of the
+ * tile) than its slots.  No counterpart in the reference.
  */
 int cvfes_tile_lists(void *stream, int64_t n_tiles, const int32_t *rows, const int32_t *nptr,
                      const int32_t *fan, int64_t max_node_elems, int32_t *head, int32_t *cols,

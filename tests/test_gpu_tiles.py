@@ -182,3 +182,76 @@ def test_batched_tiles_and_rows_in_one_ensemble(require_gpu):
     for o in outs[1:]:
         for a, b in zip(outs[0], o):
             assert np.all(np.isfinite(a)) and np.array_equal(a, b)
+
+
+def free_nodes(nodes, el, bdy, share, seed=0):
+    """The wall with `share` of its node count in nodes of no element, scattered among its own."""
+    rng = np.random.default_rng(seed)
+    n = int(round(share * nodes.shape[0]))
+    lo, hi = nodes.min(0), nodes.max(0)
+    near = nodes[rng.integers(nodes.shape[0], size=n)] + 0.02 * (hi - lo) * rng.standard_normal((n, 3))
+    every = np.vstack([nodes, near])
+    place = rng.permutation(every.shape[0])            # node i of the wall becomes place[i]
+    out = np.empty_like(every)
+    out[place] = every
+    return out, place[el], place[bdy]
+
+
+def walls_with_free_nodes(kind, share):
+    if kind == "large":
+        return free_nodes(*tube_geometry(64, 32, 0.3, 2.0), share)
+    if kind == "two":                                  # one wall inside the other, a spacing apart
+        a, ea, ba = tube_geometry(40, 24, 0.30, 2.0)
+        b, eb, bb = tube_geometry(40, 24, 0.33, 2.0)
+        return free_nodes(np.vstack([a, b]), np.vstack([ea, eb + a.shape[0]]), np.concatenate([ba, bb + a.shape[0]]), share)
+    return free_nodes(*wall(kind), share)
+
+
+@pytest.mark.parametrize("kind", ["tube", "grid", "large", "two"])
+@pytest.mark.parametrize("share", [0.05, 0.2, 0.5, 1.0])
+def test_tiles_hold_their_halo_among_free_nodes(kind, share):
+    """Nodes of no element have empty block rows: they take a row slot of a tile and no column."""
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libcvfes_mi355x.so not built")
+    nodes, el, _ = walls_with_free_nodes(kind, share)
+    rows, ip, ix = tile_rows(nodes, el)
+    assert np.array_equal(np.sort(rows[rows >= 0]), np.arange(nodes.shape[0]))
+    for r in rows:
+        own = r[r >= 0]
+        cols = np.unique(np.concatenate([ix[ip[a]:ip[a + 1]] for a in own] + [own]))
+        assert len(cols) - len(own) <= _lib.TILE_COLS - _lib.TILE_ROWS
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,share,S", [("two", 0.2, 33), ("large", 0.05, 16), ("two", 1.0, 5)])
+def test_tile_kernels_among_free_nodes(require_gpu, kind, share, S):
+    from cvfes_amd.system import MembraneSystem
+    nodes, el, bdy = walls_with_free_nodes(kind, share)
+    n, dt, beta, damp = nodes.shape[0], 1e-6, 1e-7, 5.0
+    E = 7e6 * np.exp(0.1 * np.random.default_rng(S).standard_normal((el.shape[0], S)))
+    s = MembraneSystem(nodes, el, bdy, S, vthickness=np.full(n, 0.07), elmE=E, density=1.0, nu=0.45, store_values=False)
+    assert s.n_tiles > 0
+    u0 = 1e-4 * np.random.default_rng(S).standard_normal(3 * n)
+    u, mu, p = run(s, u0, dt, beta, damp)
+    tiles, s.n_tiles = s.n_tiles, 0
+    ur, mur, _ = run(s, u0, dt, beta, damp)
+    s.n_tiles = tiles
+    assert np.array_equal(u, ur) and np.array_equal(mu, mur)
+    ref = oracle_run(nodes, el, bdy, s, u0, p, dt, beta, damp)
+    used = np.repeat(np.isin(np.arange(n), el), 3)     # a node of no element has no mass: 0 / 0 in the oracle
+    assert np.max(np.abs(u.reshape(-1, S) - ref)[used]) < 1e-10 * np.max(np.abs(ref[used]))
+
+
+@pytest.mark.gpu
+def test_lists_refuse_a_tile_that_does_not_fit(require_gpu):
+    import torch
+    nodes, el, bdy, s = build("tube", 2)
+    far = np.full((1, _lib.TILE_ROWS), -1, np.int32)
+    far[0, :4] = [40, 65, 90, 115]                     # four rows of six neighbours each, none in common
+    out = [torch.empty(k, dtype=torch.int32, device="cuda")
+           for k in (4 * _lib.TILE_ROWS, _lib.TILE_COLS - _lib.TILE_ROWS, 2 * _lib.TILE_ROWS * _lib.TILE_ELEMS)]
+    for take, good in ((3, True), (4, False)):
+        rows = torch.as_tensor(np.where(np.arange(_lib.TILE_ROWS) < take, far, -1).astype(np.int32)).cuda()
+        rc = s.lib.cvfes_tile_lists(s.stream, 1, rows.data_ptr(), s.nptr.data_ptr(), s.fan.data_ptr(),
+                                    s.max_node_elems, *[t.data_ptr() for t in out])
+        assert (rc == 0) == good
