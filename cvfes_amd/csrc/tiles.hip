@@ -11,22 +11,21 @@
 namespace cvfes {
 namespace {
 
-// Distinct columns of the block rows ids[0..n) that are not themselves among ids, at most `most + 1`
-// of them counted: the halo columns of a tile of these rows.  (A node of no element has an empty
-// row and is no column of it, so the halo is not the row's columns less n.)
-int count_halo(const int32_t *ids, int n, const int32_t *indptr, const int32_t *indices, int most) {
-    int32_t seen[kTileCols];
-    for (int i = 0; i < n; ++i) seen[i] = ids[i];
-    int m = n;
-    for (int i = 0; i < n; ++i)
+// Distinct columns of the block rows ids[0..n) that are not themselves among ids, counted row
+// by row up to `most`: the halo columns of a tile of these rows.  (A node of no element has an empty
+// row and is no column of it, so the halo is not the row's columns less n.)  `seen` [N] holds the
+// last stamp a node was counted under.
+int count_halo(const int32_t *ids, int n, const int32_t *indptr, const int32_t *indices, int most, int32_t *seen,
+               int32_t stamp) {
+    for (int i = 0; i < n; ++i) seen[ids[i]] = stamp;
+    int m = 0;
+    for (int i = 0; i < n && m <= most; ++i)
         for (int32_t p = indptr[ids[i]]; p < indptr[ids[i] + 1]; ++p) {
-            int j = 0;
-            while (j < m && seen[j] != indices[p]) ++j;
-            if (j < m) continue;
-            if (m - n == most) return most + 1;
-            seen[m++] = indices[p];
+            if (seen[indices[p]] == stamp) continue;
+            seen[indices[p]] = stamp;
+            ++m;
         }
-    return m - n;
+    return m;
 }
 
 // Halve the nodes across their longest extent, on a multiple of the tile size, until a part is a
@@ -45,6 +44,9 @@ int64_t bisect(const double *nodes, const int32_t *indptr, const int32_t *indice
                 if (d < std::numeric_limits<double>::infinity()) edge[k] += d;
             }
     for (double &d : edge) d = d > 0.0 ? 1.0 / d : 0.0;
+    std::vector<int32_t> seen(n_nodes, 0);
+    int32_t stamp = 0;                     // fewer than 2 N parts are counted, N < 2^30
+    std::vector<std::pair<double, int32_t>> keys(n_nodes);
     std::vector<std::pair<int64_t, int64_t>> todo{{0, n_nodes}};
     int64_t n_tiles = 0;
     while (!todo.empty()) {
@@ -53,7 +55,7 @@ int64_t bisect(const double *nodes, const int32_t *indptr, const int32_t *indice
         const int64_t n = b - a;
         const int halo = kTileCols - kTileRows;
         if (n == 1 || (n <= kTileRows &&
-                       count_halo(&ids[a], static_cast<int>(n), indptr, indices, halo) <= halo)) {
+                       count_halo(&ids[a], static_cast<int>(n), indptr, indices, halo, seen.data(), ++stamp) <= halo)) {
             if (n_tiles == cap) return -1;
             std::sort(ids.begin() + a, ids.begin() + b);
             for (int i = 0; i < kTileRows; ++i) rows[n_tiles * kTileRows + i] = i < n ? ids[a + i] : -1;
@@ -75,14 +77,13 @@ int64_t bisect(const double *nodes, const int32_t *indptr, const int32_t *indice
             if (edge[k] * (hi[k] - lo[k]) > edge[ax] * (hi[ax] - lo[ax])) ax = k;
         const int64_t whole = (n + kTileRows - 1) / kTileRows;
         const int64_t h = n > kTileRows ? whole / 2 * kTileRows : n / 2;
-        const auto key = [&](int32_t i) {                  // NaN last: a strict order for any input
-            const double x = nodes[3 * static_cast<int64_t>(i) + ax];
-            return x == x ? x : std::numeric_limits<double>::infinity();
-        };
-        std::nth_element(ids.begin() + a, ids.begin() + a + h, ids.begin() + b, [&](int32_t i, int32_t j) {
-            const double x = key(i), y = key(j);
-            return x != y ? x < y : i < j;
-        });
+        for (int64_t i = a; i < b; ++i) {
+            const double x = nodes[3 * static_cast<int64_t>(ids[i]) + ax];
+            // NaN last: a strict order for any input
+            keys[i] = {x == x ? x : std::numeric_limits<double>::infinity(), ids[i]};
+        }
+        std::nth_element(keys.begin() + a, keys.begin() + a + h, keys.begin() + b);
+        for (int64_t i = a; i < b; ++i) ids[i] = keys[i].second;
         todo.push_back({a + h, b});
         todo.push_back({a, a + h});
     }

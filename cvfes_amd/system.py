@@ -247,7 +247,8 @@ class MembraneSystem:
         lists on the device."""
         if self.tile_head is not None or self.fan is None or self.max_node_elems > _lib.TILE_ELEMS:
             return
-        if np.any(self._elems_h == np.roll(self._elems_h, 1, axis=1)):
+        e0, e1, e2 = self._elems_h.T
+        if np.any((e0 == e1) | (e1 == e2) | (e2 == e0)):
             return                      # an element that names a node twice: more blocks (a,a) than elements
         rows = np.empty((self.n_nodes, _lib.TILE_ROWS), np.int32)
         ip, ix = self.indptr_h.astype(np.int32), self.indices_h.astype(np.int32)
