@@ -352,12 +352,12 @@ __global__ __launch_bounds__(kBlock) void k_step_lds(StepArgs a, LdsArgs l, int6
 }
 
 // values[p][ij][s] = sum_c coef[celem[c]][s] * khat[c][ij].  The values written bound it (nine per
-// block and sample against a coefficient per contribution), so a lane holds two samples and stores
-// 16 bytes past L2: the step that follows reads more than L2 holds.  With wave-uniform rows the unit
+// block and sample against a coefficient per contribution), so a lane holds two samples (but see
+// assemble) and stores 16 bytes, past L2 where stream_blocks says so (NT).  With wave-uniform rows the unit
 // blocks of up to seven contributions, which lie next to each other, come in by one load of 63
 // lanes and are broadcast from its registers; scalar loads would miss their cache on every block.
 // 131,072 upper blocks x 128 samples (1.2 GB): 337 -> 230 us.
-template <bool UNIFORM, int VW>
+template <bool UNIFORM, int VW, bool NT>
 __global__ __launch_bounds__(kBlock) void k_assemble(int64_t nnzb, int64_t n_smp,
                                                       const int32_t *__restrict__ bmap,
                                                       const int32_t *__restrict__ cptr,
@@ -403,7 +403,10 @@ __global__ __launch_bounds__(kBlock) void k_assemble(int64_t nnzb, int64_t n_smp
     if (!active) return;
     double *out = values + p * 9 * n_smp + s;
 #pragma unroll
-    for (int ij = 0; ij < 9; ++ij) store_vec_nt<VW>(out + ij * n_smp, kv[ij]);
+    for (int ij = 0; ij < 9; ++ij) {
+        if constexpr (NT) store_vec_nt<VW>(out + ij * n_smp, kv[ij]);
+        else store_vec<VW>(out + ij * n_smp, kv[ij]);
+    }
 }
 
 // x[n][j][s] = u0[3n+j] + beta * du0[3n+j]  (tile a sample-independent vector over samples)
@@ -987,24 +990,48 @@ extern "C" int64_t cvfes_step_kernel(const cvfes_system_t *sys, int method) {
 
 namespace {
 
-template <int VW>
+template <int VW, bool NT>
 void assemble_vw(hipStream_t st, int64_t nnzb, int64_t S, const int32_t *bmap, const int32_t *cptr,
                  const int32_t *celem, const double *khat, const double *coef, double *values) {
     // padding the rows to whole wavefronts may not push the launch past 2^32 threads
     if (use_uniform<VW>(S) && nnzb < (int64_t(1) << 31) / lanes_per_row<true, VW>(S))
-        hipLaunchKernelGGL((k_assemble<true, VW>), dim3(grid_for(nnzb * lanes_per_row<true, VW>(S))), dim3(kBlock),
+        hipLaunchKernelGGL((k_assemble<true, VW, NT>), dim3(grid_for(nnzb * lanes_per_row<true, VW>(S))), dim3(kBlock),
                            0, st, nnzb, S, bmap, cptr, celem, khat, coef, values);
     else
-        hipLaunchKernelGGL((k_assemble<false, VW>), dim3(grid_for(nnzb * lanes_per_row<false, VW>(S))),
+        hipLaunchKernelGGL((k_assemble<false, VW, NT>), dim3(grid_for(nnzb * lanes_per_row<false, VW>(S))),
                            dim3(kBlock), 0, st, nnzb, S, bmap, cptr, celem, khat, coef, values);
 }
 
-// two samples per lane and 16-byte accesses where the count and both arrays allow it
+// Whether the blocks are stored past L2: where their rows of n_smp doubles cover 64-byte sectors and
+// the array is too large to wait in the Infinity Cache beside what the launch reads.  A store past L2
+// leaves as it is, so rows that start and end inside a sector leave in pieces, which only longer rows
+// and larger arrays can afford.  Past L2 / through it, 102,400 nodes: 2 samples 122 / 39 us, 6 (177 MB)
+// 167 / 112, 8 (236 MB) 103 / 131, 10 185 / 149, 16 127 / 195, 20 198 / 247, 33 364 / 541, 128 827 /
+// 862; 32,768 nodes: 20 samples (188 MB) 82 / 62, 24 (226 MB) 69 / 76; with a product behind them on
+// 16,384 nodes: 33 samples (156 MB) 106 / 86, 40 (188 MB) 125 / 130, 48 (226 MB) 141 / 152.
+bool stream_blocks(int64_t nnzb, int64_t S) {
+    const int64_t bytes = 72 * nnzb * S, mib = int64_t(1) << 20;
+    return S % 8 == 0 ? bytes >= 162 * mib : S >= 20 && bytes >= 190 * mib;
+}
+
+// Two samples per lane and 16-byte accesses where the count and both arrays allow it and a row is at
+// least a 64-byte sector: below, half as many lanes in flight take longer than their wider stores
+// save (102,400 nodes, 2 samples 101 us against 39 us with one per lane, 4 samples 76 against 54).
+// From 32 to 64 samples one per lane fills half or all of a wavefront with one block's row, and
+// stores that stay in the caches come out ahead (16,384 nodes: 32 samples 40 against 36 us, 64 of
+// 4,096 nodes 18.9 against 18.2).
 void assemble(hipStream_t st, int64_t nnzb, int64_t S, const int32_t *bmap, const int32_t *cptr,
               const int32_t *celem, const double *khat, const double *coef, double *values) {
     const uintptr_t any = reinterpret_cast<uintptr_t>(coef) | reinterpret_cast<uintptr_t>(values);
-    if (S % 2 == 0 && any % 16 == 0) assemble_vw<2>(st, nnzb, S, bmap, cptr, celem, khat, coef, values);
-    else assemble_vw<1>(st, nnzb, S, bmap, cptr, celem, khat, coef, values);
+    const bool nt = stream_blocks(nnzb, S);
+    const bool one = S % 2 != 0 || any % 16 != 0 || S < 8 || (!nt && S >= 32 && S <= 64);
+    if (one) {
+        if (nt) assemble_vw<1, true>(st, nnzb, S, bmap, cptr, celem, khat, coef, values);
+        else assemble_vw<1, false>(st, nnzb, S, bmap, cptr, celem, khat, coef, values);
+    } else {
+        if (nt) assemble_vw<2, true>(st, nnzb, S, bmap, cptr, celem, khat, coef, values);
+        else assemble_vw<2, false>(st, nnzb, S, bmap, cptr, celem, khat, coef, values);
+    }
 }
 
 }  // namespace

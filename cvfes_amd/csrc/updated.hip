@@ -328,9 +328,10 @@ __global__ __launch_bounds__(kBlock) void k_step_moved(StepArgs a, GeomArgs g, i
 //   sigma = E / (1 - nu^2) / n.n [ nu tr H (I - nn / n.n) + g (H + H^T) + (gk - g) (n (x) q + q (x) n) / n.n ]
 // whatever the in-plane axes are: one division where the frame took two square roots and seven.
 // GEO: 0 the reference geometry (the gradients are the same for a lane's samples), 1 X + u itself,
-// 2 X + ug.  The output is written once and read by no kernel: 16-byte stores past L2.
+// 2 X + ug.  The output is written once and read by no kernel, in 16-byte stores, past L2 (NT) where
+// stream_stress says so.
 // 131,840 elements x 100 samples (0.79 GB) on the reference geometry: 270 -> 155 us.
-template <bool UNIFORM, int GEO, int VW>
+template <bool UNIFORM, int GEO, int VW, bool NT>
 __global__ __launch_bounds__(kBlock) void k_element_stress(int64_t n_elms, int64_t S, GeomArgs g,
                                                            const double *__restrict__ u,
                                                            const double *__restrict__ ave_E,
@@ -395,18 +396,29 @@ __global__ __launch_bounds__(kBlock) void k_element_stress(int64_t n_elms, int64
     if (!active) return;
     double *out = stress + e * 5 * S + s;
 #pragma unroll
-    for (int k = 0; k < 5; ++k) store_vec_nt<VW>(out + k * S, o[k]);
+    for (int k = 0; k < 5; ++k) {
+        if constexpr (NT) store_vec_nt<VW>(out + k * S, o[k]);
+        else store_vec<VW>(out + k * S, o[k]);
+    }
 }
 
-template <int GEO, int VW>
+// Past L2 where the rows are whole 64-byte sectors (65,280 elements, 16 samples: 10.2 us past L2, 12.5
+// through it), or longer rows of an array that the Infinity Cache cannot hold beside the inputs: a store
+// past L2 of part of a sector leaves in pieces (204,288 elements: 4 samples 30 / 13 us, 20 51 / 41, 33
+// 99 / 136; 131,428: 33 samples, 174 MB, 63 / 73).
+bool stream_stress(int64_t n_elms, int64_t S) {
+    return S % 8 == 0 || (S >= 20 && 40 * n_elms * S >= (int64_t(162) << 20));
+}
+
+template <int GEO, int VW, bool NT>
 void launch_stress(hipStream_t st, int64_t n_elms, int64_t S, const GeomArgs &g, const double *u,
                    const double *ave_E, double *stress) {
     // padding the rows to whole wavefronts may not push the launch past 2^32 threads
     if (use_uniform<VW>(S) && n_elms < (int64_t(1) << 31) / lanes_per_row<true, VW>(S))
-        hipLaunchKernelGGL((k_element_stress<true, GEO, VW>), dim3(grid_for(n_elms * lanes_per_row<true, VW>(S))),
+        hipLaunchKernelGGL((k_element_stress<true, GEO, VW, NT>), dim3(grid_for(n_elms * lanes_per_row<true, VW>(S))),
                            dim3(kBlock), 0, st, n_elms, S, g, u, ave_E, stress);
     else
-        hipLaunchKernelGGL((k_element_stress<false, GEO, VW>), dim3(grid_for(n_elms * lanes_per_row<false, VW>(S))),
+        hipLaunchKernelGGL((k_element_stress<false, GEO, VW, NT>), dim3(grid_for(n_elms * lanes_per_row<false, VW>(S))),
                            dim3(kBlock), 0, st, n_elms, S, g, u, ave_E, stress);
 }
 
@@ -527,7 +539,9 @@ extern "C" int cvfes_element_stress(void *stream, int64_t n_elms, int64_t n_smp,
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int geom = !ug ? 0 : ug == u ? 1 : 2;
     auto launch = [&](auto geo_c, auto vw_c) {
-        launch_stress<decltype(geo_c)::value, decltype(vw_c)::value>(st, n_elms, n_smp, g, u, ave_E, stress);
+        constexpr int GEO = decltype(geo_c)::value, VW = decltype(vw_c)::value;
+        if (stream_stress(n_elms, n_smp)) launch_stress<GEO, VW, true>(st, n_elms, n_smp, g, u, ave_E, stress);
+        else launch_stress<GEO, VW, false>(st, n_elms, n_smp, g, u, ave_E, stress);
     };
     auto width = [&](auto geo_c) {
         if (n_smp % 2 == 0 && any % 16 == 0) launch(geo_c, std::integral_constant<int, 2>{});

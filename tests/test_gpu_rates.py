@@ -1,0 +1,62 @@
+"""Calls that a rule of a dispatch once sent to the slower of two kernels, timed against what they can
+be held to on the same card and in the same minute: a device copy of the bytes the call has to move,
+or the other kernel.  Best of several interleaved rounds, and limits that leave a wide margin to what
+was measured on either side."""
+import numpy as np
+import pytest
+import torch
+
+from cvfes_amd.mesh import tube_geometry
+
+pytestmark = pytest.mark.gpu
+
+
+def microseconds(calls, rounds=9, n=20):
+    """Best time of each call over interleaved rounds of n."""
+    best = [np.inf] * len(calls)
+    for c in calls:
+        c()
+    for _ in range(rounds):
+        for i, c in enumerate(calls):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(n):
+                c()
+            e1.record()
+            e1.synchronize()
+            best[i] = min(best[i], 1e3 * e0.elapsed_time(e1) / n)
+    return best
+
+
+def system(nt, nz, S, **kw):
+    from cvfes_amd.system import MembraneSystem
+    nodes, el, bdy = tube_geometry(nt, nz, 0.5, 6.0)
+    E = 7e6 * np.exp(0.1 * np.random.default_rng(S).standard_normal((el.shape[0], S)))
+    return MembraneSystem(nodes, el, bdy, S, vthickness=np.full(nodes.shape[0], 0.07), elmE=E, density=1.0, nu=0.45, **kw)
+
+
+def copy_of(n_bytes):
+    """A device copy that reads and writes n_bytes together."""
+    a = torch.zeros(int(n_bytes) // 16, dtype=torch.float64, device="cuda")
+    b = torch.empty_like(a)
+    return lambda: b.copy_(a)
+
+
+# Stores past L2 of rows of a few samples took 5.4 (blocks) and 2.3 times as long as stores through it.
+@pytest.mark.parametrize("S", [1, 2, 4])
+def test_assembly_of_few_samples(require_gpu, S):
+    s = system(256, 400, S)
+    moved = 72 * s.nnzu * S + 8 * s.coef.numel() + 8 * s.khat.numel()
+    t, copy = microseconds([s.assemble_upper, copy_of(moved)])
+    print(f"{S} samples: {t:.1f} us, copy {copy:.1f}")
+    assert t <= 2.5 * copy + 5.0
+
+
+@pytest.mark.parametrize("S", [2, 6])
+def test_stress_of_few_samples(require_gpu, S):
+    s = system(256, 400, S, store_values=False)
+    u = torch.zeros(s.state_shape(), dtype=torch.float64, device="cuda")
+    moved = 8 * (6 * s.n_elms * S + u.numel()) + 12 * s.n_elms
+    t, copy = microseconds([lambda: s.element_stress(u=u), copy_of(moved)])
+    print(f"{S} samples: {t:.1f} us, copy {copy:.1f}")
+    assert t <= 2.5 * copy + 5.0
