@@ -186,11 +186,16 @@ __device__ __forceinline__ void stored_block(const RA &k, int32_t p, int side, i
             for (int v = 0; v < VW; ++v) kv[ij][v] = t.v[v];
         }
     } else {
-        const auto *base = k.uvalues + (static_cast<int64_t>(k.vblk[p]) * 9) * k.n_smp + s;
+        // sym_entry as two offsets: the entries above the diagonal lie 2 or 4 rows further on where the
+        // block is read transposed, those below it as far back where it is or is the diagonal block.
+        // Chosen entry by entry, packed rows branch and wait for memory in both branches.
+        const int64_t n = k.n_smp, up = side < 0 ? 2 * n : 0, down = side > 0 ? 0 : 2 * n;
+        const auto *base = k.uvalues + (static_cast<int64_t>(k.vblk[p]) * 9) * n + s;
+        const int64_t at[9] = {0,     n + up,           2 * (n + up), 3 * n - down, 4 * n,
+                               5 * n + up, 2 * (3 * n - down), 7 * n - down, 8 * n};
 #pragma unroll
         for (int ij = 0; ij < 9; ++ij) {
-            const int src = side < 0 ? sym_entry(ij, -1) : (side == 0 ? sym_entry(ij, 0) : ij);
-            const Vec<VW> t = load_vec<VW>(base + src * k.n_smp);
+            const Vec<VW> t = load_vec<VW>(base + at[ij]);
 #pragma unroll
             for (int v = 0; v < VW; ++v) kv[ij][v] = t.v[v];
         }
@@ -202,12 +207,17 @@ __device__ __forceinline__ void stored_block(const RA &k, int32_t p, int side, i
 // acc += coef_e (khat_c x), so the block itself is never formed and only the three sums per
 // sample are live (khat_c is wave-uniform for wave-uniform rows: scalar loads).
 // `side`: the block's column less its row, for the symmetric storage (sym_entry).
-template <int OP, int VW, class RA>
+// PIN: all nine entries of a stored block in flight before the first is used; the compiler else waits
+// for them a few at a time in some kernels (16,384 rows of up to 13 blocks, 8 samples: 23.0 -> 13.4 us a
+// step with the other two forms of this walk, sym_entry's two offsets and the row's own state first;
+// the adjoint step of one sample per lane is scheduled well as it is: 11.9 us, pinned 12.9).
+template <int OP, int VW, bool PIN = VW == 2, class RA>
 __device__ __forceinline__ void block_apply(const RA &k, int32_t p, int side, int64_t s,
                                             const double (&x)[3][VW], double (&acc)[3][VW]) {
     if constexpr (OP != kOpMatfree) {
         double kv[9][VW];
         stored_block<OP == kOpSym, VW>(k, p, side, s, kv);
+        if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -572,7 +582,7 @@ __device__ __forceinline__ void row_product(const RA &k, DP u, DP up, double bdt
         const int64_t col = k.indices[p];
         double x[3][VW];
         state_column<BETA, VW>(u, up, bdt, col, k.n_smp, s, x);
-        block_apply<OP, VW>(k, p, static_cast<int>(col) - row, s, x, acc);
+        block_apply<OP, VW, true>(k, p, static_cast<int>(col) - row, s, x, acc);
     }
 }
 
@@ -665,17 +675,23 @@ __device__ __forceinline__ void step_update(const SA &a, int32_t row, int64_t s,
     }
 }
 
-// The same with the row's own state read here.
-template <bool DAMP, int VW, class SA>
-__device__ __forceinline__ void step_update(const SA &a, int32_t row, int64_t s, bool active,
-                                            int64_t step, const double (&acc)[3][VW]) {
-    Vec<VW> uu[3], pp[3];
+// The row's own state.
+template <int VW, class SA>
+__device__ __forceinline__ void own_state(const SA &a, int32_t row, int64_t s, Vec<VW> (&uu)[3], Vec<VW> (&pp)[3]) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         const int64_t off = (static_cast<int64_t>(row) * 3 + i) * a.k.n_smp + s;
         uu[i] = load_vec<VW>(a.u + off);
         pp[i] = load_vec<VW>(a.up + off);
     }
+}
+
+// The same with the row's own state read here.
+template <bool DAMP, int VW, class SA>
+__device__ __forceinline__ void step_update(const SA &a, int32_t row, int64_t s, bool active,
+                                            int64_t step, const double (&acc)[3][VW]) {
+    Vec<VW> uu[3], pp[3];
+    own_state<VW>(a, row, s, uu, pp);
     step_update<DAMP, VW>(a, row, s, active, step, row_load<VW>(a, row, s), acc, uu, pp);
 }
 
@@ -692,8 +708,19 @@ __device__ __forceinline__ void step_row(const SA &a, int32_t row, int64_t s, bo
         step_update<DAMP, VW>(a, row, s, active, step, acc[0]);
     } else {
         double acc[3][VW];
-        row_product<OP, BETA, VW>(a.k, a.u, a.up, a.bdt, row, s, acc);
-        step_update<DAMP, VW>(a, row, s, active, step, acc);
+        if constexpr (!UNI && (VW == 1 || !BETA)) {
+            // What the update reads is in flight during the product; with both states of two samples
+            // it would take the registers of a wave (8 samples: 14.6 -> 19.1 us).  102,400 rows, one
+            // sample: 27.2 -> 18.9 us a step, two 42.7 -> 33.8.
+            Vec<VW> uu[3], pp[3];
+            own_state<VW>(a, row, s, uu, pp);
+            const RowLoad<VW> r = row_load<VW>(a, row, s);
+            row_product<OP, BETA, VW>(a.k, a.u, a.up, a.bdt, row, s, acc);
+            step_update<DAMP, VW>(a, row, s, active, step, r, acc, uu, pp);
+        } else {
+            row_product<OP, BETA, VW>(a.k, a.u, a.up, a.bdt, row, s, acc);
+            step_update<DAMP, VW>(a, row, s, active, step, acc);
+        }
     }
 }
 
