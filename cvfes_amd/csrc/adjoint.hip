@@ -247,16 +247,16 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_step(AdjArgs a) {
 
 // The adjoint step on the symmetric storage with row records (sym_product; the bits are those of
 // k_adjoint_step<kOpSym>).
-template <bool UNIFORM, bool BETA, bool DAMP, int VW, int MAXB>
+template <bool UNIFORM, bool BETA, bool DAMP, int VW>
 __global__ __launch_bounds__(kBlock) void k_adjoint_symrec(AdjArgs a, const int32_t *__restrict__ rec) {
     int32_t row;
     int64_t s;
     bool active;
     if (!row_and_sample<UNIFORM, VW>(a.k.n_nodes, a.k.n_smp, row, s, active)) return;
-    const int32_t *r = rec + static_cast<int64_t>(row) * (2 + 2 * MAXB);
+    const int32_t *r = rec + static_cast<int64_t>(row) * (2 + 2 * kRecordSlots);
     row = r[0];
     double acc[1][3][VW];
-    sym_product<UNIFORM, VW, MAXB>(a.k, r, AdjCol<UNIFORM, BETA, VW>{a, static_cast<uint32_t>(s) * 8u}, row, acc);
+    sym_product<UNIFORM, VW>(a.k, r, AdjCol<UNIFORM, BETA, VW>{a, static_cast<uint32_t>(s) * 8u}, row, acc);
     adj_finish<DAMP, VW>(a, row, s, active, acc[0]);
 }
 
@@ -318,19 +318,19 @@ __global__ __launch_bounds__(kBlock) void k_fused_step(StepArgs f, AdjArgs a, in
 
 // The fused step on the symmetric storage with row records (the bits are those of
 // k_fused_step<kOpSym>).
-template <bool UNIFORM, bool BETA, bool DAMP, int VW, int MAXB>
+template <bool UNIFORM, bool BETA, bool DAMP, int VW>
 __global__ __launch_bounds__(kBlock) void k_fused_symrec(StepArgs f, AdjArgs a, const int32_t *__restrict__ rec,
                                                         int64_t step) {
     int32_t row;
     int64_t s;
     bool active;
     if (!row_and_sample<UNIFORM, VW>(f.k.n_nodes, f.k.n_smp, row, s, active)) return;
-    const int32_t *r = rec + static_cast<int64_t>(row) * (2 + 2 * MAXB);
+    const int32_t *r = rec + static_cast<int64_t>(row) * (2 + 2 * kRecordSlots);
     row = r[0];
     const uint32_t lane = static_cast<uint32_t>(s) * 8u;
     const FusedCol<UNIFORM, BETA, VW> col{{f.u, f.up, f.bdt, f.k.n_smp, lane}, {a, lane}, lane};
     double acc[2][3][VW];
-    sym_product<UNIFORM, VW, MAXB>(f.k, r, col, row, acc);
+    sym_product<UNIFORM, VW>(f.k, r, col, row, acc);
     step_update<DAMP, VW>(f, row, s, active, step, acc[0]);
     adj_finish<DAMP, VW>(a, row, s, active, acc[1]);
 }
@@ -581,42 +581,49 @@ void adj_dispatch(hipStream_t st, const AdjArgs &a, bool beta, bool damp) {
     }
 }
 
-template <bool UNI, int VW, int MAXB>
+template <bool UNI, int VW>
 void adj_symrec_launch(hipStream_t st, const AdjArgs &a, const int32_t *rec, bool beta, bool damp) {
     const dim3 g(grid_for(a.k.n_nodes * lanes_per_row<UNI, VW>(a.k.n_smp))), b(kBlock);
     if (beta) {
-        if (damp) hipLaunchKernelGGL((k_adjoint_symrec<UNI, true, true, VW, MAXB>), g, b, a.occ_lds, st, a, rec);
-        else hipLaunchKernelGGL((k_adjoint_symrec<UNI, true, false, VW, MAXB>), g, b, a.occ_lds, st, a, rec);
+        if (damp) hipLaunchKernelGGL((k_adjoint_symrec<UNI, true, true, VW>), g, b, a.occ_lds, st, a, rec);
+        else hipLaunchKernelGGL((k_adjoint_symrec<UNI, true, false, VW>), g, b, a.occ_lds, st, a, rec);
     } else {
-        if (damp) hipLaunchKernelGGL((k_adjoint_symrec<UNI, false, true, VW, MAXB>), g, b, a.occ_lds, st, a, rec);
-        else hipLaunchKernelGGL((k_adjoint_symrec<UNI, false, false, VW, MAXB>), g, b, a.occ_lds, st, a, rec);
+        if (damp) hipLaunchKernelGGL((k_adjoint_symrec<UNI, false, true, VW>), g, b, a.occ_lds, st, a, rec);
+        else hipLaunchKernelGGL((k_adjoint_symrec<UNI, false, false, VW>), g, b, a.occ_lds, st, a, rec);
     }
 }
 
-template <bool UNI, int VW, int MAXB>
+template <bool UNI, int VW>
 void fused_symrec_launch(hipStream_t st, const StepArgs &f, const AdjArgs &a, const int32_t *rec, bool beta,
                          bool damp) {
     const dim3 g(grid_for(f.k.n_nodes * lanes_per_row<UNI, VW>(f.k.n_smp))), b(kBlock);
     const int64_t step = 0;
     if (beta) {
-        if (damp) hipLaunchKernelGGL((k_fused_symrec<UNI, true, true, VW, MAXB>), g, b, f.occ_lds, st, f, a, rec, step);
-        else hipLaunchKernelGGL((k_fused_symrec<UNI, true, false, VW, MAXB>), g, b, f.occ_lds, st, f, a, rec, step);
+        if (damp) hipLaunchKernelGGL((k_fused_symrec<UNI, true, true, VW>), g, b, f.occ_lds, st, f, a, rec, step);
+        else hipLaunchKernelGGL((k_fused_symrec<UNI, true, false, VW>), g, b, f.occ_lds, st, f, a, rec, step);
     } else {
-        if (damp) hipLaunchKernelGGL((k_fused_symrec<UNI, false, true, VW, MAXB>), g, b, f.occ_lds, st, f, a, rec, step);
-        else hipLaunchKernelGGL((k_fused_symrec<UNI, false, false, VW, MAXB>), g, b, f.occ_lds, st, f, a, rec, step);
+        if (damp) hipLaunchKernelGGL((k_fused_symrec<UNI, false, true, VW>), g, b, f.occ_lds, st, f, a, rec, step);
+        else hipLaunchKernelGGL((k_fused_symrec<UNI, false, false, VW>), g, b, f.occ_lds, st, f, a, rec, step);
     }
 }
 
-// The adjoint step alone (f null) or fused with the forward step f, by row records of MAXB slots.
-template <int MAXB>
-void symrec_dispatch(hipStream_t st, const StepArgs *f, const AdjArgs &a, const int32_t *rec, bool beta, bool damp) {
+// The adjoint step by row records, for the sample counts that use_records leaves it.
+void adj_symrec(hipStream_t st, const AdjArgs &a, const int32_t *rec, bool beta, bool damp) {
+    const int64_t S = a.k.n_smp;
+    if (generic_vw(S) == 1) adj_symrec_launch<false, 1>(st, a, rec, beta, damp);
+    else if (use_uniform<2>(S)) adj_symrec_launch<true, 2>(st, a, rec, beta, damp);
+    else adj_symrec_launch<false, 2>(st, a, rec, beta, damp);
+}
+
+// The same fused with the forward step f.
+void fused_symrec(hipStream_t st, const StepArgs &f, const AdjArgs &a, const int32_t *rec, bool beta, bool damp) {
     const int64_t S = a.k.n_smp;
     if (generic_vw(S) == 2) {
-        if (use_uniform<2>(S)) f ? fused_symrec_launch<true, 2, MAXB>(st, *f, a, rec, beta, damp) : adj_symrec_launch<true, 2, MAXB>(st, a, rec, beta, damp);
-        else f ? fused_symrec_launch<false, 2, MAXB>(st, *f, a, rec, beta, damp) : adj_symrec_launch<false, 2, MAXB>(st, a, rec, beta, damp);
+        if (use_uniform<2>(S)) fused_symrec_launch<true, 2>(st, f, a, rec, beta, damp);
+        else fused_symrec_launch<false, 2>(st, f, a, rec, beta, damp);
     } else {
-        if (use_uniform<1>(S)) f ? fused_symrec_launch<true, 1, MAXB>(st, *f, a, rec, beta, damp) : adj_symrec_launch<true, 1, MAXB>(st, a, rec, beta, damp);
-        else f ? fused_symrec_launch<false, 1, MAXB>(st, *f, a, rec, beta, damp) : adj_symrec_launch<false, 1, MAXB>(st, a, rec, beta, damp);
+        if (use_uniform<1>(S)) fused_symrec_launch<true, 1>(st, f, a, rec, beta, damp);
+        else fused_symrec_launch<false, 1>(st, f, a, rec, beta, damp);
     }
 }
 
@@ -720,11 +727,8 @@ extern "C" int cvfes_adjoint_step(void *stream, const cvfes_system_t *sys, int m
     case kOpMatfree: adj_dispatch<kOpMatfree>(st, a, beta != 0.0, damp != 0.0); break;
     case kOpStored: adj_dispatch<kOpStored>(st, a, beta != 0.0, damp != 0.0); break;
     default:
-        switch (record_slots(sys)) {
-        case 7: symrec_dispatch<7>(st, nullptr, a, sys->row_records, beta != 0.0, damp != 0.0); break;
-        case 10: symrec_dispatch<10>(st, nullptr, a, sys->row_records, beta != 0.0, damp != 0.0); break;
-        default: adj_dispatch<kOpSym>(st, a, beta != 0.0, damp != 0.0); break;
-        }
+        if (use_records(sys, true)) adj_symrec(st, a, sys->row_records, beta != 0.0, damp != 0.0);
+        else adj_dispatch<kOpSym>(st, a, beta != 0.0, damp != 0.0);
         break;
     }
     return check_launch("k_adjoint_step");
@@ -777,11 +781,8 @@ extern "C" int cvfes_adjoint_fused_step(void *stream, const cvfes_system_t *sys,
     case kOpMatfree: fused_dispatch<kOpMatfree>(st, f, a, beta != 0.0, damp != 0.0); break;
     case kOpStored: fused_dispatch<kOpStored>(st, f, a, beta != 0.0, damp != 0.0); break;
     default:
-        switch (record_slots(sys)) {
-        case 7: symrec_dispatch<7>(st, &f, a, sys->row_records, beta != 0.0, damp != 0.0); break;
-        case 10: symrec_dispatch<10>(st, &f, a, sys->row_records, beta != 0.0, damp != 0.0); break;
-        default: fused_dispatch<kOpSym>(st, f, a, beta != 0.0, damp != 0.0); break;
-        }
+        if (use_records(sys)) fused_symrec(st, f, a, sys->row_records, beta != 0.0, damp != 0.0);
+        else fused_dispatch<kOpSym>(st, f, a, beta != 0.0, damp != 0.0);
         break;
     }
     return check_launch("k_fused_step");

@@ -53,18 +53,18 @@ __global__ __launch_bounds__(kBlock) void k_spmv(StepArgs a) {
 
 // The product with the symmetric storage by row records (sym_product; the bits of k_spmv<kOpSym>).
 // 33,024 rows x 128 samples (1.3 GB of blocks and states): 316 -> 267 us.
-template <bool UNIFORM, int VW, int MAXB>
+template <bool UNIFORM, int VW>
 __global__ __launch_bounds__(kBlock) void k_spmv_symrec(StepArgs a, const int32_t *__restrict__ rec) {
     int32_t row;
     int64_t s;
     bool active;
     if (!row_and_sample<UNIFORM, VW>(a.k.n_nodes, a.k.n_smp, row, s, active)) return;
-    const int32_t *r = rec + static_cast<int64_t>(row) * (2 + 2 * MAXB);
+    const int32_t *r = rec + static_cast<int64_t>(row) * (2 + 2 * kRecordSlots);
     row = r[0];
     typedef StateCol<UNIFORM, false, VW, const double *> Col;
     const Col col{a.u, nullptr, 0.0, a.k.n_smp, static_cast<uint32_t>(s) * 8u};
     double acc[1][3][VW];
-    sym_product<UNIFORM, VW, MAXB>(a.k, r, col, row, acc);
+    sym_product<UNIFORM, VW>(a.k, r, col, row, acc);
     if (!active) return;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -312,18 +312,18 @@ __global__ __launch_bounds__(kBlock) void k_step_sym(StepArgs a, const double *_
 
 // The generic step on the symmetric storage with row records, for any sample count (sym_product; the
 // bits are those of k_step<kOpSym>).
-template <bool UNIFORM, bool BETA, bool DAMP, int VW, int MAXB>
+template <bool UNIFORM, bool BETA, bool DAMP, int VW>
 __global__ __launch_bounds__(kBlock) void k_step_symrec(StepArgs a, const int32_t *__restrict__ rec, int64_t step) {
     int32_t row;
     int64_t s;
     bool active;
     if (!row_and_sample<UNIFORM, VW>(a.k.n_nodes, a.k.n_smp, row, s, active)) return;
-    const int32_t *r = rec + static_cast<int64_t>(row) * (2 + 2 * MAXB);
+    const int32_t *r = rec + static_cast<int64_t>(row) * (2 + 2 * kRecordSlots);
     row = r[0];
     typedef StateCol<UNIFORM, BETA, VW, const double *> Col;
     const Col col{a.u, a.up, a.bdt, a.k.n_smp, static_cast<uint32_t>(s) * 8u};
     double acc[1][3][VW];
-    sym_product<UNIFORM, VW, MAXB>(a.k, r, col, row, acc);
+    sym_product<UNIFORM, VW>(a.k, r, col, row, acc);
     step_update<DAMP, VW>(a, row, s, active, step, acc[0]);
 }
 
@@ -494,13 +494,12 @@ void spmv_op(hipStream_t st, const StepArgs &a) {
 }
 
 // The product by row records, lane width and row mapping as spmv_op.
-template <int MAXB>
 void spmv_symrec(hipStream_t st, const StepArgs &a, const int32_t *rec) {
     const int64_t S = a.k.n_smp;
     auto launch = [&](auto uni, auto vw) {
         constexpr bool UNI = decltype(uni)::value;
         constexpr int VW = decltype(vw)::value;
-        hipLaunchKernelGGL((k_spmv_symrec<UNI, VW, MAXB>), dim3(grid_for(a.k.n_nodes * lanes_per_row<UNI, VW>(S))),
+        hipLaunchKernelGGL((k_spmv_symrec<UNI, VW>), dim3(grid_for(a.k.n_nodes * lanes_per_row<UNI, VW>(S))),
                            dim3(kBlock), a.occ_lds, st, a, rec);
     };
     typedef std::integral_constant<int, 1> one;
@@ -522,11 +521,8 @@ void spmv_dispatch(hipStream_t st, const cvfes_system_t *sys, bool mf, const Ste
     case kOpMatfree: spmv_op<kOpMatfree>(st, a); break;
     case kOpStored: spmv_op<kOpStored>(st, a); break;
     default:
-        switch (record_slots(sys)) {
-        case 7: spmv_symrec<7>(st, a, sys->row_records); break;
-        case 10: spmv_symrec<10>(st, a, sys->row_records); break;
-        default: spmv_op<kOpSym>(st, a); break;
-        }
+        if (use_records(sys)) spmv_symrec(st, a, sys->row_records);
+        else spmv_op<kOpSym>(st, a);
         break;
     }
 }
@@ -664,27 +660,26 @@ void launch_sym(hipStream_t st, const cvfes_system_t *sys, const StepArgs &a, in
         launch_sym_rec<NT, MAXB, false>(st, sys, a, step, beta, damp);
 }
 
-template <bool UNI, int VW, int MAXB>
+template <bool UNI, int VW>
 void launch_symrec(hipStream_t st, const StepArgs &a, const int32_t *rec, int64_t step, bool beta, bool damp) {
     const dim3 g(grid_for(a.k.n_nodes * lanes_per_row<UNI, VW>(a.k.n_smp))), b(kBlock);
     if (beta) {
-        if (damp) hipLaunchKernelGGL((k_step_symrec<UNI, true, true, VW, MAXB>), g, b, a.occ_lds, st, a, rec, step);
-        else hipLaunchKernelGGL((k_step_symrec<UNI, true, false, VW, MAXB>), g, b, a.occ_lds, st, a, rec, step);
+        if (damp) hipLaunchKernelGGL((k_step_symrec<UNI, true, true, VW>), g, b, a.occ_lds, st, a, rec, step);
+        else hipLaunchKernelGGL((k_step_symrec<UNI, true, false, VW>), g, b, a.occ_lds, st, a, rec, step);
     } else {
-        if (damp) hipLaunchKernelGGL((k_step_symrec<UNI, false, true, VW, MAXB>), g, b, a.occ_lds, st, a, rec, step);
-        else hipLaunchKernelGGL((k_step_symrec<UNI, false, false, VW, MAXB>), g, b, a.occ_lds, st, a, rec, step);
+        if (damp) hipLaunchKernelGGL((k_step_symrec<UNI, false, true, VW>), g, b, a.occ_lds, st, a, rec, step);
+        else hipLaunchKernelGGL((k_step_symrec<UNI, false, false, VW>), g, b, a.occ_lds, st, a, rec, step);
     }
 }
 
-template <int MAXB>
 void step_symrec(hipStream_t st, const StepArgs &a, const int32_t *rec, int64_t step, bool beta, bool damp) {
     const int64_t S = a.k.n_smp;
     if (generic_vw(S) == 2) {
-        if (use_uniform<2>(S)) launch_symrec<true, 2, MAXB>(st, a, rec, step, beta, damp);
-        else launch_symrec<false, 2, MAXB>(st, a, rec, step, beta, damp);
+        if (use_uniform<2>(S)) launch_symrec<true, 2>(st, a, rec, step, beta, damp);
+        else launch_symrec<false, 2>(st, a, rec, step, beta, damp);
     } else {
-        if (use_uniform<1>(S)) launch_symrec<true, 1, MAXB>(st, a, rec, step, beta, damp);
-        else launch_symrec<false, 1, MAXB>(st, a, rec, step, beta, damp);
+        if (use_uniform<1>(S)) launch_symrec<true, 1>(st, a, rec, step, beta, damp);
+        else launch_symrec<false, 1>(st, a, rec, step, beta, damp);
     }
 }
 
@@ -968,11 +963,8 @@ void step_dispatch(hipStream_t st, const cvfes_system_t *sys, bool mf, const Ste
     case kOpMatfree: step_generic<kOpMatfree>(st, a, step, beta, damp); break;
     case kOpStored: step_generic<kOpStored>(st, a, step, beta, damp); break;
     default:
-        switch (record_slots(sys)) {
-        case 7: step_symrec<7>(st, a, sys->row_records, step, beta, damp); break;
-        case 10: step_symrec<10>(st, a, sys->row_records, step, beta, damp); break;
-        default: step_generic<kOpSym>(st, a, step, beta, damp); break;
-        }
+        if (use_records(sys)) step_symrec(st, a, sys->row_records, step, beta, damp);
+        else step_generic<kOpSym>(st, a, step, beta, damp);
         break;
     }
 }

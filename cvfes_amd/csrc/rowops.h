@@ -87,13 +87,22 @@ inline const fan_t *fan_entries(const cvfes_system_t *sys) {
     return sys->nptr && sys->n_smp < (int64_t(1) << 31) / 24 ? reinterpret_cast<const fan_t *>(sys->fan) : nullptr;
 }
 
-// Block slots of the system's row records if the kernels that read the symmetric storage by them
-// apply, else 0 (byte offsets inside a block are 32-bit: 72 S).
-inline int record_slots(const cvfes_system_t *sys) {
-    if (!sys->row_records || !sys->uvalues || 72 * sys->n_smp > INT32_MAX) return 0;
-    for (int maxb : {7, 10})
-        if (sys->record_width == 2 + 2 * maxb && sys->max_row_blocks >= 1 && sys->max_row_blocks <= maxb) return maxb;
-    return 0;
+constexpr int kRecordSlots = 7;
+
+// Whether the kernels that read a row's structure from its record (seven block slots) take the symmetric
+// storage; the others walk indptr, indices and vblk.  Byte offsets inside a block are 32-bit: 72 S.
+// Records of ten slots, those of irregular walls, serve k_step_sym alone: slots behind a row's last
+// block repeat it, a third more loads than the rows' seven or so blocks need (16,384 rows of 4 to 8
+// elements, walk / records: 64 samples 80 / 93 us a step, 8 12.0 / 13.5; 102,400 rows, 2 samples: product
+// 32 / 45 us, 33 287 / 331; few gained, 16,384 rows, 40 samples: 55 / 49).  Adjoint: the adjoint step with
+// one sample per lane loses by records in wave-uniform rows (16,384 nodes of a regular wall, 48 samples:
+// 66 / 76 us) and with one sample in all (102,400 nodes: 20.2 / 22.2).
+inline bool use_records(const cvfes_system_t *sys, bool adjoint = false) {
+    const int64_t S = sys->n_smp;
+    if (!sys->row_records || !sys->uvalues || 72 * S > INT32_MAX || sys->record_width != 2 + 2 * kRecordSlots ||
+        sys->max_row_blocks < 1 || sys->max_row_blocks > kRecordSlots)
+        return false;
+    return !adjoint || (S > 1 && (generic_vw(S) == 2 || !use_uniform<1>(S)));
 }
 
 // Node tiles (tile.h): rows per tile, column slots (39 of 64 samples and the unit blocks of 16
@@ -513,7 +522,7 @@ __device__ __forceinline__ void fan_product(const RA &k, const COL &col, int32_t
 // block in the same order, with the next block's loads issued before the current one is applied.  The walk over
 // indptr, indices and vblk puts two dependent loads in front of every block's values.  Slots behind
 // the row's last block repeat it and are not added.
-template <bool UNI, int VW, int MAXB, class COL>
+template <bool UNI, int VW, class COL>
 __device__ __forceinline__ void sym_product(const RowArgs &k, const int32_t *r, const COL &col, int32_t row,
                                             double (&acc)[COL::kCols][3][VW]) {
     constexpr int NC = COL::kCols;
@@ -535,7 +544,7 @@ __device__ __forceinline__ void sym_product(const RowArgs &k, const int32_t *r, 
     auto issue = [&](int b) {
         const int32_t node = r[2 + b];
         const int side = node - row;
-        const double *base = k.uvalues + static_cast<int64_t>(r[2 + MAXB + b]) * 9 * S;
+        const double *base = k.uvalues + static_cast<int64_t>(r[2 + kRecordSlots + b]) * 9 * S;
         x[b % D] = col.load(node);
 #pragma unroll
         for (int ij = 0; ij < 9; ++ij) {
@@ -547,8 +556,8 @@ __device__ __forceinline__ void sym_product(const RowArgs &k, const int32_t *r, 
 #pragma unroll
     for (int b = 0; b < D - 1; ++b) issue(b);
 #pragma unroll
-    for (int b = 0; b < MAXB; ++b) {
-        if (b + D - 1 < MAXB) issue(b + D - 1);
+    for (int b = 0; b < kRecordSlots; ++b) {
+        if (b + D - 1 < kRecordSlots) issue(b + D - 1);
         __builtin_amdgcn_sched_barrier(0);
         double xv[NC][3][VW];
         col.value(x[b % D], xv);
