@@ -283,7 +283,7 @@ void k_adjoint_tile(AdjArgs a, TileArgs t) {
 // bit.  The forward and the adjoint may be at different time steps (the reverse sweep of one
 // checkpoint segment runs with the recomputation of the segment before it).  (A register target
 // of 5 waves per SIMD, 94 VGPRs instead of 100 for the stored two-sample instance, measured 2-3 %
-// slower: the loads in flight per wave count for more here.)
+// slower: the loads in flight per wave count for more here.)  By fan entries see fan_as_two.
 template <int OP, bool UNIFORM, bool BETA, bool DAMP, int VW>
 __global__ __launch_bounds__(kBlock) void k_fused_step(StepArgs f, AdjArgs a, int64_t step) {
     int32_t row;
@@ -642,12 +642,25 @@ void fused_launch(hipStream_t st, const StepArgs &f, const AdjArgs &a, bool beta
 template <int MF>
 void fused_dispatch(hipStream_t st, const StepArgs &f, const AdjArgs &a, bool beta, bool damp) {
     if (generic_vw(f.k.n_smp) == 2) {
-        if (use_uniform<2>(f.k.n_smp)) fused_launch<MF, true, 2>(st, f, a, beta, damp);
-        else fused_launch<MF, false, 2>(st, f, a, beta, damp);
+        if constexpr (MF != kOpFan)         // fan_as_two
+            if (use_uniform<2>(f.k.n_smp)) return fused_launch<MF, true, 2>(st, f, a, beta, damp);
+        fused_launch<MF, false, 2>(st, f, a, beta, damp);
     } else {
         if (use_uniform<1>(f.k.n_smp)) fused_launch<MF, true, 1>(st, f, a, beta, damp);
         else fused_launch<MF, false, 1>(st, f, a, beta, damp);
     }
+}
+
+// Whether the fused matrix-free step runs as its two launches: with both columns of two samples the
+// fan walk holds the registers of two waves per SIMD, and reading the coefficients once saves less
+// than that costs (16,384 nodes of a regular / irregular wall, fused against step + adjoint: 128 samples
+// 130 / 141 against 85 / 97 us, 200 239 / 256 against 196 / 207; the walk over blocks took 139 / 131
+// and 206 / 213).
+bool fan_as_two(int64_t n_smp) { return generic_vw(n_smp) == 2 && use_uniform<2>(n_smp); }
+
+void launch_adjoint_fan(hipStream_t st, const cvfes_system_t *sys, const AdjArgs &a, bool beta, bool damp) {
+    if (tiles_apply(sys)) adj_tile(st, sys, a, beta, damp);
+    else adj_dispatch<kOpFan>(st, a, beta, damp);
 }
 
 // Operator form of the generic row kernels for this system and method (as the forward step's
@@ -720,10 +733,7 @@ extern "C" int cvfes_adjoint_step(void *stream, const cvfes_system_t *sys, int m
     const AdjArgs a = adjoint_args(sys, mu1, mu2, mu_out, obs_u, obs_ref, obs_w, dt, beta, damp, project);
     hipStream_t st = static_cast<hipStream_t>(stream);
     switch (operator_form(sys, method)) {
-    case kOpFan:
-        if (tiles_apply(sys)) adj_tile(st, sys, a, beta != 0.0, damp != 0.0);
-        else adj_dispatch<kOpFan>(st, a, beta != 0.0, damp != 0.0);
-        break;
+    case kOpFan: launch_adjoint_fan(st, sys, a, beta != 0.0, damp != 0.0); break;
     case kOpMatfree: adj_dispatch<kOpMatfree>(st, a, beta != 0.0, damp != 0.0); break;
     case kOpStored: adj_dispatch<kOpStored>(st, a, beta != 0.0, damp != 0.0); break;
     default:
@@ -777,7 +787,14 @@ extern "C" int cvfes_adjoint_fused_step(void *stream, const cvfes_system_t *sys,
     const AdjArgs a = adjoint_args(sys, mu1, mu2, mu_out, obs_u, obs_ref, obs_w, dt, beta, damp, 1);
     hipStream_t st = static_cast<hipStream_t>(stream);
     switch (operator_form(sys, method)) {
-    case kOpFan: fused_dispatch<kOpFan>(st, f, a, beta != 0.0, damp != 0.0); break;
+    case kOpFan:
+        if (fan_as_two(sys->n_smp)) {
+            launch_matfree_step(st, sys, f, beta != 0.0, damp != 0.0);
+            launch_adjoint_fan(st, sys, a, beta != 0.0, damp != 0.0);
+        } else {
+            fused_dispatch<kOpFan>(st, f, a, beta != 0.0, damp != 0.0);
+        }
+        break;
     case kOpMatfree: fused_dispatch<kOpMatfree>(st, f, a, beta != 0.0, damp != 0.0); break;
     case kOpStored: fused_dispatch<kOpStored>(st, f, a, beta != 0.0, damp != 0.0); break;
     default:

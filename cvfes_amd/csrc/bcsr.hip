@@ -970,6 +970,11 @@ void step_dispatch(hipStream_t st, const cvfes_system_t *sys, bool mf, const Ste
 }
 
 }  // namespace
+
+void launch_matfree_step(hipStream_t st, const cvfes_system_t *sys, const StepArgs &a, bool beta, bool damp) {
+    step_dispatch(st, sys, true, a, 0, beta, damp);
+}
+
 }  // namespace cvfes
 
 using namespace cvfes;

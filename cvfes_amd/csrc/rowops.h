@@ -172,6 +172,9 @@ struct GStepArgs {
     bool nt_out;
 };
 
+// One matrix-free step as cvfes_step launches it (bcsr.hip).
+void launch_matfree_step(hipStream_t st, const cvfes_system_t *sys, const StepArgs &a, bool beta, bool damp);
+
 // Entry of a stored upper block that gives entry ij of the block a row needs: `side` < 0 the block's
 // column precedes its row (read transposed), 0 it is the row's diagonal block, > 0 neither.  The
 // diagonal block of a symmetric matrix is symmetric itself, so only its upper six entries are read:

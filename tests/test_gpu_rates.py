@@ -122,3 +122,27 @@ def test_records_only_where_they_pay(require_gpu, kind, call):
     print(f"by the rule {ruled:.1f} us, walked {walked:.1f}")
     assert ruled <= 1.08 * walked
     del kept
+
+
+# The fused forward + adjoint step exists to be faster than its two launches; matrix-free, with two
+# samples per lane of wave-uniform rows, it once took 1.2 to 1.5 times as long.
+@pytest.mark.parametrize("S", [128, 256])
+def test_fused_step_keeps_to_its_two_launches(require_gpu, S):
+    s = system(128, 128, S, store_values=False)
+    load, z = s.loads(np.zeros(4)), np.zeros(3 * s.n_nodes)
+    s.initial_state(z, z, load, 1e-7, damp=1.0, method="matfree")
+    a, b, c = (torch.zeros_like(s.u) for _ in range(3))
+    p, sys, ls = _lib.ptr, ctypes.byref(s._sys), load.struct(0)
+    state = (ctypes.c_void_p * 3)(*[t.data_ptr() for t in s.state])
+
+    def fused():
+        _lib.check(s.lib.cvfes_adjoint_fused_step(s.stream, sys, 1, state, ctypes.byref(ls), p(a), p(b), p(c), None, None,
+                                                  None, 1e-7, 0.0, 1.0))
+
+    def separate():
+        _lib.check(s.lib.cvfes_step(s.stream, sys, 1, state, ctypes.byref(ls), 1, 1e-7, 0.0, 1.0))
+        _lib.check(s.lib.cvfes_adjoint_step(s.stream, sys, 1, p(a), p(b), p(c), None, None, None, 1e-7, 0.0, 1.0, 1))
+
+    one, two = microseconds([fused, separate])
+    print(f"fused {one:.1f} us, two launches {two:.1f}")
+    assert one <= 1.1 * two
