@@ -361,7 +361,10 @@ extern "C" int cvfes_batch_plan(void *stream, cvfes_batch_mesh_t *meshes, int n_
         }
         k |= m.vw == 1 ? 2 : (m.packed ? 16 : 1);
         if (m.method == CVFES_METHOD_STORED) k |= 4;
-        if (m.method == CVFES_METHOD_MATFREE && !fan_entries(&s)) k |= kKindNoFan;
+        if (m.method == CVFES_METHOD_MATFREE && !fan_entries(&s)) {
+            m.sys.fan = nullptr;        // entries that the kernels may not use: they ask the descriptor
+            k |= kKindNoFan;
+        }
         if (m.beta != 0.0 || m.damp != 0.0) k |= 8;
         CVFES_REQUIRE(m.tiled == 0 || (m.tiled == 1 && cvfes_batch_can_tile(&m)),
                       "cvfes_batch_plan: mesh %d cannot be tiled", i);

@@ -488,7 +488,7 @@ int64_t cvfes_batch_plan_bytes(int n_mesh);
  * wavefront per task is n_waves = n_tasks).  kinds receives the paths the ensemble needs (bit 0:
  * wave-uniform rows with two samples per lane, bit 1: one sample per lane, bit 2: a stored mesh,
  * bit 3: beta or damp, bit 4: packed rows with two samples per lane, bit 10: a matrix-free mesh
- * without fan entries); pass it to cvfes_batch_step
+ * without fan entries, or with entries that do not serve it: those are set to NULL); pass it to cvfes_batch_step
  * and cvfes_batch_graph_create, which then launch a kernel instance with only those paths (fewer
  * registers, more waves in flight; n_waves >= n_tasks selects the instance without the persistent
  * loop).  Blocks until the copy is done. */

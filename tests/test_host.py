@@ -713,3 +713,30 @@ def test_batch_refuses_steps_past_load_tables():
     ens.run(2, graph=False)
     assert ens.step_index == 6
 
+
+
+@pytest.mark.parametrize("n_smp,with_nptr", [((1 << 31) // 24, True), (16, False)])
+def test_batch_plan_drops_fan_entries_that_do_not_serve(n_smp, with_nptr):
+    """The batched row kernel asks the descriptor whether a mesh has fan entries.  With samples beyond
+    their 32-bit offsets, or without the node pointers they are indexed by, the planned descriptor
+    may hold none (made-up addresses that no kernel sees; the copy to the device may fail here)."""
+    import ctypes
+    import torch
+    from cvfes_amd import _lib
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libcvfes_mi355x.so not built")
+    lib = _lib.lib()
+    arr = (_lib.CvfesBatchMesh * 1)()
+    m, some = arr[0], 4096
+    m.sys.n_nodes, m.sys.n_smp, m.sys.n_elms, m.sys.nnzb = 3, n_smp, 1, 9
+    for name in ("indptr", "indices", "cptr", "celem", "khat", "coef", "lm", "f1", "fan"):
+        setattr(m.sys, name, some)
+    m.sys.nptr = some if with_nptr else None
+    m.method, m.dt, m.load.p = _lib.METHOD_MATFREE, 1e-6, some
+    for k in range(3):
+        m.state[k] = some * (k + 2)
+    buf = torch.empty(int(lib.cvfes_batch_plan_bytes(1)), dtype=torch.uint8,
+                      device="cuda" if torch.cuda.is_available() else "cpu")
+    n_tasks, kinds = ctypes.c_int64(0), ctypes.c_int64(0)
+    lib.cvfes_batch_plan(None, arr, 1, buf.data_ptr(), ctypes.byref(n_tasks), ctypes.byref(kinds))
+    assert kinds.value & 1024 and not m.sys.fan
