@@ -152,6 +152,8 @@ FAN_MAX_ELEMS = 341
 
 # Node tiles of the matrix-free kernels (CVFES_TILE_*).
 TILE_ROWS, TILE_COLS, TILE_ELEMS = 16, 39, 8
+# Workgroups that one launch of the batched tile kernel takes, less its padding (2^32 threads of 512).
+TILE_MAX_BLOCKS = (1 << 23) - 16
 
 # Doubles in the static device scratch of cvfes_initial_state_static (CVFES_STATIC_SCRATCH_DOUBLES).
 STATIC_SCRATCH_DOUBLES = 8 << 20

@@ -77,6 +77,7 @@ class BatchedEnsemble:
     def _plan(self):
         n = len(self.systems)
         arr = (CvfesBatchMesh * n)()
+        blocks = 0              # workgroups of the tiled meshes, at most: their launch has a limit
         for i, s in enumerate(self.systems):
             m = arr[i]
             m.sys = s._make_struct()
@@ -86,7 +87,10 @@ class BatchedEnsemble:
             m.load = self.loads[i].struct(0)
             m.dt, m.beta, m.damp = self.dts[i], self.betas[i], self.damps[i]
             m.vw = self.vw_hint
-            m.tiled = int(m.sys.n_tiles > 0 and self.lib.cvfes_batch_can_tile(ctypes.byref(m)) != 0)
+            more = blocks + int(m.sys.n_tiles) * (int(m.sys.n_smp) // 32 + 1) + 8
+            m.tiled = int(m.sys.n_tiles > 0 and more < _lib.TILE_MAX_BLOCKS
+                          and self.lib.cvfes_batch_can_tile(ctypes.byref(m)) != 0)
+            blocks = more if m.tiled else blocks
         self._bufs = [(s.state[0], s.state[2], s.state[1]) for s in self.systems]   # state[0..2]
         nbytes = int(self.lib.cvfes_batch_plan_bytes(n))
         self.dev_meshes = torch.empty(nbytes, dtype=torch.uint8, device=self.device)

@@ -400,7 +400,8 @@ extern "C" int cvfes_batch_plan(void *stream, cvfes_batch_mesh_t *meshes, int n_
 
 extern "C" int cvfes_batch_can_tile(const cvfes_batch_mesh_t *mesh) {
     return mesh && mesh->method == CVFES_METHOD_MATFREE && fan_entries(&mesh->sys) && mesh->sys.n_smp > kTileSmall &&
-           tiles_apply(&mesh->sys);
+           tiles_apply(&mesh->sys) &&
+           launch_fits(mesh->sys.n_tiles * tile_shape(mesh->sys.n_smp).chunks, kTileThreads);
 }
 
 extern "C" int64_t cvfes_batch_tile_bytes(int n_mesh) {
@@ -437,7 +438,7 @@ extern "C" int cvfes_batch_plan_tiles(void *stream, const cvfes_batch_mesh_t *me
         if (m.sys.max_node_elems > 6) sh |= 1 << 16;
         if (m.beta != 0.0 || m.damp != 0.0) sh |= 1 << 17;
     }
-    CVFES_REQUIRE(x * kNumXcd < (int64_t(1) << 31), "cvfes_batch_plan_tiles: too many tiles");
+    CVFES_REQUIRE(launch_fits(x * kNumXcd, kTileThreads), "cvfes_batch_plan_tiles: too many tiles");
     *n_blocks = x * kNumXcd;
     *shape = sh | chunk;
     hipStream_t st = static_cast<hipStream_t>(stream);

@@ -84,10 +84,15 @@ inline unsigned tile_grid(const TileArgs &t) {
 // and 52, against 55, 53 and 58 staged by the row's lanes).
 constexpr int kTileSmall = 8;
 
-// Whether the matrix-free kernels of this system run by tiles.
+// Whether a launch of `blocks` workgroups stays below 2^32 threads, with room for tile_grid's padding.
+inline bool launch_fits(int64_t blocks, int threads) { return blocks + kNumXcd <= ((int64_t(1) << 32) - 1) / threads; }
+
+// Whether the matrix-free kernels of this system run by tiles.  Tiles of a wall whose rows have many
+// columns are half empty, so their launch can have more threads than that of the rows.
 inline bool tiles_apply(const cvfes_system_t *sys) {
+    const TileShape h = tile_shape(sys->n_smp);
     return sys->n_tiles > 0 && sys->tile_head && sys->tile_cols && sys->tile_ents && sys->max_node_elems >= 1 &&
-           sys->max_node_elems <= kTileElems && sys->n_tiles * (sys->n_smp / 32 + 1) < (1 << 30);
+           sys->max_node_elems <= kTileElems && launch_fits(sys->n_tiles * h.chunks, 64 * h.waves);
 }
 
 // `early()` issues what the caller needs for its row's update, while the last elements are applied.

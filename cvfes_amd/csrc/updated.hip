@@ -487,6 +487,8 @@ void order_by_tiles(GeomArgs &g, const cvfes_system_t *sys, bool more) {
     if (!more || !g.fan || sys->n_tiles <= 0 || !sys->tile_head || 24 * sys->n_nodes * sys->n_smp < (int64_t(32) << 20) ||
         sys->n_tiles * CVFES_TILE_ROWS > INT32_MAX)
         return;
+    // the tiles' empty slots count as rows of the launch, which stays below 2^32 threads
+    if (sys->n_tiles * CVFES_TILE_ROWS * lanes_per_row<true, 1>(sys->n_smp) >= (int64_t(1) << 32) - kBlock * kNumXcd) return;
     g.head = sys->tile_head;
     g.n_rows = sys->n_tiles * CVFES_TILE_ROWS;
 }

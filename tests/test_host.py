@@ -740,3 +740,19 @@ def test_batch_plan_drops_fan_entries_that_do_not_serve(n_smp, with_nptr):
     n_tasks, kinds = ctypes.c_int64(0), ctypes.c_int64(0)
     lib.cvfes_batch_plan(None, arr, 1, buf.data_ptr(), ctypes.byref(n_tasks), ctypes.byref(kinds))
     assert kinds.value & 1024 and not m.sys.fan
+
+
+@pytest.mark.parametrize("n_tiles,n_smp,fits", [
+    (2_700_000, 65, 1), (2_900_000, 65, 0), (8_300_000, 64, 1), (8_400_000, 64, 0), (1 << 28, 64, 0)])
+def test_tile_launches_stay_below_2_32_threads(n_tiles, n_smp, fits):
+    """512 threads a workgroup, a workgroup per tile and chunk of at most 64 samples (32 for odd counts);
+    a mesh beyond that is left to the row kernels (made-up addresses, nothing is launched)."""
+    import ctypes
+    from cvfes_amd import _lib
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libcvfes_mi355x.so not built")
+    m = _lib.CvfesBatchMesh()
+    m.method, m.sys.n_smp, m.sys.n_tiles, m.sys.max_node_elems = _lib.METHOD_MATFREE, n_smp, n_tiles, 6
+    for name in ("nptr", "fan", "tile_head", "tile_cols", "tile_ents"):
+        setattr(m.sys, name, 4096)
+    assert _lib.lib().cvfes_batch_can_tile(ctypes.byref(m)) == fits
