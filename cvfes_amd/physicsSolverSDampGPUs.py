@@ -211,9 +211,10 @@ class GPUSolidSolver(PhysicsSolver):
             tables = self._solve_tables
         else:
             tables = self._load_tables(np.array([self.t]))[0][1]
-        if self.traction is None and isinstance(tables, LoadTables):
+        if self.traction is None and isinstance(tables, LoadTables) and not isinstance(self.pressure, torch.Tensor):
             tables.set_pressure(self.pressure)
         else:
+            # a pressure on the device stays there: no host round trip, and a captured step reads it anew
             tables.p.fill_(self.pressure)
         self._advance(tables, dt)
         self._step_load = tables

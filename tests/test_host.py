@@ -756,3 +756,32 @@ def test_tile_launches_stay_below_2_32_threads(n_tiles, n_smp, fits):
     for name in ("nptr", "fan", "tile_head", "tile_cols", "tile_ents"):
         setattr(m.sys, name, 4096)
     assert _lib.lib().cvfes_batch_can_tile(ctypes.byref(m)) == fits
+
+
+def test_solver_takes_a_pressure_tensor_without_reading_it():
+    """A coupled program may set ``pressure`` to a device scalar: ``Solve`` fills the table with it on
+    the stream (a CPU stand-in whose conversion to a number fails), and a number still goes with the
+    launch."""
+    import torch
+    from cvfes_amd.physicsSolverSDampGPUs import GPUSolidSolver
+    from cvfes_amd.system import LoadTables
+
+    class Unread(torch.Tensor):
+        def __float__(self):
+            raise AssertionError("read on the host")
+
+    seen = []
+
+    class Sys:
+        def step(self, tables, dt, **kw):
+            seen.append((tables.value, float(tables.p.as_subclass(torch.Tensor)[0])))
+
+    s = object.__new__(GPUSolidSolver)
+    s.system, s.traction, s.updateInterval = Sys(), None, None
+    s.beta = s.damp = 0.0
+    s.method = "stored"
+    s._solve_tables = LoadTables(np.zeros(1), torch.device("cpu"))
+    s.t, s.finiteCheckEvery, s._nSolve = 0.0, 0, 0
+    for s.pressure in (4.0, torch.tensor(5.0, dtype=torch.float64).as_subclass(Unread), 6.0):
+        s.Solve(0.0, 1e-6)
+    assert seen == [(4.0, 4.0), (None, 5.0), (6.0, 6.0)]
