@@ -79,6 +79,8 @@ def algorithmic_bytes(sysm, method):
 def kernel_name(sysm, method):
     """Name of the step kernel ``cvfes_step`` launches for ``sysm`` and ``method``."""
     from cvfes_amd import _lib
+    if sysm.lib.cvfes_step_by_tiles(sysm._sys, _lib.METHODS[method]):
+        return f"{method} step, node tiles"
     kern = int(sysm.lib.cvfes_step_kernel(sysm._sys, _lib.METHODS[method]))
     names = {v: k for k, v in _lib.VARIANTS.items()}
     return f"{method} step, variant {names.get(kern, kern)}"

@@ -13,7 +13,7 @@ from pathlib import Path
 import torch  # noqa: F401  (load torch's HIP runtime first)
 
 LIB_PATH = Path(__file__).resolve().parent / "libcvfes_mi355x.so"
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 METHOD_STORED = 0
 METHOD_MATFREE = 1
@@ -119,6 +119,7 @@ _SIGNATURES = {
                                 _f64, _f64, _vp]),
     "cvfes_inverse_mass": (_int, [_vp, _i64, _vp, _vp]),
     "cvfes_step_kernel": (_i64, [ctypes.POINTER(CvfesSystem), _int]),
+    "cvfes_step_by_tiles": (_int, [ctypes.POINTER(CvfesSystem), _int]),
     "cvfes_adjoint_fused_step": (_int, [_vp, ctypes.POINTER(CvfesSystem), _int, ctypes.POINTER(_vp),
                                         ctypes.POINTER(CvfesLoad), _vp, _vp, _vp, _vp, _vp, _vp,
                                         _f64, _f64, _f64]),

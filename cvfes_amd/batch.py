@@ -195,11 +195,15 @@ class BatchedEnsemble:
                  occupancies=(0, 6, 5, 4)):
         """Pick the lane width, register cap and grid size (wavefronts) with the shortest step,
         then the cap on the waves per SIMD for that choice, then the wave order of rows wider
-        than a wavefront (row by row or sample group first)."""
+        than a wavefront (row by row or sample group first).  Nothing of this reaches meshes advanced
+        by node tiles: an ensemble of those alone keeps the first choices, timed once."""
         n_grid = len(candidates) if candidates is not None else 5
         n_occ = sum(1 for o in occupancies if o != 0)
         # every timed candidate runs 1 + steps eager steps of the ensemble's load tables
         self._check_steps((len(lane_widths) * len(caps) * n_grid + n_occ + 1) * (steps + 1))
+        rows = self.n_tasks > 0          # some mesh has wave tasks
+        if not rows:
+            lane_widths, caps, occupancies = lane_widths[:1], caps[:1], ()
         cus = torch.cuda.get_device_properties(self.device).multi_processor_count
         best = None
         saved = (self.phase, self.step_index)
@@ -214,7 +218,7 @@ class BatchedEnsemble:
                 self.n_tasks]
             for cap in caps:
                 self.cap = cap
-                for w in grid:
+                for w in grid if rows else grid[:1]:
                     self.n_waves = w
                     dt = self._time(steps)
                     if best is None or dt < best[3]:
@@ -230,7 +234,7 @@ class BatchedEnsemble:
             if dt < best[3]:
                 best = best[:3] + (dt, occ)
         self.waves_per_simd = best[4]
-        if any(int(m.lanes) > 64 and not int(m.packed) for m in self.host_meshes):
+        if rows and any(int(m.lanes) > 64 and not int(m.packed) for m in self.host_meshes):
             self.groups_first = True
             dt = self._time(steps)
             if dt < best[3]:

@@ -985,6 +985,11 @@ extern "C" int64_t cvfes_step_kernel(const cvfes_system_t *sys, int method) {
     return resolve_variant(sys, method == CVFES_METHOD_MATFREE);
 }
 
+extern "C" int cvfes_step_by_tiles(const cvfes_system_t *sys, int method) {
+    return method == CVFES_METHOD_MATFREE && cvfes_step_kernel(sys, method) == CVFES_VARIANT_GENERIC &&
+           fan_entries(sys) && tiles_apply(sys);
+}
+
 namespace {
 
 template <int VW, bool NT>

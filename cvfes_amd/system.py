@@ -497,14 +497,24 @@ class MembraneSystem:
         e1.synchronize()
         return e0.elapsed_time(e1) / steps
 
+    def _tunable(self, method, candidates):
+        """The candidates of a tuning of the step kernel: all of them, or the first alone where the step
+        runs by node tiles, which take neither a visiting order nor a cap."""
+        if self.method_id(method) == _lib.METHOD_MATFREE:
+            self._ensure_tiles()
+        candidates = tuple(candidates)
+        tiles = self.lib.cvfes_step_by_tiles(ctypes.byref(self._sys), self.method_id(method))
+        return candidates[:1] if tiles else candidates
+
     def autotune_row_order(self, load, dt, beta=0.0, damp=0.0, method="stored", steps=20,
                            candidates=(("natural", 0), ("strips", 32), ("strips", 48), ("strips", 64))):
         """Time ``steps`` steps under each visiting order in ``candidates`` ((order, strip width))
         and keep the fastest; returns ``{"order", "width", "ms"}``.  The displacements do not depend
         on the order (every order gives the same result bit for bit), only the time does.  Leaves
-        a fresh zero initial state behind."""
+        a fresh zero initial state behind.  A step by node tiles has no order to tune: the first
+        candidate is kept."""
         best = None
-        for order, width in candidates:
+        for order, width in self._tunable(method, candidates):
             self.set_row_order(order, width=width)
             ms = self._time_steps(load, dt, beta, damp, method, steps)
             if best is None or ms < best["ms"]:
@@ -519,9 +529,10 @@ class MembraneSystem:
         """Time ``steps`` steps under each occupancy cap in ``candidates`` (waves per SIMD, 0 = no
         cap) and keep the fastest; returns ``{"waves_per_simd", "ms"}``.  Large rows (many
         samples, long rings) run faster with fewer rows in flight per XCD; the displacements do not
-        depend on it.  Leaves a fresh zero initial state behind."""
+        depend on it.  Leaves a fresh zero initial state behind.  A step by node tiles takes no cap:
+        the first candidate is kept."""
         best = None
-        for w in candidates:
+        for w in self._tunable(method, candidates):
             self.set_occupancy(w)
             ms = self._time_steps(load, dt, beta, damp, method, steps)
             if best is None or ms < best["ms"]:

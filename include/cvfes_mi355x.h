@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define CVFES_ABI_VERSION 14
+#define CVFES_ABI_VERSION 15
 
 #define CVFES_OK 0
 #define CVFES_ERR_ARG (-1)   /* invalid argument (null pointer, bad size)        */
@@ -353,6 +353,13 @@ int cvfes_step_pressure(void *stream, const cvfes_system_t *sys, int method, dou
  * Host only.  No counterpart in the reference (one kernel there).
  */
 int64_t cvfes_step_kernel(const cvfes_system_t *sys, int method);
+
+/*
+ * Whether cvfes_step advances this system by node tiles (1) or not (0).  cvfes_step_kernel calls that
+ * kernel CVFES_VARIANT_GENERIC, whose operations it performs, but row_order and waves_per_simd do not
+ * reach it: there is nothing to tune.
+ */
+int cvfes_step_by_tiles(const cvfes_system_t *sys, int method);
 
 /*
  * One step of the adjoint recurrence of cvfes_step (no counterpart in the reference, which has no

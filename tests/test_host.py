@@ -785,3 +785,69 @@ def test_solver_takes_a_pressure_tensor_without_reading_it():
     for s.pressure in (4.0, torch.tensor(5.0, dtype=torch.float64).as_subclass(Unread), 6.0):
         s.Solve(0.0, 1e-6)
     assert seen == [(4.0, 4.0), (None, 5.0), (6.0, 6.0)]
+
+
+@pytest.mark.parametrize("tiles,timed", [(1, 1), (0, 6)])
+def test_nothing_is_tuned_where_the_step_runs_by_tiles(tiles, timed):
+    """Stand-in system: the tile kernel takes no cap and no visiting order, so one candidate is timed
+    and noise picks nothing that the other kernels would then run under."""
+    import types
+    from cvfes_amd import _lib
+    from cvfes_amd.system import MembraneSystem
+
+    class Sys(MembraneSystem):
+        def initial_state(self, *a, **k):
+            pass
+
+        def set_occupancy(self, w=0):
+            self.waves_per_simd = w
+
+        def set_row_order(self, order="bisection", leaf=64, width=64):
+            self.order = order, width
+
+        def _time_steps(self, *a):
+            calls.append(1)
+            return 10.0 - len(calls)                   # each candidate seems faster than the last
+
+    s = object.__new__(Sys)
+    s.n_nodes, s.fan, s.tile_head, s._sys = 4, None, None, _lib.CvfesSystem()
+    s.lib = types.SimpleNamespace(cvfes_step_by_tiles=lambda sys, method: tiles)
+    calls = []
+    got = s.autotune_occupancy(None, 1e-6, method="matfree")
+    assert len(calls) == timed and got["waves_per_simd"] == s.waves_per_simd == (0 if tiles else 2)
+    calls = []
+    got = s.autotune_row_order(None, 1e-6, method="matfree")
+    assert len(calls) == min(timed, 4) and s.order == (("natural", 0) if tiles else ("strips", 64))
+    assert (got["order"], got["width"]) == s.order
+
+
+@pytest.mark.parametrize("n_tasks,timed", [(0, 1), (64, 34)])
+def test_batch_tunes_only_meshes_with_wave_tasks(monkeypatch, n_tasks, timed):
+    import types
+    import torch
+    from cvfes_amd import batch as B
+    calls = []
+
+    class Ens(B.BatchedEnsemble):
+        def _check_steps(self, n):
+            pass
+
+        def _replan(self):
+            pass
+
+        def _sync_roles(self):
+            pass
+
+        def _time(self, steps):
+            calls.append(1)
+            return 10.0 - 0.1 * len(calls)
+
+    monkeypatch.setattr(torch.cuda, "get_device_properties", lambda d: types.SimpleNamespace(multi_processor_count=256))
+    ens = object.__new__(Ens)
+    ens.device, ens._graphs, ens.phase, ens.step_index, ens.n_tasks = torch.device("cpu"), {}, 0, 0, n_tasks
+    ens.vw_hint, ens.cap, ens.waves_per_simd, ens.n_waves, ens.groups_first = 0, False, 0, 0, False
+    ens.host_meshes = [types.SimpleNamespace(lanes=128, packed=0)]
+    got = ens.autotune()
+    assert len(calls) == timed and got["waves_per_simd"] == (0 if n_tasks == 0 else 4)
+    if n_tasks == 0:
+        assert (ens.vw_hint, ens.cap, ens.groups_first, ens.waves_per_simd) == (0, False, False, 0)
