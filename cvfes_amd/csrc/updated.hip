@@ -477,18 +477,24 @@ void launch_updated_u(hipStream_t st, const StepArgs &a, const GeomArgs &g, int6
     else launch_updated_inst<false, FAST, GEO_U, VW>(st, a, g, step, beta, damp);
 }
 
-// Rows by node tiles where a neighbour takes more than its u (the damped state or a saved geometry)
-// and u is larger than the L2s: in natural order the neighbouring rings' lines leave L2 between their
-// rows.  102,400 nodes x 128 samples with beta: 3.47 -> 1.31 GB of traffic, 521 -> 503 us, a saved
-// geometry 576 -> 558 us; 65,920 x 200 611 -> 593 and 663 -> 650 us.  With u alone natural order
-// already moves 1.4 GB (450 against 458 us by tiles), and a small system gains nothing (4,096 x 33,
-// saved geometry: 13.1 against 13.4 us).
-void order_by_tiles(GeomArgs &g, const cvfes_system_t *sys, bool more) {
-    if (!more || !g.fan || sys->n_tiles <= 0 || !sys->tile_head || 24 * sys->n_nodes * sys->n_smp < (int64_t(32) << 20) ||
+// Rows by node tiles where u is larger than the L2s, a neighbour takes more than its u (the damped state
+// or a saved geometry) and rows are long: in natural order the neighbouring rings' lines then leave L2
+// between their rows.  Five steps, natural / by tiles, 16,384 nodes x 256 samples: with beta 876 / 811 us,
+// a saved geometry 1,000 / 938, both 1,312 / 1,015 (irregular wall 879 / 845, 1,020 / 987, 1,264 / 1,035);
+// 65,920 x 200: 3,078 / 2,984, 3,429 / 3,341, 3,886 / 3,672.  Shorter rows gain only with both and whole
+// wavefronts (102,400 x 128: 3,957 / 3,187; beta alone 2,615 / 2,539, on an irregular wall 2,687 /
+// 2,861), others lose by the tiles' empty slots and the wider spread of a workgroup's rows (102,400 x 64
+// with both 2,016 / 2,189, 65,920 x 180 1.03 and 1.09 times as long).  With u alone natural order already
+// moves little (102,400 x 128: 450 / 458 us a step), and a small system gains nothing (4,096 x 33: 13.1 /
+// 13.4).
+void order_by_tiles(GeomArgs &g, const cvfes_system_t *sys, bool beta, bool saved) {
+    const int64_t S = sys->n_smp;
+    if (!g.fan || sys->n_tiles <= 0 || !sys->tile_head || S % 2 != 0 || 24 * sys->n_nodes * S < (int64_t(32) << 20) ||
         sys->n_tiles * CVFES_TILE_ROWS > INT32_MAX)
         return;
+    if (S >= 192 ? !(beta || saved) : !(beta && saved && S % 128 == 0)) return;
     // the tiles' empty slots count as rows of the launch, which stays below 2^32 threads
-    if (sys->n_tiles * CVFES_TILE_ROWS * lanes_per_row<true, 1>(sys->n_smp) >= (int64_t(1) << 32) - kBlock * kNumXcd) return;
+    if (sys->n_tiles * CVFES_TILE_ROWS * lanes_per_row<true, 1>(S) >= (int64_t(1) << 32) - kBlock * kNumXcd) return;
     g.head = sys->tile_head;
     g.n_rows = sys->n_tiles * CVFES_TILE_ROWS;
 }
@@ -606,7 +612,7 @@ extern "C" int cvfes_step_updated(void *stream, const cvfes_system_t *sys, const
         a.ddt = damp / dt;
         a.order = nullptr;
         GeomArgs g = geom_args(geo, sys, geom);
-        order_by_tiles(g, sys, beta != 0.0 || (geom != nullptr && geom != cur));
+        order_by_tiles(g, sys, beta != 0.0, geom != nullptr && geom != cur);
         launch_updated(st, a, g, n, beta != 0.0, damp != 0.0, sys->variant, geom != nullptr && geom == cur);
         if (int rc = check_launch("k_step_updated")) return rc;
         double *t = prev;

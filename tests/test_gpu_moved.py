@@ -62,3 +62,26 @@ def test_rows_by_tiles_equal_natural_order(require_gpu, S, interval, beta):
         got.append(s.u.cpu().numpy())
     # the initial product runs by rows either way
     assert np.max(np.abs(got[0])) > 0 and np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("S,interval,beta", [(128, 3, 1e-7), (192, 3, 0.0), (256, 1, 1e-7)])
+def test_row_order_rule_keeps_the_bits(require_gpu, S, interval, beta):
+    """The shortest rows that take the tiles' order with a damped state and a saved geometry, and with
+    one of them."""
+    from cvfes_amd.mesh import tube_geometry
+    from cvfes_amd.system import MembraneSystem
+    nodes, el, bdy = tube_geometry(128, 97, 0.3, 2.0)
+    assert 24 * nodes.shape[0] * S > 32 << 20
+    E = 7e6 * np.exp(0.1 * np.random.default_rng(S).standard_normal((el.shape[0], S)))
+    u0 = 1e-3 * np.random.default_rng(1).standard_normal(3 * nodes.shape[0])
+    s = MembraneSystem(nodes, el, bdy, S, vthickness=np.full(nodes.shape[0], 0.07), elmE=E, density=1.0, nu=0.45,
+                       store_values=False)
+    got = []
+    for n in (s.n_tiles, 0):
+        s.n_tiles = n
+        s._sys = s._make_struct()
+        ls = s.loads(np.full(5, 1.33e4))
+        s.initial_state(u0, 0.0 * u0, ls, 1e-6, beta=beta, damp=5.0, method="matfree")
+        s.step_updated(ls, 1e-6, interval, beta=beta, damp=5.0)
+        got.append(s.u.cpu().numpy())
+    assert np.max(np.abs(got[0])) > 0 and np.array_equal(got[0], got[1])
