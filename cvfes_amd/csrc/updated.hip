@@ -330,7 +330,8 @@ __global__ __launch_bounds__(kBlock) void k_step_moved(StepArgs a, GeomArgs g, i
 // GEO: 0 the reference geometry (the gradients are the same for a lane's samples), 1 X + u itself,
 // 2 X + ug.  The output is written once and read by no kernel, in 16-byte stores, past L2 (NT) where
 // stream_stress says so.
-// 131,840 elements x 100 samples (0.79 GB) on the reference geometry: 270 -> 155 us.
+// 131,840 elements x 100 samples (0.79 GB) on the reference geometry: the call 270 -> 178 us, of which this
+// kernel takes 155 to 171.
 template <bool UNIFORM, int GEO, int VW, bool NT>
 __global__ __launch_bounds__(kBlock) void k_element_stress(int64_t n_elms, int64_t S, GeomArgs g,
                                                            const double *__restrict__ u,
