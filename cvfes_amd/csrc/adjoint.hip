@@ -642,9 +642,8 @@ void fused_launch(hipStream_t st, const StepArgs &f, const AdjArgs &a, bool beta
 template <int MF>
 void fused_dispatch(hipStream_t st, const StepArgs &f, const AdjArgs &a, bool beta, bool damp) {
     if (generic_vw(f.k.n_smp) == 2) {
-        if constexpr (MF != kOpFan)         // fan_as_two
-            if (use_uniform<2>(f.k.n_smp)) return fused_launch<MF, true, 2>(st, f, a, beta, damp);
-        fused_launch<MF, false, 2>(st, f, a, beta, damp);
+        if (use_uniform<2>(f.k.n_smp)) fused_launch<MF, true, 2>(st, f, a, beta, damp);
+        else fused_launch<MF, false, 2>(st, f, a, beta, damp);
     } else {
         if (use_uniform<1>(f.k.n_smp)) fused_launch<MF, true, 1>(st, f, a, beta, damp);
         else fused_launch<MF, false, 1>(st, f, a, beta, damp);
@@ -655,8 +654,11 @@ void fused_dispatch(hipStream_t st, const StepArgs &f, const AdjArgs &a, bool be
 // fan walk holds the registers of two waves per SIMD, and reading the coefficients once saves less
 // than that costs (16,384 nodes of a regular / irregular wall, fused against step + adjoint: 128 samples
 // 130 / 141 against 85 / 97 us, 200 239 / 256 against 196 / 207; the walk over blocks took 139 / 131
-// and 206 / 213).
-bool fan_as_two(int64_t n_smp) { return generic_vw(n_smp) == 2 && use_uniform<2>(n_smp); }
+// and 206 / 213).  Small systems are bound by the launches themselves (600 nodes x 128: 9.4 against
+// 14.1 us, 96 x 2,048: 13.7 against 15.4, 2,052 x 128: 21.6 against 21.8).
+bool fan_as_two(const cvfes_system_t *sys) {
+    return generic_vw(sys->n_smp) == 2 && use_uniform<2>(sys->n_smp) && sys->n_nodes * sys->n_smp >= (1 << 18);
+}
 
 void launch_adjoint_fan(hipStream_t st, const cvfes_system_t *sys, const AdjArgs &a, bool beta, bool damp) {
     if (tiles_apply(sys)) adj_tile(st, sys, a, beta, damp);
@@ -788,7 +790,7 @@ extern "C" int cvfes_adjoint_fused_step(void *stream, const cvfes_system_t *sys,
     hipStream_t st = static_cast<hipStream_t>(stream);
     switch (operator_form(sys, method)) {
     case kOpFan:
-        if (fan_as_two(sys->n_smp)) {
+        if (fan_as_two(sys)) {
             launch_matfree_step(st, sys, f, beta != 0.0, damp != 0.0);
             launch_adjoint_fan(st, sys, a, beta != 0.0, damp != 0.0);
         } else {

@@ -96,13 +96,14 @@ constexpr int kRecordSlots = 7;
 // elements, walk / records: 64 samples 80 / 93 us a step, 8 12.0 / 13.5; 102,400 rows, 2 samples: product
 // 32 / 45 us, 33 287 / 331; few gained, 16,384 rows, 40 samples: 55 / 49).  Adjoint: the adjoint step with
 // one sample per lane loses by records in wave-uniform rows (16,384 nodes of a regular wall, 48 samples:
-// 66 / 76 us) and with one sample in all (102,400 nodes: 20.2 / 22.2).
+// 66 / 76 us), and with one sample on large walls (102,400 nodes: 20.2 / 22.2; 16,384: 9.2 / 7.9).
 inline bool use_records(const cvfes_system_t *sys, bool adjoint = false) {
     const int64_t S = sys->n_smp;
     if (!sys->row_records || !sys->uvalues || 72 * S > INT32_MAX || sys->record_width != 2 + 2 * kRecordSlots ||
         sys->max_row_blocks < 1 || sys->max_row_blocks > kRecordSlots)
         return false;
-    return !adjoint || (S > 1 && (generic_vw(S) == 2 || !use_uniform<1>(S)));
+    if (!adjoint) return true;
+    return S == 1 ? sys->n_nodes < (1 << 16) : generic_vw(S) == 2 || !use_uniform<1>(S);
 }
 
 // Node tiles (tile.h): rows per tile, column slots (39 of 64 samples and the unit blocks of 16

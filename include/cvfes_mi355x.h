@@ -378,7 +378,7 @@ int cvfes_adjoint_step(void *stream, const cvfes_system_t *sys, int method, cons
  * One forward step (as cvfes_step with nsteps = 1: state = {u_n, u_{n-1}, out}, load entry 0 of
  * `load`) and one projected adjoint step (as cvfes_adjoint_step with project = 1) in one kernel
  * that reads the operator once for both, or in two launches where those are faster (matrix-free,
- * two samples per lane of wave-uniform rows); the two may be at different time steps.  Both outputs
+ * two samples per lane of wave-uniform rows, all but small systems); the two may be at different time steps.  Both outputs
  * equal those of the separate calls bit for bit.  Needs cvfes_step_kernel(sys, method) to be
  * CVFES_VARIANT_GENERIC (the kernel whose operations it replays) and six distinct buffers
  * (mu1 may equal mu2).  The state array is not rotated.  No counterpart in the reference (used by

@@ -255,3 +255,42 @@ def test_lists_refuse_a_tile_that_does_not_fit(require_gpu):
         rc = s.lib.cvfes_tile_lists(s.stream, 1, rows.data_ptr(), s.nptr.data_ptr(), s.fan.data_ptr(),
                                     s.max_node_elems, *[t.data_ptr() for t in out])
         assert (rc == 0) == good
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nz,S,beta,damp,tiled", [
+    (42, 128, 1e-7, 5.0, True), (42, 100, 0.0, 0.0, True), (42, 128, 1e-7, 0.0, False), (9, 128, 0.0, 5.0, True),
+    (42, 96, 0.0, 5.0, False), (42, 66, 1e-7, 0.0, True)])
+def test_fused_step_is_its_two_steps(require_gpu, nz, S, beta, damp, tiled):
+    """Two samples per lane of wave-uniform rows, large and small (two launches and one), with tiles and
+    by rows; 66 samples: packed rows."""
+    import torch
+    from cvfes_amd.system import MembraneSystem
+    nodes, el, bdy = tube_geometry(64, nz, 0.3, 2.0)
+    E = 7e6 * np.exp(0.1 * np.random.default_rng(S).standard_normal((el.shape[0], S)))
+    s = MembraneSystem(nodes, el, bdy, S, vthickness=np.full(nodes.shape[0], 0.07), elmE=E, density=1.0, nu=0.45,
+                       store_values=False)
+    if not tiled:
+        s.n_tiles = 0
+        s._sys = s._make_struct()
+    load, dt = s.loads(np.full(3, 1.33e4)), 1e-6
+    u0 = 1e-4 * np.random.default_rng(1).standard_normal(3 * nodes.shape[0])
+    s.initial_state(u0, 0.0 * u0, load, dt, beta=beta, damp=damp, method="matfree")
+    gen = torch.Generator(device="cuda").manual_seed(S)
+    m1, m2 = (torch.randn(s.state_shape(), generator=gen, dtype=torch.float64, device="cuda") for _ in range(2))
+    w = torch.linspace(0.5, 1.5, S, dtype=torch.float64, device="cuda")
+    p, got = _lib.ptr, []
+    for fused in (True, False):
+        out, mu = torch.full_like(s.u, np.nan), torch.full_like(s.u, np.nan)
+        arr = (ctypes.c_void_p * 3)(p(s.u), p(s.up), p(out))
+        ls, sys = ctypes.byref(load.struct(1)), ctypes.byref(s._sys)
+        if fused:
+            _lib.check(s.lib.cvfes_adjoint_fused_step(s.stream, sys, 1, arr, ls, p(m1), p(m2), p(mu), p(s.up), None, p(w),
+                                                      dt, beta, damp))
+        else:
+            _lib.check(s.lib.cvfes_step(s.stream, sys, 1, arr, ls, 1, dt, beta, damp))
+            _lib.check(s.lib.cvfes_adjoint_step(s.stream, sys, 1, p(m1), p(m2), p(mu), p(s.up), None, p(w), dt, beta,
+                                                damp, 1))
+        got.append((out.cpu().numpy(), mu.cpu().numpy()))
+    for a, b in zip(*got):
+        assert np.all(np.isfinite(a)) and np.max(np.abs(a)) > 0 and np.array_equal(a, b)
