@@ -100,8 +100,9 @@ typedef struct cvfes_system {
      * then the columns of its blocks and their upper-storage entries (vblk), MAXB of each, padded
      * with the row's last block, where MAXB = (record_width - 2) / 2 is the kernel's block-slot
      * count (7 or 10, as the row-load kernels choose it).  One scalar load then gives a row its
-     * whole structure.  The kernels fall back to indptr/indices/vblk when the width does not
-     * match; the results are the same either way. */
+     * whole structure.  The generic step, product, adjoint and fused kernels take records of 7.
+     * The kernels fall back to indptr/indices/vblk when the width does not match or the walk is
+     * faster; the results are the same either way. */
     const int32_t *row_records;
     int64_t record_width;
     /* Inverse lumped masses 1/lm (0 where lm = 0), same layout as lm (may be NULL).  The adjoint
