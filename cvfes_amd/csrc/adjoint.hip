@@ -382,6 +382,33 @@ __device__ __forceinline__ void grad_form(const double (&nu)[2][3][VW], const do
     }
 }
 
+// The same with all nine blocks and the vectors as they are: a system without fan entries makes no claim
+// on its unit blocks.  Entry (3 p + b, 3 i + j) of the element's block is kh(9 (3 p + b) + 3 i + j).
+constexpr int kGradAll = 81;
+
+template <int VW, class KH>
+__device__ __forceinline__ void grad_form_all(const double (&nu)[3][3][VW], const double (&x)[3][3][VW], KH kh,
+                                              double (&acc)[VW]) {
+#pragma unroll
+    for (int v = 0; v < VW; ++v) acc[v] = 0.0;
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            double t[VW] = {};
+#pragma unroll
+            for (int b = 0; b < 3; ++b)
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    const double h = kh(9 * (3 * p + b) + 3 * i + j);
+#pragma unroll
+                    for (int v = 0; v < VW; ++v) t[v] = fma(h, x[b][j][v], t[v]);
+                }
+#pragma unroll
+            for (int v = 0; v < VW; ++v) acc[v] = fma(nu[p][i][v], t[v], acc[v]);
+        }
+}
+
 __device__ __forceinline__ double grad_scale(const GradArgs &a, double m) {
     return a.minv ? a.nu_scale * m : (m != 0.0 ? a.nu_scale / m : 0.0);
 }
@@ -390,7 +417,7 @@ __device__ __forceinline__ double grad_scale(const GradArgs &a, double m) {
 // and VW samples at s, with nu = nu_scale * mu / m (nu_scale * minv with the inverse masses) and
 // x = xc + bdt (xc - xp) (PREV; else x = xc).  `sc` holds nu_scale / m of the three nodes where the
 // mass has no sample axis.  All loads are issued before the first is used.
-template <bool PREV, bool LMS, int VW, class KH>
+template <bool PREV, bool LMS, int VW, bool ALL = false, class KH>
 __device__ __forceinline__ void grad_update(const GradArgs &a, int64_t e, int64_t s, const int32_t (&ids)[3],
                                             const double (&sc)[3], KH kh) {
     Vec<VW> mu[3][3], c[3][3], p[3][3], m[3];
@@ -410,7 +437,28 @@ __device__ __forceinline__ void grad_update(const GradArgs &a, int64_t e, int64_
     const Vec<VW> cf = load_vec<VW>(a.coef + idx);
     Vec<VW> g = load_vec<VW>(a.grad + idx);
     __builtin_amdgcn_sched_barrier(0);
-    double nu0[3][VW], x0[3][VW], dn[2][3][VW], dx[2][3][VW], f[VW];
+    double f[VW];
+    if constexpr (ALL) {
+        double nu[3][3][VW], x[3][3][VW];
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int v = 0; v < VW; ++v) {
+                const double scale = LMS ? grad_scale(a, m[q].v[v]) : sc[q];
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    const double u = c[q][j].v[v];
+                    nu[q][j][v] = scale * mu[q][j].v[v];
+                    x[q][j][v] = PREV ? fma(a.bdt, u - p[q][j].v[v], u) : u;
+                }
+            }
+        grad_form_all<VW>(nu, x, kh, f);
+#pragma unroll
+        for (int v = 0; v < VW; ++v) g.v[v] = fma(-cf.v[v], f[v], g.v[v]);
+        store_vec<VW>(a.grad + idx, g);
+        return;
+    }
+    double nu0[3][VW], x0[3][VW], dn[2][3][VW], dx[2][3][VW];
 #pragma unroll
     for (int q = 0; q < 3; ++q)
 #pragma unroll
@@ -472,10 +520,11 @@ __global__ __launch_bounds__(kBlock) void k_grad_accum(GradArgs a) {
 constexpr int kGradMin = 8, kGradPair = 16;
 constexpr int kGradElems = (kBlock - 1) / kGradMin + 2;   // 33
 
-template <bool PREV, bool LMS, int VW>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(VW == 2 && !LMS ? 4 : 1))) void
+template <bool PREV, bool LMS, int VW, bool ALL = false>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(VW == 2 && !LMS && !ALL ? 4 : 1))) void
 k_grad_accum_lds(GradArgs a) {
-    __shared__ double sk[kGradElems * kGradKh];
+    constexpr int KH = ALL ? kGradAll : kGradKh;
+    __shared__ double sk[kGradElems * KH];
     __shared__ double ssc[kGradElems * 3];
     __shared__ int32_t sid[kGradElems * 3];
     const uint32_t lpr = static_cast<uint32_t>(a.n_smp / VW), g0 = static_cast<uint32_t>(xcd_block() * kBlock);
@@ -488,9 +537,10 @@ k_grad_accum_lds(GradArgs a) {
         sid[q] = id;
         ssc[q] = LMS ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[id]);
     }
-    for (int q = threadIdx.x; q < nel * kGradKh; q += kBlock) {
-        const int le = q / kGradKh, r = q - le * kGradKh;
-        sk[q] = a.khat[9 * static_cast<int64_t>(a.cpos[9 * static_cast<int64_t>(e0 + le) + grad_block(r)]) + r % 9];
+    for (int q = threadIdx.x; q < nel * KH; q += kBlock) {
+        const int le = q / KH, r = q - le * KH;
+        const int block = ALL ? r / 9 : grad_block(r);
+        sk[q] = a.khat[9 * static_cast<int64_t>(a.cpos[9 * static_cast<int64_t>(e0 + le) + block]) + r % 9];
     }
     __syncthreads();
     const uint32_t g = g0 + threadIdx.x, e = g / lpr;
@@ -498,25 +548,26 @@ k_grad_accum_lds(GradArgs a) {
     const int le = static_cast<int>(e - e0);
     const int32_t ids[3] = {sid[3 * le], sid[3 * le + 1], sid[3 * le + 2]};
     const double sc[3] = {ssc[3 * le], ssc[3 * le + 1], ssc[3 * le + 2]};
-    grad_update<PREV, LMS, VW>(a, e, static_cast<int64_t>(g - e * lpr) * VW, ids, sc,
-                    [&](int i) { return sk[kGradKh * le + i]; });
+    grad_update<PREV, LMS, VW, ALL>(a, e, static_cast<int64_t>(g - e * lpr) * VW, ids, sc,
+                                    [&](int i) { return sk[KH * le + i]; });
 }
 
 // Fewer than 8 samples: everything read per lane.
-template <bool PREV, bool LMS>
+template <bool PREV, bool LMS, bool ALL = false>
 __global__ __launch_bounds__(kBlock) void k_grad_accum_lane(GradArgs a) {
     const int64_t g = xcd_block() * kBlock + threadIdx.x;
     if (g >= a.n_elms * a.n_smp) return;
     const int64_t e = g / a.n_smp;
     const int32_t ids[3] = {a.elems[3 * e], a.elems[3 * e + 1], a.elems[3 * e + 2]};
+    constexpr int BLOCKS = ALL ? 9 : 3;
     double sc[3];
-    const double *kh[3];
+    const double *kh[BLOCKS];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        sc[q] = LMS ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[ids[q]]);
-        kh[q] = a.khat + 9 * static_cast<int64_t>(a.cpos[9 * e + grad_block(9 * q)]);
-    }
-    grad_update<PREV, LMS, 1>(a, e, g - e * a.n_smp, ids, sc, [&](int i) { return kh[i / 9][i % 9]; });
+    for (int q = 0; q < 3; ++q) sc[q] = LMS ? 1.0 : grad_scale(a, (a.minv ? a.minv : a.lm)[ids[q]]);
+#pragma unroll
+    for (int q = 0; q < BLOCKS; ++q)
+        kh[q] = a.khat + 9 * static_cast<int64_t>(a.cpos[9 * e + (ALL ? q : grad_block(9 * q))]);
+    grad_update<PREV, LMS, 1, ALL>(a, e, g - e * a.n_smp, ids, sc, [&](int i) { return kh[i / 9][i % 9]; });
 }
 
 template <int MF, bool UNI, int VW>
@@ -829,7 +880,11 @@ extern "C" int cvfes_grad_accum(void *stream, const cvfes_system_t *sys, const i
         auto launch = [&](auto kernel, int vw) {
             hipLaunchKernelGGL(kernel, dim3(grid_for(work / vw)), dim3(kBlock), 0, st, a);
         };
-        if (S % 128 == 0 && pairs) launch(k_grad_accum<PREV, LMS>, 2);
+        if (!sys->fan) {        // no claim on the unit blocks: all of them
+            if (S >= kGradPair && pairs) launch(k_grad_accum_lds<PREV, LMS, 2, true>, 2);
+            else if (S >= kGradMin) launch(k_grad_accum_lds<PREV, LMS, 1, true>, 1);
+            else launch(k_grad_accum_lane<PREV, LMS, true>, 1);
+        } else if (S % 128 == 0 && pairs) launch(k_grad_accum<PREV, LMS>, 2);
         else if (S >= kGradPair && pairs) launch(k_grad_accum_lds<PREV, LMS, 2>, 2);
         else if (S >= kGradMin) launch(k_grad_accum_lds<PREV, LMS, 1>, 1);
         else launch(k_grad_accum_lane<PREV, LMS>, 1);

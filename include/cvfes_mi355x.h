@@ -47,9 +47,10 @@ typedef struct cvfes_system {
     const double *values;     /* [nnzb][9][S] stored values                                    */
     const int32_t *cptr;      /* [nnzb+1] contribution ranges per block                        */
     const int32_t *celem;     /* [9E] element of each contribution                             */
-    const double *khat;       /* [9E][9] unit-coefficient element block of each contribution; the
-                                 kernels by fan entries, by tiles and of the gradient take an
-                                 element's rows to sum to zero and its block to be symmetric     */
+    const double *khat;       /* [9E][9] unit-coefficient element block of each contribution; with
+                                 fan entries (`fan`) the matrix-free kernels and the gradient take
+                                 an element's rows to sum to zero and its block to be symmetric,
+                                 as cvfes_element_matrices writes them; without, any block       */
     const double *coef;       /* [E][S] stiffness coefficient per element and sample           */
     const double *lm;         /* lumped mass, [N][S] (lm_sstride = 1) or [N] (lm_sstride = 0)  */
     int64_t lm_sstride;
